@@ -61,6 +61,12 @@ def make_params(name):
     return table[name]()
 
 
+def direct_solve(p):
+    """tolerance mode solved by fast sine transforms (no V-cycle sweeps given)"""
+    return (p.mg_mode == pic2d.MG_TOL and p.nodes <= 4097 and
+            (p.mg_sweeps == -1 or p.nodes <= 65))
+
+
 def describe(name, p, tuning):
     nu = tuning["mg_sweeps"]
     return {
@@ -73,6 +79,7 @@ def describe(name, p, tuning):
         "walls": "absorbing" if p.wall == pic2d.WALL_ABSORB else "steady-state plop",
         "mode": "physical" if p.mode == pic2d.MODE_PHYSICAL else "reference",
         "multigrid": ("fp64 FMG ncycle=%d" % p.mg_ncycle) if p.mg_mode == pic2d.MG_FIXED
+        else ("fp64 direct sine-transform solve, tol %g" % p.mg_tol) if direct_solve(p)
         else ("fp32 red-black V(%d,%d) cycles + fp64 refinement, tol %g"
               % (nu, nu, p.mg_tol)),
         # launch shapes in effect (explicit, or the library's tuned table)
@@ -460,10 +467,14 @@ def main():
     # multigrid roofline: about 50 B per node per level visit of a V-cycle
     # (smoothing, residual, restriction, prolongation; 4/3 N^2 nodes over the
     # levels) and 40 B per finest node per FP64 refinement pass; the fixed
-    # FMG visits (4/3)^2 N^2 nodes ncycle times.  The field phase's time
-    # (rho, right-hand side, solve, E) is the denominator: latency-bound.
+    # FMG visits (4/3)^2 N^2 nodes ncycle times; the direct solve reads and
+    # writes 16 B per node in each of its three passes, and 16 B are read for
+    # its residual.  The field phase's time (rho, right-hand side, solve, E)
+    # is the denominator: latency-bound.
     nn = float(p.nodes) ** 2
-    if p.mg_mode == pic2d.MG_TOL:
+    if direct_solve(p):
+        mg_bytes = phase["mg_cycles_per_step"] * 64.0 * nn
+    elif p.mg_mode == pic2d.MG_TOL:
         mg_bytes = phase["mg_cycles_per_step"] * (50.0 * nn * 4.0 / 3.0 + 40.0 * nn)
     else:
         mg_bytes = 50.0 * p.mg_ncycle * (4.0 / 3.0) ** 2 * nn

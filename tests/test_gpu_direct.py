@@ -1,0 +1,107 @@
+"""The direct FP64 Poisson solve (fast sine transforms) on every grid size it
+has a transform for, against a sine-transform solve in numpy and an analytic
+mode; its refinement, its start from a caller's guess, and the switch between
+it and the V-cycles a caller asks for."""
+import numpy as np
+import pytest
+
+import orc
+import pic2d
+import workloads
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(np.float64).eps
+L = 0.01
+
+
+def dst(a):
+    m, n = a.shape[0], a.shape[1] + 1
+    z = np.zeros((m, 2 * n))
+    z[:, 1:n] = a
+    z[:, n + 1:] = -a[:, ::-1]
+    return -0.5 * np.fft.rfft(z, axis=1).imag[:, 1:n]
+
+
+def poisson(f):
+    n = f.shape[0] - 1
+    lam = -(4.0 * (n / L) ** 2) * np.sin(np.pi * np.arange(1, n) / (2.0 * n)) ** 2
+    u = np.zeros_like(f)
+    t = dst(dst(f[1:n, 1:n]).T) / (lam[:, None] + lam[None, :])
+    u[1:n, 1:n] = dst(dst(t).T) * (2.0 / n) ** 2
+    return u
+
+
+@pytest.mark.parametrize("n", [4, 8, 16, 32, 64, 128, 256, 512, 1024, 2048])
+def test_against_numpy_transforms(n):
+    """both solves apply four FP64 transforms: each is within a few eps
+    log2(2n) of the exact solution"""
+    print(f"direct n={n}", flush=True)
+    f = np.random.default_rng(n).standard_normal((n + 1, n + 1)) * 1e9
+    u, cycles, rr = pic2d.poisson_tol(f, length=L, tol=1e-11)
+    ref = poisson(f)
+    err = np.linalg.norm(u - ref) / np.linalg.norm(ref)
+    assert cycles == 1 and rr <= 1e-11
+    assert err < 4 * EPS * np.log2(2 * n), err
+    assert np.all(u[0] == 0) and np.all(u[-1] == 0) and np.all(u[:, 0] == 0) and np.all(u[:, -1] == 0)
+
+
+def test_largest_transform_analytic_mode():
+    n = 4096
+    print(f"direct n={n}", flush=True)
+    x = np.arange(n + 1)
+    sx, sy = np.sin(3 * np.pi * x / n), np.sin(5 * np.pi * x / n)
+    lam = -4.0 * (n / L) ** 2 * (np.sin(3 * np.pi / (2 * n)) ** 2 + np.sin(5 * np.pi / (2 * n)) ** 2)
+    f = np.outer(sx, sy)
+    u, cycles, _ = pic2d.poisson_tol(f, length=L, tol=1e-7)
+    assert cycles == 1
+    assert np.linalg.norm(u - f / lam) < 4 * EPS * np.log2(2 * n) * np.linalg.norm(f / lam)
+
+
+@pytest.mark.parametrize("n", [16, 64, 256])
+def test_refinement_stops_at_rounding(n):
+    """a tolerance below rounding: solves are added while they halve the
+    residual, then the loop ends; the reported residual is the iterate's"""
+    x = np.sin(np.pi * np.arange(n + 1) / n)
+    f = np.outer(x, x)
+    u, cycles, rr = pic2d.poisson_tol(f, length=L, tol=1e-30, max_iter=40)
+    assert 1 <= cycles <= 8
+    assert abs(orc.relres(u, f, L) - rr) <= 1e-3 * rr
+    _, one, rr1 = pic2d.poisson_tol(f, length=L, tol=1e-30, max_iter=1)
+    assert one == 1 and rr <= 1.5 * rr1
+
+
+@pytest.mark.parametrize("n", [32, 128])
+def test_start_from_a_guess_with_wall_values(n):
+    """the guess's wall nodes are the solution's wall values.  f is 1e9 and u
+    about 1: rounding u moves A u by eps 8 (n/L)^2 = 3e-7 at 128, far below
+    tol |f| = 0.1"""
+    rng = np.random.default_rng(n)
+    f, u0 = 1e9 * rng.standard_normal((n + 1, n + 1)), rng.standard_normal((n + 1, n + 1))
+    u, cycles, rr = pic2d.poisson_tol(f, u0=u0, length=L, tol=1e-10)
+    assert cycles == 1 and rr <= 1e-10
+    edge = np.ones_like(f, dtype=bool)
+    edge[1:-1, 1:-1] = False
+    assert np.array_equal(u[edge], u0[edge])
+    # A u = f with these walls
+    r = f[1:-1, 1:-1] - (u[2:, 1:-1] + u[:-2, 1:-1] + u[1:-1, 2:] + u[1:-1, :-2]
+                         - 4 * u[1:-1, 1:-1]) * (n / L) ** 2
+    assert np.linalg.norm(r) <= 2e-10 * np.linalg.norm(f[1:-1, 1:-1])
+
+
+@pytest.mark.parametrize("cells", [32, 128])
+def test_steps_with_and_without_given_sweeps(cells):
+    """the library's choice (direct) and V-cycles asked for by mg_sweeps give
+    the potential of the same charge to the tolerance; a tolerance too tight
+    to be met by every first solve (verdict read per step) changes nothing"""
+    phi = []
+    for sweeps, tol in ((-1, 1e-9), (2, 1e-12), (-1, 1e-14)):
+        p = workloads.discharge(cells, 20, te=4.0)
+        p.mg_tol, p.mg_sweeps, p.mg_max_iter = tol, sweeps, 30
+        with pic2d.Pic(p) as sim:
+            sim.run(4)
+            cyc, total, rr = sim.mg_stats()
+            assert cyc >= 1 and total >= 4 and (rr <= tol or tol == 1e-14)
+            phi.append(sim.get_phi())
+    for x in phi[1:]:
+        assert np.linalg.norm(x - phi[0]) < 1e-9 * np.linalg.norm(phi[0])

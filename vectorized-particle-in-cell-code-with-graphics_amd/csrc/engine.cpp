@@ -87,29 +87,54 @@ long lds_limit() {
     return v;
 }
 
-int alloc_mg(pic_handle *h, MgLevels &M, int N) {
+// What solves the Poisson equation of a grid: the reference's FP64 multigrid,
+// the FP32 V-cycles with FP64 refinement, or the direct solve.  The tolerance
+// mode takes the direct solve unless the caller gave a sweep count for the
+// V-cycles (mg_sweeps) on a grid that has levels to sweep, or the grid is
+// beyond the direct solve's transforms.
+enum class Solver { FIXED, VCYCLE, DIRECT };
+Solver solver_for(int N, int mg_mode, int mg_sweeps) {
+    if (mg_mode != PIC_MG_TOL) return Solver::FIXED;
+    const bool levels = levels_of(N) - 1 > mg_coarse_level_for(lds_limit(), levels_of(N));
+    return direct_ok(N) && !(mg_sweeps > 0 && levels) ? Solver::DIRECT : Solver::VCYCLE;
+}
+
+int alloc_mg(pic_handle *h, MgLevels &M, int N, Solver what) {
     M.ng = levels_of(N);
     long lds = lds_limit();
     M.lds = lds;
     M.lc = mg_coarse_level_for(lds, M.ng);
+    const int top = M.ng - 1;
+    const size_t nf = (size_t)N * N;
+    CHECK(dalloc(h, &M.d.rhsF[top], nf));
+    CHECK(dalloc(h, &M.d.u[top], nf));
+    HIPCHK(h, hipMemset(M.d.u[top], 0, nf * sizeof(double)));  // cold start of the iterate
+    if (what == Solver::DIRECT) {
+        const int rc = direct_plan(M.dir, N, [&](double **p, size_t n) { return dalloc(h, p, n); });
+        if (rc == DIRECT_DEVICE) return seterr(h, PIC_ERR_DEVICE, "direct solve: tables");
+        return rc;
+    }
     mg_set_coarse_attr(lds);
-    if (mg_dst_tables(M) != 0) return seterr(h, PIC_ERR_ALLOC, "multigrid: coarse tables");
     for (int l = M.lc; l < M.ng; l++) {
         size_t s = (size_t)((1 << (l + 1)) + 1) * ((1 << (l + 1)) + 1);
-        CHECK(dalloc(h, &M.d.rhsF[l], s));
-        CHECK(dalloc(h, &M.d.u[l], s));
+        if (what == Solver::FIXED) {
+            if (l == top) continue;
+            CHECK(dalloc(h, &M.d.rhsF[l], s));
+            CHECK(dalloc(h, &M.d.u[l], s));
+            CHECK(dalloc(h, &M.d.cres[l], s));
+            CHECK(dalloc(h, &M.d.cv[l], s));
+            continue;
+        }
         CHECK(dalloc(h, &M.f.rhsF[l], s));
         CHECK(dalloc(h, &M.f.u[l], s));
         if (l > M.lc) CHECK(dalloc(h, &M.f.us[l], s));
-        if (l < M.ng - 1) {
-            CHECK(dalloc(h, &M.d.cres[l], s));
-            CHECK(dalloc(h, &M.d.cv[l], s));
+        if (l < top) {
             CHECK(dalloc(h, &M.f.cres[l], s));
             CHECK(dalloc(h, &M.f.cv[l], s));
         }
     }
-    size_t nf = (size_t)N * N;
-    HIPCHK(h, hipMemset(M.d.u[M.ng - 1], 0, nf * sizeof(double)));  // cold start of the iterate
+    if (what == Solver::FIXED) return PIC_OK;
+    if (mg_dst_tables(M) != 0) return seterr(h, PIC_ERR_ALLOC, "multigrid: coarse tables");
     M.nparts = (int)std::min<size_t>(1024, (nf + 255) / 256);
     // block partial sums: the residual pass's blocks, or one per tile of the
     // top level (the fused post-smoothing and residual kernel; tiles of 16 x
@@ -117,7 +142,6 @@ int alloc_mg(pic_handle *h, MgLevels &M, int N) {
     const size_t tiles = (size_t)((N + 15) / 16) * (size_t)((N + 15) / 16);
     CHECK(dalloc(h, &M.partials, 2 * std::max((size_t)M.nparts, tiles)));
     CHECK(dalloc(h, &M.r32alt, nf));
-    CHECK(dalloc(h, &M.uprev, nf));
     CHECK(dalloc(h, &M.flags, 4));
     HIPCHK(h, hipMemset(M.flags, 0, 4 * sizeof(int)));
     CHECK(dalloc(h, &M.ualt, nf));
@@ -139,6 +163,7 @@ void free_mg(MgLevels &M) {
     }
     M.d = MgArrays<double>();
     M.f = MgArrays<float>();
+    direct_free(M.dir);
     if (M.dst_S) hipFree(M.dst_S);
     if (M.dst_D) hipFree(M.dst_D);
     M.dst_S = M.dst_D = nullptr;
@@ -921,22 +946,47 @@ int absorb_species(pic_handle *h, int si, bool plop) {
     return PIC_OK;
 }
 
+// The direct solve's work after (or instead of) the first: while the
+// residual exceeds the tolerance, the residual is solved for and added, at
+// most `left` more times; a residual that does not halve is of rounding size
+// and ends it.  dir_pass launches k_phi_resid with a residual array (have_r:
+// the last one launched already had it); `used` counts the solves.
+int direct_refine(pic_handle *h, hipStream_t st, MgLevels &M, double length, double tol, int left,
+                  bool have_r, const std::function<void(double *)> &dir_pass, int *used,
+                  double *relres) {
+    const int top = M.ng - 1, N = M.dir.n + 1;
+    double last = 0.0;
+    for (int it = 0;; it++) {
+        if (direct_relres(st, M.dir, relres) != 0)
+            return seterr(h, PIC_ERR_DEVICE, "direct solve: stream error");
+        const bool stalled = it > 0 && !(*relres <= 0.5 * last);
+        if (*relres <= tol || it >= left || stalled) return PIC_OK;
+        last = *relres;
+        if (it == 0 && !have_r) {  // the residual itself
+            if (!M.dir.r64) CHECK(dalloc(h, &M.dir.r64, (size_t)N * N));
+            dir_pass(M.dir.r64);
+        }
+        direct_solve(st, M.dir, M.dir.r64, M.d.u[top], length, true);
+        (*used)++;
+        dir_pass(M.dir.r64);
+    }
+}
+
+// the residual of the last direct solve, which the step did not wait for:
+// read before anything reports the solver's figures
+int mg_harvest(pic_handle *h) {
+    if (!h->M.pending) return PIC_OK;
+    h->M.pending = 0;
+    if (direct_relres(h->st, h->M.dir, &h->mg_relres) != 0)
+        return seterr(h, PIC_ERR_DEVICE, "direct solve: stream error");
+    return PIC_OK;
+}
+
 // phi from the solve with the boundary values; with_e: E (and its fp32 copy
 // for the gather) from the same values in the same launch.  timestep: the
 // fused step's field_start has already formed the rhs, the extrapolated start
 // and the flag reset, and phi/E are queued before the host waits for the
 // last cycles (they take the final iterate by the cycle count's parity).
-// the verdict of a one-workgroup tolerance solve queued without a wait:
-// read before anything reports the solver's figures or starts another solve
-int mg_harvest(pic_handle *h) {
-    if (!h->M.pending) return PIC_OK;
-    const int used = mg_tol_verdict(h->M, &h->mg_relres);
-    if (used < 0) return seterr(h, PIC_ERR_DEVICE, "multigrid: stream error");
-    h->mg_cycles = used;
-    h->mg_cycles_total += used;
-    return PIC_OK;
-}
-
 int solve_potential(pic_handle *h, double phi0X, double phiR, double phi0Y, double phiLY,
                     bool with_e = false, bool timestep = false) {
     const pic_params &P = h->P;
@@ -950,6 +1000,28 @@ int solve_potential(pic_handle *h, double phi0X, double phiR, double phi0Y, doub
         launch_fold(h->st, h->rho, N, 1.0 / P.epsilon, phi0X, phiR, phi0Y, phiLY,
                     1.0 / (h->dx * h->dx), M.d.rhsF[M.ng - 1]);
     bool queued_e = false;
+    if (M.dir.n > 0) {
+        // phi (and E), then nothing is waited for where the first solve
+        // always meets the tolerance: its residual is read when reported
+        double *u = M.d.u[M.ng - 1];
+        const double *f = M.d.rhsF[M.ng - 1];
+        auto pass = [&](double *r64) {
+            launch_phi_resid(h->st, M.dir, u, f, phi0X, phiR, phi0Y, phiLY, P.length, h->dx, h->phi,
+                             with_e ? h->ex64 : nullptr, h->ey64, h->E32, r64);
+        };
+        direct_solve(h->st, M.dir, f, u, P.length, false);
+        pass(nullptr);
+        int used = 1;
+        if (direct_always_meets(N, P.mg_tol))
+            M.pending = 1;
+        else
+            CHECK(direct_refine(h, h->st, M, P.length, P.mg_tol, P.mg_max_iter - 1, false, pass,
+                                &used, &h->mg_relres));
+        h->mg_cycles = used;
+        h->mg_cycles_total += used;
+        h->have_phi = true;
+        return PIC_OK;
+    }
     if (P.mg_mode == PIC_MG_TOL) {
         const bool early = timestep && with_e;
         std::function<void(const double *, const double *)> phi_e;
@@ -958,15 +1030,11 @@ int solve_potential(pic_handle *h, double phi0X, double phiR, double phi0Y, doub
                 launch_phi_efield(h->st, u0, N, phi0X, phiR, phi0Y, phiLY, h->dx, h->phi,
                                   h->ex64, h->ey64, h->E32, u1, M.flags);
             };
-        CHECK(mg_harvest(h));
         int used = mg_tol_solve(h->st, M, P.length, P.mg_tol, P.mg_max_iter, &h->mg_relres,
                                 timestep, phi_e);
-        if (used < 0 && used != MG_PENDING)
-            return seterr(h, PIC_ERR_DEVICE, "multigrid: stream error");
-        if (used >= 0) {
-            h->mg_cycles = used;
-            h->mg_cycles_total += used;
-        }
+        if (used < 0) return seterr(h, PIC_ERR_DEVICE, "multigrid: stream error");
+        h->mg_cycles = used;
+        h->mg_cycles_total += used;
         queued_e = early;
     } else {
         mg_fixed_solve(h->st, M, P.mg_ncycle, P.length);
@@ -988,7 +1056,7 @@ int field_step(pic_handle *h, int64_t step) {
     double phiR = P.phi_right * cos(P.phi_period * (double)step);
     int p = prof_begin(h, 3);
     // rho, rhs, the tolerance solve's extrapolated start and flag reset
-    const bool tol = P.mg_mode == PIC_MG_TOL;
+    const bool tol = P.mg_mode == PIC_MG_TOL && M.dir.n == 0;
     int extrap = 0;
     if (tol) {
         extrap = M.have_prev ? 2 : 1;
@@ -1011,6 +1079,7 @@ int field_step(pic_handle *h, int64_t step) {
 int alloc_ref(pic_handle *h) {
     if (h->ref_phi) return PIC_OK;
     MgLevels &R = h->ref;
+    mg_set_coarse_attr(lds_limit());
     R.ng = h->M.ng;
     // the refinement V-cycles of the reference start above the level solved
     // in one workgroup (a grid that fits it whole, 65^2 with 160 KB of LDS,
@@ -1382,7 +1451,10 @@ int pic_create(const pic_params *Pin, int restart, const char *dump_dir, pic_han
     hipMemsetAsync(h->ex64, 0, 8ull * (N + 1) * (N + 1), h->st);
     hipMemsetAsync(h->ey64, 0, 8ull * (N + 1) * (N + 1), h->st);
     hipMemsetAsync(h->E32, 0, 8ull * ((N + 1) * N + 1), h->st);  // pic.cpp:1086: first gather sees E = 0
-    if ((rc = alloc_mg(h, h->M, N)) != PIC_OK) return fail(rc);
+    if ((rc = alloc_mg(h, h->M, N, solver_for(N, P.mg_mode, P.mg_sweeps))) != PIC_OK ||
+        (rc = dalloc(h, &h->M.uprev, (size_t)N * N)) != PIC_OK)
+        return fail(rc);
+    hipMemsetAsync(h->M.uprev, 0, 8ull * N * N, h->st);
     h->M.nu = P.mg_sweeps > 0 ? P.mg_sweeps : tuned_row(h->N).mg_sweeps;
     h->M.use_graphs = P.graphs != 0;
 
@@ -1518,7 +1590,6 @@ int pic_advance(pic_handle *h, int32_t nsteps) {
 int pic_sync(pic_handle *h) {
     if (!h) return set_global_error(PIC_ERR_ARG, "null handle");
     HIPCHK(h, hipStreamSynchronize(h->st));
-    CHECK(mg_harvest(h));
     return check_overflow(h, true);
 }
 
@@ -1767,7 +1838,7 @@ int pic_mglin(double *u, int32_t n, int32_t ncycle, double length) {
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
         return set_global_error(PIC_ERR_DEVICE, "no HIP device available");
     pic_handle tmp;
-    int rc = alloc_mg(&tmp, tmp.M, n);
+    int rc = alloc_mg(&tmp, tmp.M, n, Solver::FIXED);
     hipStream_t st = nullptr;
     if (rc == PIC_OK && hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess)
         rc = set_global_error(PIC_ERR_DEVICE, "stream");
@@ -1795,7 +1866,7 @@ int pic_poisson_tol(const double *f, double *u, int32_t n, double length, double
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
         return set_global_error(PIC_ERR_DEVICE, "no HIP device available");
     pic_handle tmp;
-    int rc = alloc_mg(&tmp, tmp.M, n);
+    int rc = alloc_mg(&tmp, tmp.M, n, solver_for(n, PIC_MG_TOL, -1));
     hipStream_t st = nullptr;
     if (rc == PIC_OK && hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess)
         rc = set_global_error(PIC_ERR_DEVICE, "stream");
@@ -1805,11 +1876,24 @@ int pic_poisson_tol(const double *f, double *u, int32_t n, double length, double
         hipMemcpyAsync(M.d.rhsF[M.ng - 1], f, bytes, hipMemcpyHostToDevice, st);
         hipMemcpyAsync(M.d.u[M.ng - 1], u, bytes, hipMemcpyHostToDevice, st);
         double rr = 0.0;
-        int used = mg_tol_solve(st, M, length, tol, max_iter, &rr);
-        if (used == MG_PENDING) used = mg_tol_verdict(M, &rr);
+        int used = 0;
+        if (M.dir.n > 0) {
+            // from the caller's guess: its residual, then corrections
+            auto pass = [&](double *r64) {
+                launch_phi_resid(st, M.dir, M.d.u[M.ng - 1], M.d.rhsF[M.ng - 1], 0.0, 0.0, 0.0, 0.0,
+                                 length, 0.0, nullptr, nullptr, nullptr, nullptr, r64);
+            };
+            rc = dalloc(&tmp, &M.dir.r64, (size_t)n * n);
+            if (rc == PIC_OK) {
+                pass(M.dir.r64);
+                rc = direct_refine(&tmp, st, M, length, tol, max_iter, true, pass, &used, &rr);
+            }
+        } else {
+            used = mg_tol_solve(st, M, length, tol, max_iter, &rr);
+        }
         hipMemcpyAsync(u, M.d.u[M.ng - 1], bytes, hipMemcpyDeviceToHost, st);
         hipError_t e = hipStreamSynchronize(st);
-        if (e != hipSuccess || used < 0)
+        if (rc == PIC_OK && (e != hipSuccess || used < 0))
             rc = set_global_error(PIC_ERR_DEVICE, e != hipSuccess ? hipGetErrorString(e) : "mg");
         if (cycles) *cycles = used;
         if (relres) *relres = rr;
@@ -2537,6 +2621,7 @@ int pic_checkpoint_read(pic_handle *h, const char *path) {
         return true;
     };
     HIPCHK(h, hipStreamSynchronize(h->st));
+    h->M.pending = 0;  // the read state brings its own figures
     CkHeader H;
     pic_params P;
     if (!get(&H, sizeof(H)) || memcmp(H.magic, CK_MAGIC, 8) != 0 || H.version != CK_VERSION ||

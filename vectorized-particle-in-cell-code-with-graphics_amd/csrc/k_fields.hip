@@ -528,82 +528,12 @@ __global__ void __launch_bounds__(1024)
 // transform: with S[p][q] = sin(pi (p+1)(q+1)/M) (S S = M/2 I) and
 // lambda_k = -4 sin^2(pi (k+1) / 2M), the solution of A u = f on the m = M-1
 // interior nodes is u = (2/M)^2 S ((S f S) ./ ((lambda_p + lambda_q)/h^2)) S:
-// four M x M products, done here in LDS by one workgroup (2x2 register tiles,
-// fp32).  It replaces the coarse V-cycle of the tolerance mode's correction
-// solve; the FP64 refinement around it is unchanged.
+// four 64 x 64 products (M = 64: the 65^2 level, below which the direct solve
+// of k_direct.hip takes the whole grid), done here in LDS by one workgroup on
+// the matrix cores.  It replaces the coarse V-cycle of the tolerance mode's
+// correction solve; the FP64 refinement around it is unchanged.
 
-// C = A B for M x M matrices in LDS, rows ld floats apart (M, ld multiples
-// of 4, M <= 64): thread t < (M/4)^2 computes a 4x4 tile, per k four
-// broadcast reads of A and one float4 of B feeding 16 FMAs.  Ends with a
-// barrier.
-__device__ void lds_gemm(const float *A, const float *B, float *C, int M, int ld) {
-    const int T = M >> 2;
-    const int t = threadIdx.x;
-    if (t < T * T) {
-        const int ti = t / T, tj = t - (t / T) * T;
-        const float *a = A + (4 * ti) * ld;
-        float c[4][4] = {};
-        for (int k = 0; k < M; k += 4) {  // four k per step: float4 reads of A and B
-            float4 ar[4], br[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                ar[r] = *reinterpret_cast<const float4 *>(a + r * ld + k);
-                br[r] = *reinterpret_cast<const float4 *>(B + (k + r) * ld + 4 * tj);
-            }
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                const float4 b = br[kk];
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float x = kk == 0 ? ar[r].x : kk == 1 ? ar[r].y : kk == 2 ? ar[r].z : ar[r].w;
-                    c[r][0] = fmaf(x, b.x, c[r][0]);
-                    c[r][1] = fmaf(x, b.y, c[r][1]);
-                    c[r][2] = fmaf(x, b.z, c[r][2]);
-                    c[r][3] = fmaf(x, b.w, c[r][3]);
-                }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            *reinterpret_cast<float4 *>(C + (4 * ti + r) * ld + 4 * tj) =
-                make_float4(c[r][0], c[r][1], c[r][2], c[r][3]);
-    }
-    __syncthreads();
-}
-
-// The same product on the matrix cores (M a multiple of 16): one 16 x 16
-// block of C per wavefront, v_mfma_f32_16x16x4f32 over k.  Lane layout of
-// the instruction: A[i][k] in lane i + 16 k, B[k][j] in lane j + 16 k,
-// C[i][j] in lane j + 16 (i / 4), register i % 4.  A row stride ld = M + 4
-// keeps the 16 rows of an A fragment on 8 banks (2-way at most).  Ends with
-// a barrier.
 typedef float mf4 __attribute__((ext_vector_type(4)));
-__device__ void lds_gemm_mfma(const float *A, const float *B, float *C, int M, int ld) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    const int nb = M >> 4, li = lane & 15, lk = lane >> 4;
-    for (int blk = w; blk < nb * nb; blk += nw) {
-        const int bi = blk / nb, bj = blk - (blk / nb) * nb;
-        const float *a = A + (16 * bi + li) * ld + lk;
-        const float *b = B + lk * ld + 16 * bj + li;
-        mf4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int k = 0; k < M; k += 4)
-            c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], b[k * ld], c, 0, 0, 0);
-        float *o = C + (16 * bi + 4 * lk) * ld + 16 * bj + li;
-        o[0] = c[0];
-        o[ld] = c[1];
-        o[2 * ld] = c[2];
-        o[3 * ld] = c[3];
-    }
-    __syncthreads();
-}
-
-// the products of the unfolded DST (M < 64; M = 64 takes dstf_solve)
-__device__ __forceinline__ void dst_gemm(const float *A, const float *B, float *C, int M, int ld) {
-    if ((M & 15) == 0)
-        lds_gemm_mfma(A, B, C, M, ld);
-    else
-        lds_gemm(A, B, C, M, ld);
-}
 
 // LDS floats of the DST solve: three M x M matrices with row stride M + 4
 __host__ __device__ inline long dst_lds_floats(int M) { return 3L * M * (M + 4); }
@@ -627,8 +557,9 @@ __host__ __device__ inline long dstf_table_floats() { return 2L * 32 * DSTF_LDH;
 
 // one 16 x 16 block of C = A B with k = 32 on the matrix cores; A(i, k) is
 // A[k lda + i] when AT, else A[i lda + k]; B(k, j) is B[j ldb + k] when BT,
-// else B[k ldb + j] (operands offset to the block); the lane layout of
-// v_mfma_f32_16x16x4f32 as in lds_gemm_mfma
+// else B[k ldb + j] (operands offset to the block).  Lane layout of
+// v_mfma_f32_16x16x4f32: A[i][k] in lane i + 16 k, B[k][j] in lane j + 16 k,
+// C[i][j] in lane j + 16 (i / 4), register i % 4
 template <bool AT, bool BT>
 __device__ __forceinline__ void dstf_block(const float *A, int lda, const float *B, int ldb,
                                            float *C, int ldc) {
@@ -754,29 +685,11 @@ __device__ void dst_solve(const float *__restrict__ rhs_in, float *__restrict__ 
         const int p = k >> (lc + 1), q = k & (M - 1);
         X[p * ld + q] = (p < M - 1 && q < M - 1) ? rhs_in[(p + 1) * n + q + 1] : 0.0f;
     }
-    if (M == 64) {  // the folded tables (dstf_solve), in S's space
-        for (int k = threadIdx.x; k < 2048; k += blockDim.x)
-            S[(k >> 10) * 32 * DSTF_LDH + ((k >> 5) & 31) * DSTF_LDH + (k & 31)] = Sg[k];
-        __syncthreads();
-        dstf_solve(X, Y, S, dk, ld);  // X = u on the interior
-    } else {
-        for (int k = threadIdx.x; k < M * M; k += blockDim.x)
-            S[(k >> (lc + 1)) * ld + (k & (M - 1))] = Sg[k];
-        __syncthreads();
-        dst_gemm(S, X, Y, M, ld);  // Y = S f
-        dst_gemm(Y, S, X, M, ld);  // X = S f S
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int k = threadIdx.x + r * blockDim.x;
-            if (k < M * M) {
-                const int p = k >> (lc + 1), q = k & (M - 1);
-                X[p * ld + q] = X[p * ld + q] * dk[r];
-            }
-        }
-        __syncthreads();
-        dst_gemm(S, X, Y, M, ld);
-        dst_gemm(Y, S, X, M, ld);  // X = u on the interior
-    }
+    // the folded tables (dstf_solve), in S's space
+    for (int k = threadIdx.x; k < 2048; k += blockDim.x)
+        S[(k >> 10) * 32 * DSTF_LDH + ((k >> 5) & 31) * DSTF_LDH + (k & 31)] = Sg[k];
+    __syncthreads();
+    dstf_solve(X, Y, S, dk, ld);  // X = u on the interior
     for (int k = threadIdx.x; k < n * n; k += blockDim.x) {
         const int i = k / n, j = k - (k / n) * n;
         const bool in = i > 0 && j > 0 && i < n - 1 && j < n - 1;
@@ -1051,41 +964,30 @@ static void coarse_dst_launch(hipStream_t st, const MgLevels &M, const float *rh
                        st, rhs, u, lc, (float)(h * h), M.dst_S, M.dst_D, skip);
 }
 
+// the folded form's tables (dstf_solve) of the 65^2 level: H1 (odd frequencies
+// a = 2i+1) and H2 (even a = 2i+2) over b = p+1, the scale in split order
 int mg_dst_tables(MgLevels &M) {
-    const int m = 1 << (M.lc + 1);
+    const int m = 64;
+    if (M.lc != 5) return -1;  // levels below 65^2 fit the LDS limit
     const double pi = 3.14159265358979323846;
-    std::vector<float> S((size_t)m * m, 0.0f), D((size_t)m * m, 0.0f);
-    for (int p = 0; p < m - 1; p++) {
-        double lp = -4.0 * std::pow(std::sin(pi * (p + 1) / (2.0 * m)), 2);
-        for (int q = 0; q < m - 1; q++) {
-            // (p+1)(q+1) mod 2m keeps the sine argument small
-            long r = ((long)(p + 1) * (q + 1)) % (2L * m);
-            S[(size_t)p * m + q] = (float)std::sin(pi * (double)r / (double)m);
-            double lq = -4.0 * std::pow(std::sin(pi * (q + 1) / (2.0 * m)), 2);
-            D[(size_t)p * m + q] = (float)((2.0 / m) * (2.0 / m) / (lp + lq));
+    // a b mod 2m keeps the sine argument small
+    auto sinab = [&](long a, long b) {
+        return (float)std::sin(pi * (double)((a * b) % (2L * m)) / (double)m);
+    };
+    std::vector<float> S(2048, 0.0f), D((size_t)m * m, 0.0f);
+    for (int i = 0; i < 32; i++)
+        for (int p = 0; p < 32; p++) {
+            S[i * 32 + p] = sinab(2 * i + 1, p + 1);
+            if (i < 31 && p < 31) S[1024 + i * 32 + p] = sinab(2 * i + 2, p + 1);
         }
-    }
-    if (m == 64) {
-        // the folded form (dstf_solve): H1 (odd frequencies a = 2i+1) and H2
-        // (even a = 2i+2) over b = p+1, then the scale in split order
-        auto sinab = [&](long a, long b) {
-            return (float)std::sin(pi * (double)((a * b) % (2L * m)) / (double)m);
-        };
-        std::vector<float> H(2048, 0.0f), Ds((size_t)m * m, 0.0f);
-        for (int i = 0; i < 32; i++)
-            for (int p = 0; p < 32; p++) {
-                H[i * 32 + p] = sinab(2 * i + 1, p + 1);
-                if (i < 31 && p < 31) H[1024 + i * 32 + p] = sinab(2 * i + 2, p + 1);
-            }
-        // split index -> natural frequency index (a - 1), -1: none
-        auto nat = [](int r) { return r < 32 ? 2 * r : (r < 63 ? 2 * (r - 32) + 1 : -1); };
-        for (int r = 0; r < m; r++)
-            for (int c = 0; c < m; c++)
-                if (nat(r) >= 0 && nat(c) >= 0)
-                    Ds[(size_t)r * m + c] = D[(size_t)nat(r) * m + nat(c)];
-        S.swap(H);
-        D.swap(Ds);
-    }
+    // split index -> natural frequency index (a - 1), -1: none
+    auto nat = [](int r) { return r < 32 ? 2 * r : (r < 63 ? 2 * (r - 32) + 1 : -1); };
+    auto lam = [&](int a) { return -4.0 * std::pow(std::sin(pi * (a + 1) / (2.0 * m)), 2); };
+    for (int r = 0; r < m; r++)
+        for (int c = 0; c < m; c++)
+            if (nat(r) >= 0 && nat(c) >= 0)
+                D[(size_t)r * m + c] =
+                    (float)((2.0 / m) * (2.0 / m) / (lam(nat(r)) + lam(nat(c))));
     if (hipMalloc((void **)&M.dst_S, S.size() * sizeof(float)) != hipSuccess ||
         hipMalloc((void **)&M.dst_D, D.size() * sizeof(float)) != hipSuccess)
         return -1;
@@ -1150,22 +1052,11 @@ int mg_coarse_level_for(long lds_bytes, int ng) {
     return lc;
 }
 
-template <bool FOLD>
-__global__ void __launch_bounds__(1024)
-    k_tol_solve_dst(double *__restrict__ ug, const double *__restrict__ fg, int n, double h2i,
-                    int lc, float h2, const float *__restrict__ Sg, const float *__restrict__ Dg,
-                    double tol, int max_cycles, int *__restrict__ flags,
-                    double *__restrict__ relres_host, int *__restrict__ host_flags);
-
 void mg_set_coarse_attr(long lds_bytes) {
     hipFuncSetAttribute((const void *)k_mg_coarse<double>,
                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     hipFuncSetAttribute((const void *)k_mg_coarse_dst, hipFuncAttributeMaxDynamicSharedMemorySize,
                         (int)lds_bytes);
-    hipFuncSetAttribute((const void *)k_tol_solve_dst<true>,
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-    hipFuncSetAttribute((const void *)k_tol_solve_dst<false>,
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     hipFuncSetAttribute((const void *)k_mg_coarse<float>,
                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
 }
@@ -1460,158 +1351,6 @@ static hipError_t wait_published(hipStream_t st, MgLevels &M, int passes) {
     return wait_flags(M, passes);
 }
 
-int mg_tol_verdict(MgLevels &M, double *relres_out) {
-    const int passes = M.pending;
-    if (passes <= 0) return -1;
-    M.pending = 0;
-    if (wait_flags(M, passes) != hipSuccess) return -1;
-    const bool conv = (__atomic_load_n(&M.host_flags[2], __ATOMIC_ACQUIRE) & MG_PUB_CONV) != 0;
-    const int used = M.host_flags[1];
-    M.pred = used + (conv ? 0 : 1);
-    if (relres_out) *relres_out = *M.relres;
-    return used;
-}
-
-// The whole tolerance solve of a grid whose finest level is the DST level
-// (65^2 and below: C1, the small runs of ensembles and serving), in one
-// workgroup of 1024 threads, everything resident in LDS: the FP64 iterate
-// and right-hand side, the sine table, and the FP32 residual / correction
-// matrix R with its product scratch W (the layout of dst_solve's X and Y:
-// node (i, j) of the interior at R[(i-1) ld + (j-1)]).  The initial residual,
-// then per cycle the exact DST solve of R in place, the update u += e and
-// the residual of the updated iterate into R -- the arithmetic of
-// k_mg_coarse_dst and k_tol_update node for node, each thread summing its
-// nodes in ascending order as there, so iterates, residuals and cycle
-// counts are the launched cycles' -- until ||f - Au|| <= tol ||f|| or
-// max_cycles cycles.  The final iterate is written to u; the verdict is
-// published as k_tol_finish publishes it, once, at the end.  One launch per
-// solve and no host wait: these grids are bound by latency.
-#define SMALL_NPT 5  // nodes per thread: n^2 <= 5 x 1024 for n <= 65
-
-__host__ __device__ inline long tol_small_lds_bytes(int m) {
-    const long n = m + 1;
-    return (2 * n * n + 16) * (long)sizeof(double) + dst_lds_floats(m) * (long)sizeof(float);
-}
-
-__device__ __forceinline__ double block_sum_1024(double v, double *ws) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) ws[w] = v;
-    __syncthreads();
-    double t = 0.0;
-    for (int k = 0; k < (int)(blockDim.x >> 6); k++) t += ws[k];  // fixed order
-    __syncthreads();
-    return t;
-}
-
-template <bool FOLD>
-__global__ void __launch_bounds__(1024)
-    k_tol_solve_dst(double *__restrict__ ug, const double *__restrict__ fg, int n, double h2i,
-                    int lc, float h2, const float *__restrict__ Sg, const float *__restrict__ Dg,
-                    double tol, int max_cycles, int *__restrict__ flags,
-                    double *__restrict__ relres_host, int *__restrict__ host_flags) {
-    const int m = 1 << (lc + 1), ld = m + 4, nn = n * n;
-    // no static LDS: the attribute grants the dynamic region the whole
-    // per-workgroup limit
-    extern __shared__ double lds_raw[];
-    double *U = lds_raw, *F = U + nn, *ws = F + nn;
-    float *S = reinterpret_cast<float *>(ws + 16), *R = S + m * ld, *W = R + m * ld;
-    // this thread's nodes: k = threadIdx.x + r * 1024; o[r] = its R slot, or
-    // -1 off the interior (and past the grid)
-    int o[SMALL_NPT];
-    double ff = 0.0;
-#pragma unroll
-    for (int r = 0; r < SMALL_NPT; r++) {
-        const int k = (int)threadIdx.x + r * 1024;
-        o[r] = -1;
-        if (k < nn) {
-            const int i = k / n, j = k - (k / n) * n;
-            if (i > 0 && j > 0 && i < n - 1 && j < n - 1) o[r] = (i - 1) * ld + (j - 1);
-            const double fk = fg[k];
-            U[k] = ug[k];
-            F[k] = fk;
-            if (o[r] >= 0) ff += fk * fk;
-        }
-    }
-    float dk[4];  // the eigenvalue scale of this thread's R entries
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int k = (int)threadIdx.x + r * 1024;
-        dk[r] = k < m * m ? Dg[k] * h2 : 0.0f;
-    }
-    for (int k = (int)threadIdx.x; k < m * ld; k += 1024) R[k] = 0.0f;
-    if (FOLD)  // m = 64: the folded tables (dstf_solve)
-        for (int k = (int)threadIdx.x; k < 2048; k += 1024)
-            S[(k >> 10) * 32 * DSTF_LDH + ((k >> 5) & 31) * DSTF_LDH + (k & 31)] = Sg[k];
-    else
-        for (int k = (int)threadIdx.x; k < m * m; k += 1024)
-            S[(k >> (lc + 1)) * ld + (k & (m - 1))] = Sg[k];
-    ff = block_sum_1024(ff, ws);  // its barriers also publish U, F, S and R
-    // the residual of U into R, its sum of squares
-    auto residual = [&]() -> double {
-        double rr = 0.0;
-#pragma unroll
-        for (int r = 0; r < SMALL_NPT; r++) {
-            const int k = (int)threadIdx.x + r * 1024;
-            if (o[r] >= 0) {
-                // the stencil of resid_node: north, south, east, west
-                const double res =
-                    -h2i * (U[k + n] + U[k - n] + U[k + 1] + U[k - 1] - 4.0 * U[k]) + F[k];
-                rr += res * res;
-                R[o[r]] = (float)res;
-            }
-        }
-        return block_sum_1024(rr, ws);
-    };
-    double rr = residual();
-    double rel = (ff > 0.0) ? sqrt(rr / ff) : sqrt(rr);
-    int q = 0;
-    while (!(rel <= tol) && q < max_cycles) {  // uniform: every thread holds the same sums
-        if (FOLD) {
-            dstf_solve(R, W, S, dk, ld);  // R = e on the interior
-        } else {
-            dst_gemm(S, R, W, m, ld);  // W = S r
-            dst_gemm(W, S, R, m, ld);  // R = S r S
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int k = (int)threadIdx.x + r * 1024;
-                if (k < m * m) {
-                    const int p = k >> (lc + 1), c = k & (m - 1);
-                    R[p * ld + c] = R[p * ld + c] * dk[r];
-                }
-            }
-            __syncthreads();
-            dst_gemm(S, R, W, m, ld);
-            dst_gemm(W, S, R, m, ld);  // R = e on the interior
-        }
-#pragma unroll
-        for (int r = 0; r < SMALL_NPT; r++) {
-            const int k = (int)threadIdx.x + r * 1024;
-            if (o[r] >= 0) U[k] = U[k] + (double)R[o[r]];
-        }
-        __syncthreads();
-        rr = residual();
-        rel = (ff > 0.0) ? sqrt(rr / ff) : sqrt(rr);
-        q++;
-    }
-#pragma unroll
-    for (int r = 0; r < SMALL_NPT; r++) {
-        const int k = (int)threadIdx.x + r * 1024;
-        if (o[r] >= 0) ug[k] = U[k];
-    }
-    if (threadIdx.x == 0) {
-        const int conv = rel <= tol;
-        flags[0] = conv;
-        flags[1] = q;
-        flags[3] = 1 + q;
-        *relres_host = rel;
-        host_flags[0] = conv;
-        host_flags[1] = q;
-        __threadfence_system();
-        host_flags[2] = (1 + q) | (conv ? MG_PUB_CONV : 0);
-    }
-}
-
 int mg_tol_solve(hipStream_t st, MgLevels &M, double length, double tol, int max_iter,
                  double *relres_out, bool flags_reset,
                  const std::function<void(const double *, const double *)> &after_batch) {
@@ -1629,10 +1368,10 @@ int mg_tol_solve(hipStream_t st, MgLevels &M, double length, double tol, int max
     // the top post leg fused with the residual pass saves a launch per cycle
     // where the levels are latency-bound; at 1025^2 the wider halo's extra
     // reads cost more than the launch (measured), so the passes stay apart
-    const bool fuse_top = lf > M.lc && n <= 513;
+    const bool fuse_top = n <= 513;
     // residual-pass blocks of a cycle (the partials its verdict sums)
     const int top_tiles = (n + mg_tile(n) - 1) / mg_tile(n);
-    const int cyc_nb = (lf > M.lc && fuse_top) ? top_tiles * top_tiles : M.nparts;
+    const int cyc_nb = fuse_top ? top_tiles * top_tiles : M.nparts;
     // vfirst: the verdict of the residual pass before this cycle (the
     // solve's initial pass, or the previous cycle's) is formed by this
     // cycle's first kernel, else k_tol_finish formed it after the pass; fin:
@@ -1643,44 +1382,23 @@ int mg_tol_solve(hipStream_t st, MgLevels &M, double length, double tol, int max
                                                   queued > 0 ? 1 : 0, M.flags, M.relres,
                                                   M.host_flags}
                                      : TolVerdict{};
-        if (lf > M.lc && !fuse_top) {
+        if (!fuse_top) {
             vcycle_fused(st, M, lf, e32, r32, length, skip, vd);
             hipLaunchKernelGGL(k_tol_update, dim3(M.nparts), dim3(TOL_THREADS), 0, st,
                                (const double *)buf[queued & 1], (const float *)e32,
                                buf[(queued + 1) & 1], f, n, h2i, r32, M.partials, M.flags);
             if (fin) tol_finish_launch(st, M, M.nparts, tol, true);
-        } else if (lf == M.lc) {
-            coarse_dst_launch(st, M, r32, e32, length, skip);
-            hipLaunchKernelGGL(k_tol_update, dim3(M.nparts), dim3(TOL_THREADS), 0, st,
-                               (const double *)buf[queued & 1], (const float *)e32,
-                               buf[(queued + 1) & 1], f, n, h2i, r32, M.partials, M.flags);
-            tol_finish_launch(st, M, M.nparts, tol, true);
         } else {
             vcycle_top(st, M, lf, rb[queued & 1], buf[queued & 1], buf[(queued + 1) & 1], f, h2i,
                        rb[(queued + 1) & 1], tol, length, vd, fin);
         }
     };
-    // the coarsest-level branch keeps k_tol_finish after every pass, and so
-    // does a solve allowed no cycles
-    const bool vfuse = lf > M.lc && max_iter > 0;
+    // a solve allowed no cycles keeps k_tol_finish
+    const bool vfuse = max_iter > 0;
     // nothing on the device writes the host copies now (the last solve's
     // remaining cycles were skipped): clear them for this solve's verdict
-    if (M.pending && mg_tol_verdict(M, nullptr) < 0) return -1;
     __atomic_store_n(&M.host_flags[2], 0, __ATOMIC_RELEASE);
     M.host_flags[0] = M.host_flags[1] = 0;
-    if (lf == M.lc && n * n <= SMALL_NPT * 1024 && tol_small_lds_bytes(n - 1) <= M.lds) {
-        // the whole solve in one workgroup (k_tol_solve_dst)
-        const int m = n - 1;
-        const double hc = length / (double)m;
-        hipLaunchKernelGGL((m == 64 ? k_tol_solve_dst<true> : k_tol_solve_dst<false>), dim3(1),
-                           dim3(1024), (size_t)tol_small_lds_bytes(m),
-                           st, u, f, n, h2i, M.lc, (float)(hc * hc), M.dst_S, M.dst_D, tol,
-                           max_iter, M.flags, M.relres, M.host_flags);
-        if (after_batch) after_batch(u, u);
-        if (hipEventRecord(M.done, st) != hipSuccess) return -1;
-        M.pending = 1 + max_iter;
-        return MG_PENDING;
-    }
     if (!flags_reset) hipLaunchKernelGGL(k_tol_reset, dim3(1), dim3(1), 0, st, M.flags);
     hipLaunchKernelGGL(k_tol_update, dim3(M.nparts), dim3(TOL_THREADS), 0, st, (const double *)u,
                        (const float *)nullptr, (double *)nullptr, f, n, h2i, r32, M.partials,

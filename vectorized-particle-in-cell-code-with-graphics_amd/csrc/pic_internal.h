@@ -93,7 +93,19 @@ struct MgArrays {
 #define MG_PUB_COUNT 0x3FFFFFFF
 #define MG_PUB_CONV 0x40000000
 
+// Direct FP64 solve by fast sine transforms (k_direct.hip) of a grid of n + 1
+// nodes per side: tables (twiddles exp(-2 pi i k / 2n), then 4 sin^2(pi k /
+// 2n), k = 0..n), the transform between its launches (n > 64), the residual
+// where it is solved for again, and the block sums of r^2 and f^2 (nparts
+// pairs) with their pinned host copy
+struct DirectPlan {
+    int n = 0, nparts = 0;
+    double *table = nullptr, *T = nullptr, *r64 = nullptr;
+    double *parts = nullptr, *parts_host = nullptr;
+};
+
 struct MgLevels {
+    DirectPlan dir;      // tolerance mode without given sweeps (dir.n > 0)
     int ng = 0, lc = 0;
     long lds = 0;        // LDS bytes a workgroup may allocate on this device
     MgArrays<double> d;  // FP64 full multigrid (fixed mode) and the FP64 iterate
@@ -110,12 +122,11 @@ struct MgLevels {
     double *relres = nullptr;    // pinned host: last relative residual
     int *host_flags = nullptr;   // pinned host copy of flags
     int pred = 4;                // predicted V-cycles per solve
-    int pending = 0;             // passes a queued one-workgroup solve publishes (0: none)
-    // exact coarsest-level solve of the tolerance mode: discrete sine
-    // transform tables of level lc, M x M with M = 2^(lc+1) (padded by one)
-    float *dst_S = nullptr;      // S[p][q] = sin(pi (p+1)(q+1) / M); M = 64: the folded halves
-    float *dst_D = nullptr;      // (2/M)^2 / (lambda_p + lambda_q), h^2 applied in the kernel
-                                 // (M = 64: rows and columns in the folded, split order)
+    int pending = 0;             // a direct solve's residual has not been read yet
+    // exact solve of the V-cycles' coarsest level (65^2): the folded halves of
+    // the discrete sine transform and (2/64)^2 / (lambda_p + lambda_q) in their
+    // split order, h^2 applied in the kernel
+    float *dst_S = nullptr, *dst_D = nullptr;
     int nu = 2;                  // red-black sweeps per leg of the fused V-cycle
     hipEvent_t done = nullptr;   // end of a queued batch of cycles (host wait)
     // tolerance mode: a batch of k cycles from a given parity and iterate
@@ -381,14 +392,25 @@ int field_diff_sums(hipStream_t st, const double *a0, const double *b0, const do
 int mg_tol_solve(hipStream_t st, MgLevels &M, double length, double tol, int max_iter,
                  double *relres_out, bool flags_reset = false,
                  const std::function<void(const double *, const double *)> &after_batch = nullptr);
-// A grid whose finest level is the DST level (lf == lc) is solved whole by
-// one kernel that leaves the final iterate in M.d.u[ng-1]: mg_tol_solve then
-// queues it, and after_batch, without waiting and returns MG_PENDING;
-// mg_tol_verdict waits for that solve's verdict and returns its V-cycles (-1
-// on a HIP error or with no solve pending).  mg_tol_solve reads a pending
-// verdict itself (and drops it) before it starts another solve.
-constexpr int MG_PENDING = -2;
-int mg_tol_verdict(MgLevels &M, double *relres_out);
 
+// ---- k_direct.hip
+constexpr int DIRECT_DEVICE = -1000;
+bool direct_ok(int N);  // grids the direct solve takes
+// whether one solve always reaches ||f - Au|| <= tol ||f||
+bool direct_always_meets(int N, double tol);
+int direct_plan(DirectPlan &D, int N, const std::function<int(double **, size_t)> &alloc);
+void direct_free(DirectPlan &D);
+// A u = f on the interior (add: u += A^-1 f); boundary nodes are not touched
+void direct_solve(hipStream_t st, const DirectPlan &D, const double *f, double *u, double length,
+                  bool add);
+// phi and (ex64 given) E of the iterate u, with r64 its FP64 residual; the
+// block sums of the residual's norm to D.parts
+void launch_phi_resid(hipStream_t st, const DirectPlan &D, const double *u, const double *f,
+                      double phi0X, double phiR, double phi0Y, double phiLY, double length,
+                      double dx, double *phi, double *ex64, double *ey64, float2 *E32,
+                      double *r64);
+// the relative residual of the last launch_phi_resid (waits for the stream;
+// -1 on an error)
+int direct_relres(hipStream_t st, const DirectPlan &D, double *relres);
 
 }  // namespace pic
