@@ -78,15 +78,6 @@ int levels_of(int n) {
     return ng;
 }
 
-long lds_limit() {
-    int dev = 0, v = 0;
-    hipGetDevice(&dev);
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-        v <= 0)
-        v = 65536;
-    return v;
-}
-
 // What solves the Poisson equation of a grid: the reference's FP64 multigrid,
 // the FP32 V-cycles with FP64 refinement, or the direct solve.  The tolerance
 // mode takes the direct solve unless the caller gave a sweep count for the
@@ -95,15 +86,13 @@ long lds_limit() {
 enum class Solver { FIXED, VCYCLE, DIRECT };
 Solver solver_for(int N, int mg_mode, int mg_sweeps) {
     if (mg_mode != PIC_MG_TOL) return Solver::FIXED;
-    const bool levels = levels_of(N) - 1 > mg_coarse_level_for(lds_limit(), levels_of(N));
+    const bool levels = levels_of(N) - 1 > mg_coarse_level_for(levels_of(N));
     return direct_ok(N) && !(mg_sweeps > 0 && levels) ? Solver::DIRECT : Solver::VCYCLE;
 }
 
 int alloc_mg(pic_handle *h, MgLevels &M, int N, Solver what) {
     M.ng = levels_of(N);
-    long lds = lds_limit();
-    M.lds = lds;
-    M.lc = mg_coarse_level_for(lds, M.ng);
+    M.lc = mg_coarse_level_for(M.ng);
     const int top = M.ng - 1;
     const size_t nf = (size_t)N * N;
     CHECK(dalloc(h, &M.d.rhsF[top], nf));
@@ -114,15 +103,14 @@ int alloc_mg(pic_handle *h, MgLevels &M, int N, Solver what) {
         if (rc == DIRECT_DEVICE) return seterr(h, PIC_ERR_DEVICE, "direct solve: tables");
         return rc;
     }
-    mg_set_coarse_attr(lds);
     for (int l = M.lc; l < M.ng; l++) {
         size_t s = (size_t)((1 << (l + 1)) + 1) * ((1 << (l + 1)) + 1);
         if (what == Solver::FIXED) {
+            CHECK(dalloc(h, &M.d.cv[l], s));
             if (l == top) continue;
             CHECK(dalloc(h, &M.d.rhsF[l], s));
             CHECK(dalloc(h, &M.d.u[l], s));
             CHECK(dalloc(h, &M.d.cres[l], s));
-            CHECK(dalloc(h, &M.d.cv[l], s));
             continue;
         }
         CHECK(dalloc(h, &M.f.rhsF[l], s));
@@ -1079,21 +1067,17 @@ int field_step(pic_handle *h, int64_t step) {
 int alloc_ref(pic_handle *h) {
     if (h->ref_phi) return PIC_OK;
     MgLevels &R = h->ref;
-    mg_set_coarse_attr(lds_limit());
     R.ng = h->M.ng;
     // the refinement V-cycles of the reference start above the level solved
-    // in one workgroup (a grid that fits it whole, 65^2 with 160 KB of LDS,
-    // would have no coarse-grid arrays for the V-cycle to restrict into);
-    // a lower coarsest level fits the LDS as well
+    // in one workgroup (a grid that fits it whole, 65^2,
+    // would have no coarse-grid arrays for the V-cycle to restrict into)
     R.lc = std::min(h->M.lc, R.ng - 2);
     for (int l = R.lc; l < R.ng; l++) {
         size_t s = (size_t)((1 << (l + 1)) + 1) * ((1 << (l + 1)) + 1);
         CHECK(dalloc(h, &R.d.rhsF[l], s));
         CHECK(dalloc(h, &R.d.u[l], s));
-        if (l < R.ng - 1) {
-            CHECK(dalloc(h, &R.d.cres[l], s));
-            CHECK(dalloc(h, &R.d.cv[l], s));
-        }
+        CHECK(dalloc(h, &R.d.cv[l], s));
+        if (l < R.ng - 1) CHECK(dalloc(h, &R.d.cres[l], s));
     }
     const size_t N = (size_t)h->N, E = (N + 1) * (N + 1);
     CHECK(dalloc(h, &h->ref_ex, E));

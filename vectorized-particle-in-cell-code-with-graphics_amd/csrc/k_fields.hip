@@ -1,11 +1,7 @@
-// k_fields.hip -- charge -> rhs, multigrid Poisson solve, E = -grad(phi).
-//
-// Multigrid (mglin.cpp:21-196): full multigrid with ncycle V(1,1) cycles per
-// level, red-black Gauss-Seidel, half-weighting restriction, bilinear
-// prolongation.  Every per-node expression keeps the reference's FP64
-// association, so FIXED mode reproduces Mglin bit for bit.  Levels up to
-// 65x65 (or what the LDS holds) run inside one workgroup with all arrays in
-// LDS; finer levels use one launch per operation.
+// k_fields.hip -- charge -> rhs, E = -grad(phi), and the tolerance mode's
+// V-cycles (FP32 smoothing, FP64 residual and accumulation), taken where the
+// caller gives the sweeps or the grid is beyond the direct solve's transforms
+// (k_direct.hip); the reference's FP64 multigrid is in k_fmg.hip.
 #include <chrono>
 #include <cmath>
 #include <thread>
@@ -254,44 +250,6 @@ void launch_efield(hipStream_t st, const double *phi, int N, double dx, double *
 // ------------------------------------------------------ multigrid: nodes
 // Arrays are row-major, u[i*n + j] == NR's u[i][j].
 
-template <typename T>
-__device__ __forceinline__ T relax_node(const T *u, const T *rhs, int n, int i, int j, T h2) {
-    return (T)0.25 * (u[(i + 1) * n + j] + u[(i - 1) * n + j] + u[i * n + j + 1] +
-                      u[i * n + j - 1] - h2 * rhs[i * n + j]);
-}
-
-template <typename T>
-__device__ __forceinline__ T resid_node(const T *u, const T *rhs, int n, int i, int j, T h2i) {
-    return -h2i * (u[(i + 1) * n + j] + u[(i - 1) * n + j] + u[i * n + j + 1] +
-                   u[i * n + j - 1] - (T)4.0 * u[i * n + j]) +
-           rhs[i * n + j];
-}
-
-// half weighting of the residual at coarse (ic,jc), residual evaluated on
-// the fly (mglin.cpp:151-169 applied to mglin.cpp:133-144's output)
-template <typename T>
-__device__ __forceinline__ T resid_rstrct_node(const T *u, const T *rhs, int nf, int ic, int jc,
-                                               T h2i) {
-    int nc = (nf + 1) / 2;
-    if (ic == 0 || jc == 0 || ic == nc - 1 || jc == nc - 1) return (T)0.0;
-    int i = 2 * ic, j = 2 * jc;
-    return (T)0.5 * resid_node(u, rhs, nf, i, j, h2i) +
-           (T)0.125 * (resid_node(u, rhs, nf, i + 1, j, h2i) + resid_node(u, rhs, nf, i - 1, j, h2i) +
-                       resid_node(u, rhs, nf, i, j + 1, h2i) + resid_node(u, rhs, nf, i, j - 1, h2i));
-}
-
-template <typename T>
-__device__ __forceinline__ T rstrct_node(const T *uf, int nc, int ic, int jc) {
-    int nf = 2 * nc - 1, ncc = 2 * nc - 2;
-    if (jc == 0) return uf[(2 * ic) * nf + 0];
-    if (jc == nc - 1 && ic != 0 && ic != nc - 1) return uf[(2 * ic) * nf + ncc];
-    if (ic == 0) return uf[0 * nf + 2 * jc];
-    if (ic == nc - 1) return uf[ncc * nf + 2 * jc];
-    int i = 2 * ic, j = 2 * jc;
-    return (T)0.5 * uf[i * nf + j] + (T)0.125 * (uf[(i + 1) * nf + j] + uf[(i - 1) * nf + j] +
-                                                 uf[i * nf + j + 1] + uf[i * nf + j - 1]);
-}
-
 // bilinear prolongation value at fine (i,j) (mglin.cpp:70-82)
 template <typename T>
 __device__ __forceinline__ T interp_even_col(const T *uc, int nc, int i, int j) {
@@ -304,59 +262,8 @@ __device__ __forceinline__ T interp_node(const T *uc, int nc, int i, int j) {
     return (T)0.5 * (interp_even_col(uc, nc, i, j + 1) + interp_even_col(uc, nc, i, j - 1));
 }
 
-// ------------------------------------------- multigrid: grid-wide kernels
-// `skip` (may be null) is the tolerance solver's converged flag: once set,
-// the remaining queued iterations return immediately.
-#define SKIP_IF_DONE(skip) \
-    if ((skip) && *(skip)) return
-
 template <typename T>
-__global__ void k_mg_relax(T *__restrict__ u, const T *__restrict__ rhs, int n, T h2, int color,
-                           const int *__restrict__ skip) {
-    SKIP_IF_DONE(skip);
-    int i = blockIdx.y + 1;  // interior row
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    int j = 1 + ((i + 1 + color) & 1) + 2 * t;  // (i+j)%2 == color
-    if (i > n - 2 || j > n - 2) return;
-    u[i * n + j] = relax_node(u, rhs, n, i, j, h2);
-}
-
-template <typename T>
-__global__ void k_mg_resid_rstrct(const T *__restrict__ u, const T *__restrict__ rhs, int nf, T h2i,
-                                  T *__restrict__ uc, const int *__restrict__ skip) {
-    SKIP_IF_DONE(skip);
-    int nc = (nf + 1) / 2;
-    int jc = blockIdx.x * blockDim.x + threadIdx.x, ic = blockIdx.y;
-    if (jc >= nc) return;
-    uc[ic * nc + jc] = resid_rstrct_node(u, rhs, nf, ic, jc, h2i);
-}
-
-template <typename T>
-__global__ void k_mg_rstrct(T *__restrict__ uc, int nc, const T *__restrict__ uf) {
-    int jc = blockIdx.x * blockDim.x + threadIdx.x, ic = blockIdx.y;
-    if (jc >= nc) return;
-    uc[ic * nc + jc] = rstrct_node(uf, nc, ic, jc);
-}
-
-template <typename T>
-__global__ void k_mg_interp(T *__restrict__ uf, int nf, const T *__restrict__ uc) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
-    if (j >= nf) return;
-    uf[i * nf + j] = interp_node(uc, (nf + 1) / 2, i, j);
-}
-
-template <typename T>
-__global__ void k_mg_addint(T *__restrict__ uf, int nf, const T *__restrict__ uc,
-                            const int *__restrict__ skip) {
-    SKIP_IF_DONE(skip);
-    int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
-    if (j >= nf) return;
-    uf[i * nf + j] = uf[i * nf + j] + interp_node(uc, (nf + 1) / 2, i, j);
-}
-
-template <typename T>
-__global__ void k_fill(T *__restrict__ p, long n, T v, const int *__restrict__ skip) {
-    SKIP_IF_DONE(skip);
+__global__ void k_fill(T *__restrict__ p, long n, T v) {
     long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) p[k] = v;
 }
@@ -364,8 +271,7 @@ __global__ void k_fill(T *__restrict__ p, long n, T v, const int *__restrict__ s
 template <typename T>
 void launch_fill(hipStream_t st, T *p, long n, T v) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_fill<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n, v,
-                       (const int *)nullptr);
+    hipLaunchKernelGGL(k_fill<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n, v);
 }
 template void launch_fill<double>(hipStream_t, double *, long, double);
 template void launch_fill<float>(hipStream_t, float *, long, float);
@@ -373,155 +279,12 @@ template void launch_fill<unsigned long long>(hipStream_t, unsigned long long *,
                                               unsigned long long);
 template void launch_fill<uint32_t>(hipStream_t, uint32_t *, long, uint32_t);
 
-// --------------------------------------- multigrid: one-workgroup coarse part
-
 static __host__ __device__ inline int lvl_size(int l) { return (1 << (l + 1)) + 1; }
 
-// LDS layout of the coarse part topped at level lc (levels 0..lc):
-//   rhs[0..lc] | cres[0], cv[0], cres[1], cv[1], ... cres[lc-1], cv[lc-1] | u
-// Offsets are computed arithmetically (wave-uniform) so no pointer table is
-// kept per lane.
-static __host__ __device__ inline long sq_below(int l) {
-    long s = 0;
-    for (int k = 0; k < l; k++) s += (long)lvl_size(k) * lvl_size(k);
-    return s;
-}
-
-// doubles (or floats) of LDS needed for a coarse part topped at level lc
-static __host__ __device__ inline long coarse_lds_elems(int lc) {
-    return sq_below(lc + 1) + 2 * sq_below(lc) + (long)lvl_size(lc) * lvl_size(lc);
-}
-
-template <typename T>
-struct CoarseLds {
-    T *base;
-    int lc;
-    __device__ __forceinline__ T *rhs(int l) const { return base + sq_below(l); }
-    __device__ __forceinline__ T *cres(int l) const {
-        return base + sq_below(lc + 1) + 2 * sq_below(l);
-    }
-    __device__ __forceinline__ T *cv(int l) const { return cres(l) + (long)lvl_size(l) * lvl_size(l); }
-    __device__ __forceinline__ T *u() const { return base + sq_below(lc + 1) + 2 * sq_below(lc); }
-};
-
-__device__ __forceinline__ double lvl_h2(int l, double length) {
-    double h = length / (lvl_size(l) - 1);
-    return h * h;
-}
-
-template <typename T>
-__device__ void co_relax(T *u, const T *rhs, int n, T h2) {
-    int m = n - 2;  // interior per row
-    int half = (m + 1) / 2;
-    for (int color = 0; color < 2; color++) {
-        for (int k = threadIdx.x; k < m * half; k += blockDim.x) {
-            int i = 1 + k / half, t = k % half;
-            int j = 1 + ((i + 1 + color) & 1) + 2 * t;
-            if (j <= n - 2) u[i * n + j] = relax_node(u, rhs, n, i, j, h2);
-        }
-        __syncthreads();
-    }
-}
-
-// residual restricted to the coarse grid (mglin.cpp:189-190) and the coarse
-// correction zeroed (mglin.cpp:185), one pass
-template <typename T>
-__device__ void co_resid_rstrct_zero(const T *u, const T *rhs, int nf, T h2i, T *cres, T *cv) {
-    int nc = (nf + 1) / 2;
-    for (int k = threadIdx.x; k < nc * nc; k += blockDim.x) {
-        cres[k] = resid_rstrct_node(u, rhs, nf, k / nc, k % nc, h2i);
-        cv[k] = (T)0.0;
-    }
-    __syncthreads();
-}
-
-template <typename T>
-__device__ void co_rstrct(T *uc, int nc, const T *uf) {
-    for (int k = threadIdx.x; k < nc * nc; k += blockDim.x) uc[k] = rstrct_node(uf, nc, k / nc, k % nc);
-    __syncthreads();
-}
-
-template <typename T>
-__device__ void co_interp(T *uf, int nf, const T *uc, bool add) {
-    int nc = (nf + 1) / 2;
-    for (int k = threadIdx.x; k < nf * nf; k += blockDim.x) {
-        T v = interp_node(uc, nc, k / nf, k % nf);
-        uf[k] = add ? uf[k] + v : v;
-    }
-    __syncthreads();
-}
-
-template <typename T>
-__device__ void co_zero(T *p, int n) {
-    for (int k = threadIdx.x; k < n; k += blockDim.x) p[k] = (T)0.0;
-    __syncthreads();
-}
-
-template <typename T>
-__device__ void co_slvsml(T *u, const T *rhs, double length) {
-    // mglin.cpp:103-110
-    if (threadIdx.x < 9) {
-        T h = (T)(0.5 * length);
-        u[threadIdx.x] = (threadIdx.x == 4) ? -h * h * rhs[4] / (T)4.0 : (T)0.0;
-    }
-    __syncthreads();
-}
-
-// V(1,1) cycle at level j on (U, R), recursion unrolled (mglin.cpp:176-196)
-template <typename T>
-__device__ void co_vcycle(const CoarseLds<T> &L, int j, T *U, const T *R, double length) {
-    T *Ul = U;
-    const T *Rl = R;
-    for (int l = j; l >= 1; l--) {
-        int n = lvl_size(l);
-        double h2 = lvl_h2(l, length);
-        co_relax(Ul, Rl, n, (T)h2);
-        co_resid_rstrct_zero(Ul, Rl, n, (T)(1.0 / h2), L.cres(l - 1), L.cv(l - 1));
-        Ul = L.cv(l - 1);
-        Rl = L.cres(l - 1);
-    }
-    co_slvsml(L.cv(0), L.cres(0), length);
-    for (int l = 1; l <= j; l++) {
-        T *Uu = (l == j) ? U : L.cv(l);
-        const T *Ru = (l == j) ? R : L.cres(l);
-        co_interp(Uu, lvl_size(l), L.cv(l - 1), true);
-        co_relax(Uu, Ru, lvl_size(l), (T)lvl_h2(l, length));
-    }
-}
-
-// mode 0: full multigrid from rhs_in (level lc) -> u_out;  mode 1: ncycle
-// V-cycles on a zero initial guess (the coarse-grid correction of a finer
-// V-cycle) -> u_out.
-template <typename T>
-__global__ void __launch_bounds__(1024)
-    k_mg_coarse(const T *__restrict__ rhs_in, T *__restrict__ u_out, int lc, int mode, int ncycle,
-                double length, const int *__restrict__ skip) {
-    SKIP_IF_DONE(skip);
-    extern __shared__ double lds_raw[];
-    CoarseLds<T> L{reinterpret_cast<T *>(lds_raw), lc};
-    int nc = lvl_size(lc);
-    T *top = L.rhs(lc);
-    for (int k = threadIdx.x; k < nc * nc; k += blockDim.x) top[k] = rhs_in[k];
-    __syncthreads();
-    if (mode == 0) {
-        for (int l = lc - 1; l >= 0; l--) co_rstrct(L.rhs(l), lvl_size(l), L.rhs(l + 1));
-        // the full-multigrid iterate of level j < lc lives in cv(j) (free at
-        // that point: a V-cycle at level j only touches cv(0..j-1))
-        T *prev = (lc == 0) ? L.u() : L.cv(0);
-        co_slvsml(prev, L.rhs(0), length);
-        for (int j = 1; j <= lc; j++) {
-            T *Uj = (j == lc) ? L.u() : L.cv(j);
-            co_interp(Uj, lvl_size(j), prev, false);
-            for (int c = 0; c < ncycle; c++) co_vcycle(L, j, Uj, L.rhs(j), length);
-            prev = Uj;
-        }
-    } else {
-        co_zero(L.u(), nc * nc);
-        for (int c = 0; c < ncycle; c++) co_vcycle(L, lc, L.u(), L.rhs(lc), length);
-    }
-    T *u = L.u();
-    for (int k = threadIdx.x; k < nc * nc; k += blockDim.x) u_out[k] = u[k];
-}
+// `skip` (may be null) is the tolerance solver's converged flag: once set,
+// the remaining queued iterations return immediately.
+#define SKIP_IF_DONE(skip) \
+    if ((skip) && *(skip)) return
 
 // ------------------------------------- exact coarsest-level solve (TOL)
 // The 5-point Laplacian with zero walls is diagonalised by the discrete sine
@@ -997,90 +760,6 @@ int mg_dst_tables(MgLevels &M) {
     return 0;
 }
 
-// ------------------------------------------------------------ MG driver
-
-template <typename T>
-static void relax_launch(hipStream_t st, T *u, const T *rhs, int n, double length,
-                         const int *skip) {
-    double h = length / (n - 1);
-    T h2 = (T)(h * h);
-    int m = n - 2, half = (m + 1) / 2;
-    dim3 g((half + 127) / 128, m);
-    for (int c = 0; c < 2; c++)
-        hipLaunchKernelGGL(k_mg_relax<T>, g, dim3(128), 0, st, u, rhs, n, h2, c, skip);
-}
-
-template <typename T>
-static void coarse_launch(hipStream_t st, int lc, const T *rhs, T *u, int mode, int ncycle,
-                          double length, const int *skip) {
-    hipLaunchKernelGGL(k_mg_coarse<T>, dim3(1), dim3(1024), coarse_lds_elems(lc) * sizeof(T), st,
-                       rhs, u, lc, mode, ncycle, length, skip);
-}
-
-// V(1,1) cycle at level j > lc on (Uj, Rj) (mglin.cpp:176-196)
-// dst (fp32 only): solve the coarsest level exactly instead of by a V-cycle
-template <typename T>
-static void vcycle_launch(hipStream_t st, MgArrays<T> &A, int lc, int j, T *Uj, const T *Rj,
-                          double length, const int *skip, const MgLevels *dst = nullptr) {
-    int nf = lvl_size(j), nc = lvl_size(j - 1);
-    relax_launch<T>(st, Uj, Rj, nf, length, skip);
-    double h = length / (nf - 1);
-    hipLaunchKernelGGL(k_mg_resid_rstrct<T>, dim3((nc + 127) / 128, nc), dim3(128), 0, st, Uj, Rj,
-                       nf, (T)(1.0 / (h * h)), A.cres[j - 1], skip);
-    if (j - 1 == lc) {
-        if constexpr (std::is_same<T, float>::value) {
-            if (dst) coarse_dst_launch(st, *dst, A.cres[j - 1], A.cv[j - 1], length, skip);
-            else coarse_launch<T>(st, lc, A.cres[j - 1], A.cv[j - 1], 1, 1, length, skip);
-        } else {
-            coarse_launch<T>(st, lc, A.cres[j - 1], A.cv[j - 1], 1, 1, length, skip);
-        }
-    } else {
-        long s = (long)nc * nc;
-        hipLaunchKernelGGL(k_fill<T>, dim3((unsigned)((s + 255) / 256)), dim3(256), 0, st,
-                           A.cv[j - 1], s, (T)0, skip);
-        vcycle_launch<T>(st, A, lc, j - 1, A.cv[j - 1], A.cres[j - 1], length, skip, dst);
-    }
-    hipLaunchKernelGGL(k_mg_addint<T>, dim3((nf + 127) / 128, nf), dim3(128), 0, st, Uj, nf,
-                       A.cv[j - 1], skip);
-    relax_launch<T>(st, Uj, Rj, nf, length, skip);
-}
-
-int mg_coarse_level_for(long lds_bytes, int ng) {
-    int lc = 0;
-    for (int l = 1; l <= 5 && l < ng; l++)
-        if (coarse_lds_elems(l) * (long)sizeof(double) <= lds_bytes) lc = l;
-    return lc;
-}
-
-void mg_set_coarse_attr(long lds_bytes) {
-    hipFuncSetAttribute((const void *)k_mg_coarse<double>,
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-    hipFuncSetAttribute((const void *)k_mg_coarse_dst, hipFuncAttributeMaxDynamicSharedMemorySize,
-                        (int)lds_bytes);
-    hipFuncSetAttribute((const void *)k_mg_coarse<float>,
-                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
-}
-
-// FP64 full multigrid (mglin.cpp:21-55) on the device.  rhs = M.d.rhsF[ng-1]
-// (finest) on entry; the solution is written to M.d.u[ng-1].
-void mg_fixed_solve(hipStream_t st, MgLevels &M, int ncycle, double length) {
-    MgArrays<double> &A = M.d;
-    int lf = M.ng - 1, lc = M.lc;
-    for (int l = lf - 1; l >= lc; l--) {
-        int nc = lvl_size(l);
-        hipLaunchKernelGGL(k_mg_rstrct<double>, dim3((nc + 127) / 128, nc), dim3(128), 0, st,
-                           A.rhsF[l], nc, A.rhsF[l + 1]);
-    }
-    coarse_launch<double>(st, lc, A.rhsF[lc], A.u[lc], 0, ncycle, length, nullptr);
-    for (int j = lc + 1; j <= lf; j++) {
-        int nf = lvl_size(j);
-        hipLaunchKernelGGL(k_mg_interp<double>, dim3((nf + 127) / 128, nf), dim3(128), 0, st,
-                           A.u[j], nf, A.u[j - 1]);
-        for (int c = 0; c < ncycle; c++)
-            vcycle_launch<double>(st, A, lc, j, A.u[j], A.rhsF[j], length, nullptr);
-    }
-}
-
 // ---------------------------------------------- tolerance (mixed precision)
 // Iterative refinement: r = f - A u in FP64 (the reference's stencil and
 // association), the correction equation A e = r solved approximately by one
@@ -1531,7 +1210,7 @@ int mg_fp64_reference(hipStream_t st, MgLevels &R, double length, double tol, in
                       double *partials, double *host, int nb, double *relres) {
     const int lf = R.ng - 1, n = lvl_size(lf);
     // the V-cycle at lf restricts into cres[lf-1]: levels lc..lf-1 must exist
-    if (R.lc >= lf || !R.d.cres[lf - 1] || !R.d.cv[lf - 1]) return -1;
+    if (R.lc >= lf || !R.d.cres[lf - 1] || !R.d.cv[lf]) return -1;
     const double h = length / (n - 1), h2i = 1.0 / (h * h);
     double *u = R.d.u[lf];
     const double *f = R.d.rhsF[lf];
@@ -1544,7 +1223,7 @@ int mg_fp64_reference(hipStream_t st, MgLevels &R, double length, double tol, in
         if (host_block_sums(st, partials, host, nb, 2, sums) != 0) return -1;
         *relres = sums[1] > 0.0 ? sqrt(sums[0] / sums[1]) : sqrt(sums[0]);
         if (*relres <= tol || c >= max_cycles) break;
-        vcycle_launch<double>(st, R.d, R.lc, lf, u, f, length, nullptr);
+        mg_fixed_vcycle(st, R, length);
         c++;
     }
     return c;

@@ -19,17 +19,18 @@ constexpr int NOALLOC_MAX_N = 1025;
 constexpr int lvl_n(int l) { return (1 << (l + 1)) + 1; }
 // arrays start on 256-byte boundaries (32 doubles)
 constexpr size_t pad32(size_t n) { return (n + 31) & ~(size_t)31; }
-// the finest level's right-hand side plus, for every coarser level down to
-// 3 x 3, its right-hand side, full-multigrid iterate and V-cycle arrays
+// the finest level's right-hand side and iterate between the legs of a cycle
+// plus, for every coarser level down to 3 x 3, its right-hand side,
+// full-multigrid iterate and V-cycle arrays
 constexpr size_t scratch_doubles(int maxn) {
     int lf = 0;
     while (lvl_n(lf) < maxn) lf++;
-    size_t t = pad32((size_t)lvl_n(lf) * lvl_n(lf));
+    size_t t = 2 * pad32((size_t)lvl_n(lf) * lvl_n(lf));
     for (int l = 0; l < lf; l++) t += 4 * pad32((size_t)lvl_n(l) * lvl_n(l));
     return t;
 }
-constexpr size_t SCRATCH_DOUBLES = scratch_doubles(NOALLOC_MAX_N);  // 2 457 888 (19.7 MB)
-static_assert(SCRATCH_DOUBLES * sizeof(double) < (20u << 20), "scratch stays modest");
+constexpr size_t SCRATCH_DOUBLES = scratch_doubles(NOALLOC_MAX_N);  // 3 508 544 (28.1 MB)
+static_assert(SCRATCH_DOUBLES * sizeof(double) < (27u << 20), "scratch stays modest");
 
 }  // namespace
 
@@ -41,20 +42,10 @@ namespace {
 constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
 double *g_scratch[MAX_DEVICES] = {};  // device address of `scratch`, per device
-long g_lds[MAX_DEVICES] = {};
-
-long device_lds_limit(int dev) {
-    int v = 0;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-        v <= 0)
-        v = 65536;
-    return v;
-}
 
 // set-up once per device, with that device current: the address of this
 // device's copy of `scratch` (the host-side name is not a device address)
-// and the coarsest level's LDS attribute
-int scratch_for_current_device(double **out, long *lds) {
+int scratch_for_current_device(double **out) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES)
         return pic_host::set_global_error(PIC_ERR_DEVICE, "no current HIP device");
@@ -65,12 +56,9 @@ int scratch_for_current_device(double **out, long *lds) {
         if (e != hipSuccess || !p)
             return pic_host::set_global_error(
                 PIC_ERR_DEVICE, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-        g_lds[dev] = device_lds_limit(dev);
-        pic::mg_set_coarse_attr(g_lds[dev]);
         g_scratch[dev] = static_cast<double *>(p);
     }
     *out = g_scratch[dev];
-    *lds = g_lds[dev];
     return PIC_OK;
 }
 
@@ -88,14 +76,13 @@ extern "C" int pic_mglin_noalloc(double *u, int32_t n, int32_t ncycle, double le
             PIC_ERR_CAPACITY, "pic_mglin_noalloc: n = " + std::to_string(n) +
                                   " exceeds the scratch array's largest grid, n <= 1025");
     double *base = nullptr;
-    long lds = 0;
-    int rc = scratch_for_current_device(&base, &lds);
+    int rc = scratch_for_current_device(&base);
     if (rc != PIC_OK) return rc;
     pic::MgLevels R;
     int ng = 0;
     for (int nn = n; nn >>= 1;) ng++;
     R.ng = ng;
-    R.lc = pic::mg_coarse_level_for(lds, ng);
+    R.lc = pic::mg_coarse_level_for(ng);
     const int lf = ng - 1;
     size_t off = 0;
     auto take = [&](int l) {
@@ -105,6 +92,7 @@ extern "C" int pic_mglin_noalloc(double *u, int32_t n, int32_t ncycle, double le
     };
     R.d.rhsF[lf] = take(lf);
     R.d.u[lf] = u;  // the solution goes straight to the caller's buffer
+    R.d.cv[lf] = take(lf);
     for (int l = R.lc; l < lf; l++) {
         R.d.rhsF[l] = take(l);
         R.d.u[l] = take(l);

@@ -84,7 +84,7 @@ struct MgArrays {
     T *rhsF[16] = {};  // full-multigrid right-hand side per level
     T *u[16] = {};     // full-multigrid solution per level (u[ng-1]: result)
     T *cres[16] = {};  // V-cycle coarse right-hand side
-    T *cv[16] = {};    // V-cycle coarse correction
+    T *cv[16] = {};    // V-cycle coarse correction (FP64 finest: the iterate between two legs)
     T *us[16] = {};    // pre-smoothed iterate of the fused V-cycle (fp32 levels > lc)
 };
 
@@ -107,7 +107,6 @@ struct DirectPlan {
 struct MgLevels {
     DirectPlan dir;      // tolerance mode without given sweeps (dir.n > 0)
     int ng = 0, lc = 0;
-    long lds = 0;        // LDS bytes a workgroup may allocate on this device
     MgArrays<double> d;  // FP64 full multigrid (fixed mode) and the FP64 iterate
     MgArrays<float> f;   // FP32 correction solves (tolerance mode)
     // tolerance mode state (device): flags[0] done, flags[1] V-cycles applied,
@@ -366,10 +365,7 @@ void launch_efield(hipStream_t st, const double *phi, int N, double dx, double *
                    float2 *E32);
 template <typename T>
 void launch_fill(hipStream_t st, T *p, long n, T v);
-int mg_coarse_level_for(long lds_bytes, int ng);
 int mg_dst_tables(MgLevels &M);
-void mg_set_coarse_attr(long lds_bytes);
-void mg_fixed_solve(hipStream_t st, MgLevels &M, int ncycle, double length);
 // FP64 reference solve of R.d.rhsF[top] into R.d.u[top]: full multigrid, then
 // FP64 V(1,1) cycles to ||f - Au|| <= tol ||f|| (at most max_cycles);
 // partials: device, >= 2 nb doubles; host: >= 6 nb doubles.  Returns the
@@ -392,6 +388,13 @@ int field_diff_sums(hipStream_t st, const double *a0, const double *b0, const do
 int mg_tol_solve(hipStream_t st, MgLevels &M, double length, double tol, int max_iter,
                  double *relres_out, bool flags_reset = false,
                  const std::function<void(const double *, const double *)> &after_batch = nullptr);
+
+// ---- k_fmg.hip: the reference's FP64 full multigrid.  Needs rhsF, u, cv of
+// levels lc .. ng-1 and cres of lc .. ng-2 in M.d.
+int mg_coarse_level_for(int ng);  // the level solved in one workgroup, and below
+void mg_fixed_solve(hipStream_t st, MgLevels &M, int ncycle, double length);
+// one more V(1,1) cycle on M.d.u[ng-1] (ng - 1 > lc)
+void mg_fixed_vcycle(hipStream_t st, MgLevels &M, double length);
 
 // ---- k_direct.hip
 constexpr int DIRECT_DEVICE = -1000;
