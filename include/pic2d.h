@@ -308,7 +308,7 @@ int pic_mglin(double *u, int32_t n, int32_t ncycle, double length);
  * DEVICE pointer to n*n doubles (the rhs on entry, the solution on exit, as
  * pic_mglin); the work is queued on `stream` (a hipStream_t of the current
  * device; NULL = its default stream) and not waited for.  The multigrid
- * levels live in a library-owned static device array of 19.7 MB per GPU
+ * levels live in a library-owned static device array of 28.1 MB per GPU
  * (grids up to n = 1025; larger n returns PIC_ERR_CAPACITY), so no call
  * allocates or frees.  Calls that overlap on one GPU share that array and
  * race: order them on one stream.  Results are pic_mglin's, bit for bit. */
