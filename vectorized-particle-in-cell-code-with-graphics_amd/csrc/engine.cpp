@@ -218,14 +218,17 @@ void prof_flush(pic_handle *h) {
 // ------------------------------------------------------------ species
 int species_alloc(pic_handle *h, Species &s, int64_t cap) {
     s.cap = cap;
+    // whole blocks of the particle passes: they load a block's words without
+    // testing each against the count
+    const size_t pad = ((size_t)cap + PASS_BLOCK - 1) / PASS_BLOCK * PASS_BLOCK;
     for (int b = 0; b < 2; b++) {
-        CHECK(dalloc(h, &s.buf[b].cell, cap));
-        CHECK(dalloc(h, &s.buf[b].ox, cap));
-        CHECK(dalloc(h, &s.buf[b].oy, cap));
-        CHECK(dalloc(h, &s.buf[b].vx, cap));
-        CHECK(dalloc(h, &s.buf[b].vy, cap));
-        CHECK(dalloc(h, &s.buf[b].vz, cap));
-        CHECK(dalloc(h, &s.buf[b].id, cap));
+        CHECK(dalloc(h, &s.buf[b].cell, pad));
+        CHECK(dalloc(h, &s.buf[b].ox, pad));
+        CHECK(dalloc(h, &s.buf[b].oy, pad));
+        CHECK(dalloc(h, &s.buf[b].vx, pad));
+        CHECK(dalloc(h, &s.buf[b].vy, pad));
+        CHECK(dalloc(h, &s.buf[b].vz, pad));
+        CHECK(dalloc(h, &s.buf[b].id, pad));
     }
     for (int b = 0; b < 2; b++) {
         CHECK(dalloc(h, &s.qbuf[b], (size_t)h->N * h->N));

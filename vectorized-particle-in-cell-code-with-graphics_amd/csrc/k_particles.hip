@@ -195,7 +195,7 @@ __device__ __forceinline__ bool collide_take(bool blk, int qs, PState &s, int &e
 // full); each distinct key then costs one global atomic per block, and the
 // block's particles of one key take consecutive slots.  Every particle's rank
 // within its key comes from the LDS counter of its entry.
-#define IPP 4
+#define IPP (PASS_BLOCK / 256)
 #define HASH_BITS 11
 #define HASH_SIZE (1 << HASH_BITS)  // >= 2 x 256 x IPP
 #define HASH_EMPTY 0xFFFFFFFFu
@@ -619,64 +619,67 @@ __device__ __forceinline__ void block_deposit_n(const bool (&dep)[P], const PSta
                                                 unsigned long long *sq) {
     constexpr int DEP_HALF = dep_half(WCAP);
     static_assert((2 * DEP_HALF + 2) * (2 * DEP_HALF + 2) <= WCAP, "fallback window size");
-    __shared__ int red[4][6];
+    __shared__ int red[4][4];
     const int big = 1 << 30;
-    int mnx = big, mny = big, mxx = -big, mxy = -big, sx = 0, sy = 0, cnt = 0;
+    int mnx = big, mny = big, mxx = -big, mxy = -big;
 #pragma unroll
-    for (int r = 0; r < P; r++)
-        if (dep[r]) {
-            mnx = min(mnx, s[r].jx);
-            mny = min(mny, s[r].jy);
-            mxx = max(mxx, s[r].jx);
-            mxy = max(mxy, s[r].jy);
-            sx += s[r].jx;
-            sy += s[r].jy;
-            cnt++;
-        }
+    for (int r = 0; r < P; r++) {
+        mnx = min(mnx, dep[r] ? s[r].jx : big);
+        mny = min(mny, dep[r] ? s[r].jy : big);
+        mxx = max(mxx, dep[r] ? s[r].jx : -big);
+        mxy = max(mxy, dep[r] ? s[r].jy : -big);
+    }
     mnx = wave_min(mnx);
     mny = wave_min(mny);
     mxx = wave_max(mxx);
     mxy = wave_max(mxy);
-    sx = wave_sum(sx);
-    sy = wave_sum(sy);
-    cnt = wave_sum(cnt);
-    const int w = threadIdx.x >> 6;
+    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     if ((threadIdx.x & 63) == 0) {
         red[w][0] = mnx;
         red[w][1] = mny;
         red[w][2] = mxx;
         red[w][3] = mxy;
-        red[w][4] = sx;
-        red[w][5] = sy;
     }
-    __shared__ int redc[4];
-    if ((threadIdx.x & 63) == 0) redc[w] = cnt;
     __syncthreads();
-    const int nw = blockDim.x >> 6;
-    mnx = red[0][0];
-    mny = red[0][1];
-    mxx = red[0][2];
-    mxy = red[0][3];
-    sx = red[0][4];
-    sy = red[0][5];
-    cnt = redc[0];
-    for (int k = 1; k < nw; k++) {
+    for (int k = 0; k < nw; k++) {
         mnx = min(mnx, red[k][0]);
         mny = min(mny, red[k][1]);
         mxx = max(mxx, red[k][2]);
         mxy = max(mxy, red[k][3]);
-        sx += red[k][4];
-        sy += red[k][5];
-        cnt += redc[k];
     }
-    __syncthreads();  // red[] is reused by the next call in the same kernel
-    if (cnt == 0) return;  // nothing to deposit (uniform: all threads)
+    if (mxx < mnx) {  // nothing to deposit (uniform: all threads)
+        __syncthreads();  // red[] is reused by the next call in the same kernel
+        return;
+    }
     // a depositing particle has jx in [0, N-2]: its nodes jx, jx+1 <= N-1
     int x0 = mnx, y0 = mny, ww = mxx - mnx + 2, wh = mxy - mny + 2;
-    if (ww * wh > WCAP) {
-        const int cx = sx / cnt, cy = sy / cnt;
-        x0 = cx - DEP_HALF;
-        y0 = cy - DEP_HALF;
+    if (ww * wh > WCAP) {  // uniform: the block's mean cell is needed only here
+        int sx = 0, sy = 0, cnt = 0;
+#pragma unroll
+        for (int r = 0; r < P; r++)
+            if (dep[r]) {
+                sx += s[r].jx;
+                sy += s[r].jy;
+                cnt++;
+            }
+        sx = wave_sum(sx);
+        sy = wave_sum(sy);
+        cnt = wave_sum(cnt);
+        __syncthreads();  // red[] has been read
+        if ((threadIdx.x & 63) == 0) {
+            red[w][0] = sx;
+            red[w][1] = sy;
+            red[w][2] = cnt;
+        }
+        __syncthreads();
+        sx = sy = cnt = 0;
+        for (int k = 0; k < nw; k++) {
+            sx += red[k][0];
+            sy += red[k][1];
+            cnt += red[k][2];
+        }
+        x0 = sx / cnt - DEP_HALF;
+        y0 = sy / cnt - DEP_HALF;
         ww = wh = 2 * DEP_HALF + 2;
     }
     const int area = ww * wh;
@@ -690,7 +693,7 @@ __device__ __forceinline__ void block_deposit_n(const bool (&dep)[P], const PSta
         if (dep[r]) {
             const FxW fw = fx_weights_w(s[r].ox, s[r].oy, pw[r]);
             const int dx = s[r].jx - x0, dy = s[r].jy - y0;
-            if (dx >= 0 && dx <= ww - 2 && dy >= 0 && dy <= wh - 2) {
+            if ((unsigned)dx <= (unsigned)(ww - 2) && (unsigned)dy <= (unsigned)(wh - 2)) {
                 const int b = cb + dy * ww + dx;
                 atomicAdd(&sq[b], fw.a4);
                 atomicAdd(&sq[b + 1], fw.a3);
@@ -701,11 +704,17 @@ __device__ __forceinline__ void block_deposit_n(const bool (&dep)[P], const PSta
             }
         }
     __syncthreads();
-    // window nodes outside the grid (fallback window at an edge) stay zero
+    // window nodes outside the grid (fallback window at an edge) stay zero.
+    // The row of node k is k / ww in fp32: (k + 1/2) / ww is at least 1 / 2ww
+    // off every integer and its rounding error below area 2^-23 / ww.
+    const float inv = 1.0f / (float)ww;
     for (int k = threadIdx.x; k < area; k += blockDim.x) {
         unsigned long long v = 0ull;
         for (int c = 0; c < copies; c++) v += sq[c * area + k];
-        if (v) atomicAdd(&q[(long)(y0 + k / ww) * N + x0 + k % ww], v);
+        if (v) {
+            const int row = (int)(((float)k + 0.5f) * inv);
+            atomicAdd(&q[(long)(y0 + row) * N + (x0 + k - row * ww)], v);
+        }
     }
 }
 
@@ -749,6 +758,36 @@ __device__ __forceinline__ void count_events(int ev, unsigned long long *__restr
         atomicAdd(&events[cnt_slot() * 8 + threadIdx.x], (unsigned long long)se[threadIdx.x]);
 }
 
+// Products of a physical-mode ionisation of particle pid at `pre` (its state
+// before the push), weight w
+__device__ __forceinline__ void stage_ionisation(const mcc::Child &ch, const PState &pre,
+                                                 uint32_t pid, const float2 *__restrict__ E,
+                                                 const PushConst &pc, const Spawn &sp,
+                                                 uint32_t *__restrict__ lost6, float w) {
+    // ejected electron: born at the parent's position, pushed this step
+    // as the reference pushes particles appended before move_particles
+    PState ce = pre;
+    ce.vx = ch.vx;
+    ce.vy = ch.vy;
+    ce.vz = ch.vz;
+    push_one(ce, E, pc);
+    const int cst = classify(ce, pc.N, pc.mode);
+    if (cst != ST_KEPT) {
+        // left the domain during its first push: it still takes its id
+        // (as it does when created before the push), but is not stored
+        atomicAdd(&lost6[cnt_slot() * 6 + cst - 1], 1u);
+        ce.jx = ce.jy = CELL_DEAD;
+    }
+    stage_put(sp.se, &sp.ce->stage_count, &sp.ce->overflow, ce, (unsigned long long)pid, w);
+    // new ion at the same place; the ion pass of this step moves it
+    PState ci = pre;
+    ci.vx = ch.ivx;
+    ci.vy = ch.ivy;
+    ci.vz = ch.ivz;
+    // products take the parent's weight (e_collisions.cpp:413,441)
+    stage_put(sp.si, &sp.ci->stage_count, &sp.ci->overflow, ci, (unsigned long long)pid, w);
+}
+
 // Products of one particle's step: the ejected electron and the new ion of a
 // physical-mode ionisation, and the electron-ion pair re-injected for an ion
 // lost through a wall (sp.plop).  `pre` is the state before the push.
@@ -758,30 +797,8 @@ __device__ __forceinline__ void stage_products(int ev, const mcc::Child &ch, con
                                                const mcc::MccConst &mc, uint32_t step,
                                                const Spawn &sp, uint32_t *__restrict__ lost6,
                                                float w, const PState &post) {
-    if (EV_KIND(ev) == mcc::EV_IONIZE && mc.mode == PIC_DEV_MODE_PHYS) {
-        // ejected electron: born at the parent's position, pushed this step
-        // as the reference pushes particles appended before move_particles
-        PState ce = pre;
-        ce.vx = ch.vx;
-        ce.vy = ch.vy;
-        ce.vz = ch.vz;
-        push_one(ce, E, pc);
-        int cst = classify(ce, pc.N, pc.mode);
-        if (cst != ST_KEPT) {
-            // left the domain during its first push: it still takes its id
-            // (as it does when created before the push), but is not stored
-            atomicAdd(&lost6[cnt_slot() * 6 + cst - 1], 1u);
-            ce.jx = ce.jy = CELL_DEAD;
-        }
-        stage_put(sp.se, &sp.ce->stage_count, &sp.ce->overflow, ce, (unsigned long long)pid, w);
-        // new ion at the same place; the ion pass of this step moves it
-        PState ci = pre;
-        ci.vx = ch.ivx;
-        ci.vy = ch.ivy;
-        ci.vz = ch.ivz;
-        // products take the parent's weight (e_collisions.cpp:413,441)
-        stage_put(sp.si, &sp.ci->stage_count, &sp.ci->overflow, ci, (unsigned long long)pid, w);
-    }
+    if (EV_KIND(ev) == mcc::EV_IONIZE && mc.mode == PIC_DEV_MODE_PHYS)
+        stage_ionisation(ch, pre, pid, E, pc, sp, lost6, w);
     if (sp.plop && valid && st >= ST_LEFT && st <= ST_TOP) {
         PState pe, pi;
         mcc::plop_pair(mc, pid, step, pc.N, sp.se_sigma, sp.si_sigma, sp.plop_ref, pe, pi);
@@ -1123,7 +1140,7 @@ __global__ void __launch_bounds__(256)
 #endif
 
 
-// one particle of k_push_inplace: collide (block-wide when blk), push, store
+// one particle of the generic k_push_inplace: collide (block-wide when blk), push, store
 // in place or leave a hole, count, stage products; dep = deposit it
 __device__ __forceinline__ void inplace_round(const SpView &sp, uint32_t i, uint32_t n, PState &s,
                                               uint32_t pid, bool live, bool &dep, bool &kept_out,
@@ -1132,21 +1149,13 @@ __device__ __forceinline__ void inplace_round(const SpView &sp, uint32_t i, uint
                                               const Spawn &spn, uint32_t *__restrict__ lost6,
                                               bool need_vz, bool blk, int qs, uint32_t *sl,
                                               uint32_t *shole, uint32_t *se,
-                                              const unsigned long long *lds, float w,
-                                              bool defer) {
+                                              const unsigned long long *lds, float w) {
     const PState pre = s;
     int ev = mcc::EV_NONE;
     mcc::Child ch{};
-    // deferred: a candidate stays as it is for k_collide_q
-    bool cand = false;
-    if (defer) {
-        // (a deferring species has no energy bins: its bound is global)
-        cand = live && mcc::candidate(mc, pid, step, 0.0f);
-        defer_queue(spn, cand, i);
-    }
-    const bool done = defer || collide_take(blk, qs, s, ev, ch, lds);
+    const bool done = collide_take(blk, qs, s, ev, ch, lds);
     int st = ST_HOLE;
-    if (live && !cand) st = advance_one(s, pid, E, pc, mc, step, 1, ev, ch, done);
+    if (live) st = advance_one(s, pid, E, pc, mc, step, 1, ev, ch, done);
     const bool kept = (st == ST_KEPT);
     kept_out = kept;
     dep = kept && deposit_ok(s, pc.N, pc.mode);
@@ -1162,7 +1171,7 @@ __device__ __forceinline__ void inplace_round(const SpView &sp, uint32_t i, uint
         sp.vx[i] = s.vx;
         sp.vy[i] = s.vy;
         if (need_vz && __float_as_uint(s.vz) != __float_as_uint(pre.vz)) sp.vz[i] = s.vz;
-    } else if (live && !cand) {
+    } else if (live) {
         sp.cell[i] = cell_pack(CELL_HOLE, CELL_HOLE);
         atomicAdd(&sl[st - 1], 1u);
         atomicAdd(shole, 1u);
@@ -1177,33 +1186,13 @@ __device__ __forceinline__ void inplace_round(const SpView &sp, uint32_t i, uint
     stage_products(ev, ch, pre, st, i < n, pid, E, pc, mc, step, spn, lost6, w, s);
 }
 
-// In-place timestep of one species between sort passes: the same collide +
-// push as the sort pass, the state written back to its own slot, the
-// deposit through one LDS window per block.  A particle that leaves (or that
-// a collision removes) becomes a hole; the next sort pass compacts the store.
-// Each thread handles IPP particles (strided by the block size, so every
-// load and store stays coalesced): one deposit window and one flush of the
-// block's counters then serve 256 * IPP particles.  Reads 20-28 B and writes
-// 20-24 B per particle, with no histogram or slot claims.
-// LDS of an in-place pass (u64 words): the collision queue, then the
-// deposit window, then the sort histogram.  The electrons' collisional
-// variant runs at 5 waves per SIMD (its registers): 28 KB fit five blocks
-// per CU and give its deposit a 58 x 58 fallback window for particles that
-// moved up to three steps since their store was sorted; the others, at 8
-// waves, keep 16 KB.
-template <int V>
-constexpr int inplace_lds_u64() {
-    return V == PV_COLL_E ? 3584 : BLOCK_LDS_U64;
-}
-
-template <int V>
-__device__ __forceinline__ void push_inplace_body(
+// The in-place pass with every option taken at run time (push_inplace_body's
+// comment says what an in-place pass is).
+__device__ __forceinline__ void push_inplace_generic(
     SpView sp, const uint32_t *__restrict__ nptr, const float2 *__restrict__ E, PushConst pc,
     mcc::MccConst mc, uint32_t step, unsigned long long *__restrict__ q, int deposit, Spawn spn,
     unsigned long long *__restrict__ events, uint32_t *__restrict__ lost6,
     uint32_t *__restrict__ holes, uint32_t *__restrict__ hist, uint32_t bid) {
-    pin_variant<V>(pc, mc, sp);
-    pin_spawn<V>(spn);
     const uint32_t n = *nptr;
     // the grid covers the capacity: blocks past the live count leave at once
     // (uniformly, before any barrier); bid: this block's index in the species
@@ -1211,7 +1200,7 @@ __device__ __forceinline__ void push_inplace_body(
     __shared__ uint32_t sl[6];
     __shared__ uint32_t shole;
     __shared__ uint32_t se[8];
-    constexpr int LDS_U64 = inplace_lds_u64<V>();
+    constexpr int LDS_U64 = BLOCK_LDS_U64;
     __shared__ unsigned long long lds[LDS_U64];
     if (threadIdx.x < 6) sl[threadIdx.x] = 0;
     if (threadIdx.x < 8) se[threadIdx.x] = 0;
@@ -1220,10 +1209,9 @@ __device__ __forceinline__ void push_inplace_body(
     // vz and the id are read only where something uses them: the magnetic
     // rotation, collisions, re-injection keyed by the id, and the wall
     // queue (surface physics needs the full velocity and the id's draws)
-    // (a deferred pass moves no candidate: the others keep their vz)
-    const bool need_vz = pc.bfield != 0 || (mc.on && V != PV_DEFER) || spn.wall;
+    const bool need_vz = pc.bfield != 0 || mc.on || spn.wall;
     const bool need_id = mc.on || spn.plop || spn.wall;
-    const bool blk = mc.on && mc.mode == PIC_DEV_MODE_PHYS && V != PV_DEFER;
+    const bool blk = mc.on && mc.mode == PIC_DEV_MODE_PHYS;
     PState s[IPP];
     uint32_t pid[IPP];
     bool live[IPP];
@@ -1252,20 +1240,16 @@ __device__ __forceinline__ void push_inplace_body(
     // the rounds are spelled out so every array index is a compile-time constant
     inplace_round(sp, base + 0 * blockDim.x, n, s[0], pid[0], live[0], dep[0], kept[0], E, pc,
                   mc, step,
-                  spn, lost6, need_vz, blk, qs[0], sl, &shole, se, lds, w[0],
-                  V == PV_DEFER);
+                  spn, lost6, need_vz, blk, qs[0], sl, &shole, se, lds, w[0]);
     inplace_round(sp, base + 1 * blockDim.x, n, s[1], pid[1], live[1], dep[1], kept[1], E, pc,
                   mc, step,
-                  spn, lost6, need_vz, blk, qs[1], sl, &shole, se, lds, w[1],
-                  V == PV_DEFER);
+                  spn, lost6, need_vz, blk, qs[1], sl, &shole, se, lds, w[1]);
     inplace_round(sp, base + 2 * blockDim.x, n, s[2], pid[2], live[2], dep[2], kept[2], E, pc,
                   mc, step,
-                  spn, lost6, need_vz, blk, qs[2], sl, &shole, se, lds, w[2],
-                  V == PV_DEFER);
+                  spn, lost6, need_vz, blk, qs[2], sl, &shole, se, lds, w[2]);
     inplace_round(sp, base + 3 * blockDim.x, n, s[3], pid[3], live[3], dep[3], kept[3], E, pc,
                   mc, step,
-                  spn, lost6, need_vz, blk, qs[3], sl, &shole, se, lds, w[3],
-                  V == PV_DEFER);
+                  spn, lost6, need_vz, blk, qs[3], sl, &shole, se, lds, w[3]);
     // block_deposit_n passes a barrier before it writes the window, so every
     // round has read its collision result from the shared LDS by then
     if (deposit) block_deposit_n<IPP, LDS_U64>(dep, s, w, q, pc.N, lds);
@@ -1286,6 +1270,315 @@ __device__ __forceinline__ void push_inplace_body(
     if (threadIdx.x == 0 && shole) atomicAdd(&holes[cnt_slot()], shole);
 }
 
+// ---- the passes with pinned options (physical mode, no magnetic field, no
+// per-particle weights)
+
+// A copy of the collision constants the compiler takes for new: expressions of
+// them are then evaluated where they are used.  (Hoisted out of the queue's
+// loop they are uniform floats in some 40 VGPRs, held across it.)
+__device__ __forceinline__ mcc::MccConst fresh(mcc::MccConst c) {
+    asm volatile("" : "+s"(c.mass), "+s"(c.M), "+s"(c.q), "+s"(c.ng), "+s"(c.opal_B), "+s"(c.vtn));
+    asm volatile("" : "+s"(c.e_exc), "+s"(c.e_iz), "+s"(c.kev_amu_div), "+s"(c.nu_max), "+s"(c.gas));
+    return c;
+}
+
+// mcc's block-level collisions on the pinned passes (COLL_E, COLL_I): the
+// candidates of the block's P x 256 particles are queued in LDS and collide
+// on dense lanes; vx and vy come back to the particles' lanes, everything
+// else -- the new vz, the event counts, the products of an ionisation -- is
+// settled by the lane that made the collision, so none of it takes code or
+// registers in the particles' rounds.  The queue holds every particle of the
+// block (5 words each): it cannot overflow.  q: free on entry and again after
+// the next barrier.  The store's words of the block are not yet overwritten.
+#define CQ_WORDS 5
+template <int P>
+__device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)[P],
+                                              float (&vy)[P], const float (&vz)[P],
+                                              const uint32_t (&id)[P], const SpView &sp,
+                                              uint32_t blk0, const float2 *__restrict__ E,
+                                              const PushConst &pc, const mcc::MccConst &mc0,
+                                              uint32_t step, const Spawn &spn,
+                                              uint32_t *__restrict__ lost6, uint32_t *se,
+                                              const float2 *tab, float *q) {
+    constexpr uint32_t CAP = P * 256;
+    __shared__ uint32_t wcnt[4];
+    uint32_t *qu = reinterpret_cast<uint32_t *>(q);  // v (3), id, slot
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    uint32_t pos[P], wtot = 0;
+#pragma unroll
+    for (int r = 0; r < P; r++) {
+        const bool cand =
+            live[r] && mcc::candidate(mc0, id[r], step,
+                                      vx[r] * vx[r] + vy[r] * vy[r] + vz[r] * vz[r], tab);
+        const uint64_t bal = __ballot(cand);
+        pos[r] = cand ? wtot + (uint32_t)__popcll(bal & below) : 0xFFFFFFFFu;
+        wtot += (uint32_t)__popcll(bal);
+    }
+    if (lane == 0) wcnt[w] = wtot;
+    __syncthreads();
+    uint32_t base = 0, total = 0;
+    for (int k = 0; k < 4; k++) {
+        if (k < w) base += wcnt[k];
+        total += wcnt[k];
+    }
+#pragma unroll
+    for (int r = 0; r < P; r++) {
+        if (pos[r] != 0xFFFFFFFFu) {
+            const uint32_t t = pos[r] += base;
+            q[t] = vx[r];
+            q[CAP + t] = vy[r];
+            q[2 * CAP + t] = vz[r];
+            qu[3 * CAP + t] = id[r];
+            qu[4 * CAP + t] = blk0 + threadIdx.x + r * 256;
+        }
+    }
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < total; t += 256) {
+        const mcc::MccConst mc = fresh(mc0);
+        float ux = q[t], uy = q[CAP + t], uz = q[2 * CAP + t];
+        const uint32_t pid = qu[3 * CAP + t], i = qu[4 * CAP + t];
+        mcc::Child ch{};
+        const int ev = mc.electron
+                           ? mcc::collide_electron<true>(mc, ux, uy, uz, pid, step, true, ch, tab)
+                           : mcc::collide_ion<true>(mc, ux, uy, uz, pid, step);
+        q[t] = ux;
+        q[CAP + t] = uy;
+        sp.vz[i] = uz;
+        if (EV_KIND(ev) > 0) atomicAdd(&se[EV_KIND(ev)], 1u);
+        if (ev & EV_OVER_BOUND) atomicAdd(&se[6], 1u);
+        if (EV_KIND(ev) == mcc::EV_IONIZE)
+            stage_ionisation(ch, load_state(sp, i, false), pid, E, pc, spn, lost6, 1.0f);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < P; r++)
+        if (pos[r] != 0xFFFFFFFFu) {
+            vx[r] = q[pos[r]];
+            vy[r] = q[CAP + pos[r]];
+        }
+}
+
+// gather_one's field of two particles, every load issued before the first is
+// used; a particle that cannot move (ok false) reads node 0
+__device__ __forceinline__ void gather_two(const PState (&s)[2], const bool (&ok)[2],
+                                           const float2 *__restrict__ E, int N, float (&ex)[2],
+                                           float (&ey)[2]) {
+    float2 e00[2], e01[2], e10[2], e11[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const uint32_t b = ok[r] ? (uint32_t)(s[r].jy * N + s[r].jx) : 0u;
+        const float2 *lo = E + b, *hi = E + (b + (uint32_t)N);
+        e00[r] = lo[0];
+        e01[r] = lo[1];
+        e10[r] = hi[0];
+        e11[r] = hi[1];
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const float wj = s[r].ox, wk = s[r].oy;
+        const float a4 = (1.0f - wj) * (1.0f - wk), a3 = wj * (1.0f - wk);
+        const float a2 = wk * (1.0f - wj), a1 = wj * wk;
+        ex[r] = a4 * e00[r].x + a3 * e01[r].x + a2 * e10[r].x + a1 * e11[r].x;
+        ey[r] = a4 * e00[r].y + a3 * e01[r].y + a2 * e10[r].y + a1 * e11[r].y;
+    }
+}
+
+// reposition without branches
+__device__ __forceinline__ void reposition_sel(int j, float t, int &jn, float &on) {
+    const float k0 = floorf(t), f0 = t - k0;
+    const bool up = f0 >= 1.0f;  // t just below an integer: t - k rounded up to 1
+    const int jj = min(max(j + (int)(up ? k0 + 1.0f : k0), -CELL_FAR), CELL_FAR);
+    const bool in = t > -POS_GUARD && t < POS_GUARD;  // false for NaN
+    jn = in ? jj : (t > 0.0f ? CELL_FAR : -CELL_FAR);
+    on = (in && !up) ? f0 : 0.0f;
+}
+
+// move_one without a magnetic field; ok false: unchanged
+__device__ __forceinline__ void move_sel(PState &s, bool ok, float ex, float ey,
+                                         const PushConst &pc) {
+    float ux = s.vx + pc.cE * ex, uy = s.vy + pc.cE * ey;
+    ux = ux + pc.cE * ex;
+    uy = uy + pc.cE * ey;
+    int jx, jy;
+    float ox, oy;
+    reposition_sel(s.jx, s.ox + ux * pc.dtdx, jx, ox);
+    reposition_sel(s.jy, s.oy + uy * pc.dtdy, jy, oy);
+    s.jx = ok ? jx : s.jx;
+    s.jy = ok ? jy : s.jy;
+    s.ox = ok ? ox : s.ox;
+    s.oy = ok ? oy : s.oy;
+    s.vx = ok ? ux : s.vx;
+    s.vy = ok ? uy : s.vy;
+}
+
+__device__ __forceinline__ bool inside_cells(const PState &s, int N) {
+    return (unsigned)s.jx <= (unsigned)(N - 2) && (unsigned)s.jy <= (unsigned)(N - 2);
+}
+
+// LDS of an in-place pass (u64 words): the collision queue, then the deposit
+// window, then the sort histogram (which needs 16 KB).  The electrons'
+// collisional variant takes a 58 x 58 fallback window (28 KB, five blocks per
+// CU) for particles that moved up to three steps since their store was
+// sorted.
+template <int V>
+constexpr int inplace_lds_u64() {
+    return V == PV_COLL_E ? 3584 : V == PV_COLL_I ? 2560 : BLOCK_LDS_U64;
+}
+
+// In-place timestep of one species between sort passes: the same collide +
+// push as the sort pass, the state written back to its own slot, the
+// deposit through one LDS window per block.  A particle that leaves (or that
+// a collision removes) becomes a hole; the next sort pass compacts the store.
+// Each thread handles IPP particles (strided by the block size, so every
+// load and store stays coalesced): one deposit window and one flush of the
+// block's counters then serve 256 * IPP particles.  Reads 20-28 B and writes
+// 20-24 B per particle, with no histogram or slot claims.
+//
+// Bound by HBM (257^2, 13.1 M particles: 129 us the ions, 149 us the
+// electrons, against 122 us for a copy of their 48 B) and by VALU issue about
+// equally.  The loads of all four particles are issued before the first is
+// decoded (the arrays are padded to whole blocks: no bounds test before a
+// load), the field loads of two at a time, and the rounds are straight-line
+// selects: only particles that leave take a branch, and the collisions'
+// products are settled on the queue's lanes.  Before, each particle waited
+// for its own cell and then its own field loads, and the collision code was
+// inlined once more in every round (queue overflow): 269 VALU instructions
+// per ion and 374 per electron instead of 196 and 261, 158 and 210 us.
+template <int V>
+__device__ __forceinline__ void push_inplace_body(
+    SpView sp, const uint32_t *__restrict__ nptr, const float2 *__restrict__ E, PushConst pc,
+    mcc::MccConst mc, uint32_t step, unsigned long long *__restrict__ q, int deposit, Spawn spn,
+    unsigned long long *__restrict__ events, uint32_t *__restrict__ lost6,
+    uint32_t *__restrict__ holes, uint32_t *__restrict__ hist, uint32_t bid) {
+    pin_variant<V>(pc, mc, sp);
+    pin_spawn<V>(spn);
+    constexpr bool COLL = V == PV_COLL_E || V == PV_COLL_I;
+    constexpr bool ID = COLL || V == PV_DEFER;
+    const uint32_t n = *nptr, blk0 = bid * (256 * IPP);
+    // the grid covers the capacity: blocks past the live count leave at once
+    // (uniformly, before any barrier); bid: this block's index in the species
+    if (blk0 >= n) return;
+    __shared__ uint32_t sl[6];
+    __shared__ uint32_t shole;
+    __shared__ uint32_t se[8];
+    constexpr int LDS_U64 = inplace_lds_u64<V>();
+    __shared__ unsigned long long lds[LDS_U64];
+    static_assert(!COLL || CQ_WORDS * IPP * 256 * 4 <= LDS_U64 * 8, "collision queue size");
+    const uint32_t tid = threadIdx.x;
+    if (tid < 6) sl[tid] = 0;
+    if (tid < 8) se[tid] = 0;
+    if (tid == 0) shole = 0;
+    uint32_t c0[IPP], pid[IPP];
+    float ox[IPP], oy[IPP], vx[IPP], vy[IPP], vz[IPP];
+    {
+        const uint32_t *pc_ = sp.cell + blk0, *pi = sp.id + blk0;
+        const float *px = sp.ox + blk0, *py = sp.oy + blk0, *pu = sp.vx + blk0,
+                    *pv = sp.vy + blk0, *pz = sp.vz + blk0;
+#pragma unroll
+        for (int r = 0; r < IPP; r++) {  // every load first
+            c0[r] = pc_[tid + r * 256];
+            if (ID) pid[r] = pi[tid + r * 256];
+            vx[r] = pu[tid + r * 256];
+            vy[r] = pv[tid + r * 256];
+            if (COLL) vz[r] = pz[tid + r * 256];
+            ox[r] = px[tid + r * 256];
+            oy[r] = py[tid + r * 256];
+        }
+    }
+    // the electrons' null-collision bounds in LDS (loaded beside the state)
+    __shared__ float2 sbins[MCC_BINS];
+    if (COLL && mc.bins && tid < MCC_BINS) sbins[tid] = mc.bins[tid];
+    bool live[IPP], cand[IPP];
+#pragma unroll
+    for (int r = 0; r < IPP; r++) {
+        live[r] = blk0 + tid + r * 256 < n && cell_jx(c0[r]) != CELL_HOLE;
+        cand[r] = false;
+    }
+    __syncthreads();  // counters initialised, bounds staged
+    if (COLL)
+        collide_queue<IPP>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step, spn, lost6, se,
+                           mc.bins ? sbins : nullptr, reinterpret_cast<float *>(lds));
+    if (V == PV_DEFER) {
+        // a candidate stays as it is for k_collide_q (a deferring species has
+        // no energy bins: its bound is global)
+#pragma unroll
+        for (int r = 0; r < IPP; r++) {
+            cand[r] = live[r] && mcc::candidate(mc, pid[r], step, 0.0f, nullptr);
+            defer_queue(spn, cand[r], blk0 + tid + r * 256);
+        }
+    }
+    PState s[IPP];
+    bool dep[IPP];
+    float w[IPP];
+    uint32_t *pc_ = sp.cell + blk0;
+    float *px = sp.ox + blk0, *py = sp.oy + blk0, *pu = sp.vx + blk0, *pv = sp.vy + blk0;
+#pragma unroll
+    for (int h = 0; h < IPP; h += 2) {  // the field loads of two particles at a time
+        PState t[2];
+        bool ok[2];
+        float ex[2], ey[2];
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const int r = h + g;
+            t[g] = PState{cell_jx(c0[r]), cell_jy(c0[r]), ox[r], oy[r], vx[r], vy[r], 0.0f};
+            ok[g] = live[r] && inside_cells(t[g], pc.N);
+        }
+        gather_two(t, ok, E, pc.N, ex, ey);
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const int r = h + g;
+            s[r] = t[g];
+            w[r] = 1.0f;
+            move_sel(s[r], ok[g], ex[g], ey[g], pc);
+            const bool move = live[r] && !cand[r];
+            dep[r] = move && inside_cells(s[r], pc.N);
+            if (dep[r]) {
+                // a word whose bits did not change (the cell of a particle
+                // that stayed in its cell) is not written again, and a
+                // wavefront with no changed lane issues no store
+                const uint32_t c1 = cell_pack(s[r].jx, s[r].jy);
+                if (c1 != c0[r]) pc_[tid + r * 256] = c1;
+                px[tid + r * 256] = s[r].ox;
+                py[tid + r * 256] = s[r].oy;
+                pu[tid + r * 256] = s[r].vx;
+                pv[tid + r * 256] = s[r].vy;
+            } else if (move) {
+                pc_[tid + r * 256] = cell_pack(CELL_HOLE, CELL_HOLE);
+                const int st = classify(s[r], pc.N, pc.mode);
+                atomicAdd(&sl[st - 1], 1u);
+                atomicAdd(&shole, 1u);
+                // the id and vz are read again only here
+                const uint32_t i = blk0 + tid + r * 256;
+                if (spn.lost_ids) queue_lost(spn, sp.id[i], 1.0f);
+                if (COLL && spn.wall) {  // waits for the surface pass
+                    PState post = s[r];
+                    post.vz = sp.vz[i];
+                    stage_put(spn.wq, &spn.cw->wall_count, &spn.cw->overflow, post,
+                              (unsigned long long)sp.id[i]);
+                }
+            }
+        }
+    }
+    // block_deposit_n passes a barrier before it writes the window, so every
+    // lane has read its collision result from the shared LDS by then
+    if (deposit) block_deposit_n<IPP, LDS_U64>(dep, s, w, q, pc.N, lds);
+    __syncthreads();
+    // ahead of a sort pass: the histogram of the cells the particles end the
+    // step in, the keys that pass claims by (no k_key_count then)
+    if (hist) {
+        uint32_t key[IPP];
+#pragma unroll
+        for (int r = 0; r < IPP; r++)
+            key[r] = dep[r] ? bin_key(s[r].jx, s[r].jy, pc.tilesX) >> pc.keyshift : 0u;
+        block_key_hist<IPP>(dep, key, hist, reinterpret_cast<uint32_t *>(lds));
+    }
+    if (tid < 6 && sl[tid]) atomicAdd(&lost6[cnt_slot() * 6 + tid], sl[tid]);
+    if (COLL && tid < 8 && se[tid])
+        atomicAdd(&events[cnt_slot() * 8 + tid], (unsigned long long)se[tid]);
+    if (tid == 0 && shole) atomicAdd(&holes[cnt_slot()], shole);
+}
+
 #define PUSH_INPLACE_PARAMS                                                                    \
     SpView sp, const uint32_t *__restrict__ nptr, const float2 *__restrict__ E, PushConst pc, \
         mcc::MccConst mc, uint32_t step, unsigned long long *__restrict__ q, int deposit,     \
@@ -1296,32 +1589,53 @@ __global__ void __launch_bounds__(256) k_push_inplace(PUSH_INPLACE_PARAMS) {
     push_inplace_body<V>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes, hist,
                          blockIdx.x);
 }
-// The collisionless variants fit 8 waves per SIMD in 42 VGPRs; left to
-// itself the scheduler gives SPAWN (PLAIN plus a rare queue write) 84 and 5
-// waves, so both ask for 8 (no spills).
 template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
+__global__ void __launch_bounds__(256) k_push_inplace<PV_GENERIC>(PUSH_INPLACE_PARAMS) {
+    push_inplace_generic(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes, hist,
+                         blockIdx.x);
+}
+// Waves per SIMD, measured over 4 to 8 at 257^2 and 1025^2 (20 and 10 steps
+// of the argon discharge): 7 for the collisionless variants (66-72 VGPRs) and
+// 5 for the collisional ones (87), 7.37 and 36.3 ms; 6 and 4: 7.58 and 37.0; 8
+// and 6 (a few spills): 7.63 and 37.0; 8 and 7 (ten): 8.05 and 37.9.
+#define INPL_WAVES_PLAIN 7
+#define INPL_WAVES_COLL 5
+template <>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
     k_push_inplace<PV_PLAIN>(PUSH_INPLACE_PARAMS) {
     push_inplace_body<PV_PLAIN>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
                                 hist, blockIdx.x);
 }
 template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
     k_push_inplace<PV_SPAWN>(PUSH_INPLACE_PARAMS) {
     push_inplace_body<PV_SPAWN>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
                                 hist, blockIdx.x);
 }
 template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
     k_push_inplace<PV_DEFER>(PUSH_INPLACE_PARAMS) {
     push_inplace_body<PV_DEFER>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
+                                hist, blockIdx.x);
+}
+
+template <>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_COLL, INPL_WAVES_COLL)))
+    k_push_inplace<PV_COLL_E>(PUSH_INPLACE_PARAMS) {
+    push_inplace_body<PV_COLL_E>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
+                                hist, blockIdx.x);
+}
+template <>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_COLL, INPL_WAVES_COLL)))
+    k_push_inplace<PV_COLL_I>(PUSH_INPLACE_PARAMS) {
+    push_inplace_body<PV_COLL_I>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
                                 hist, blockIdx.x);
 }
 
 // Both species' collisionless in-place passes in one launch (the first nba
 // blocks advance a, the rest b): the kernel of each species pass as it is,
 // one launch's fixed cost instead of two on the small grids
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
     k_push_inplace_pair(InplaceArgs a, InplaceArgs b, uint32_t nba,
                         const float2 *__restrict__ E, uint32_t step, int deposit) {
     if (blockIdx.x < nba)
@@ -1457,33 +1771,8 @@ __global__ void __launch_bounds__(256)
         sp.vx[i] = vx;
         sp.vy[i] = vy;
         sp.vz[i] = vz;
-        if (EV_KIND(ev) == mcc::EV_IONIZE) {
-            // ejected electron: born at the parent's position, pushed this
-            // step as the reference pushes particles appended before
-            // move_particles
-            PState ce = pre;
-            ce.vx = ch.vx;
-            ce.vy = ch.vy;
-            ce.vz = ch.vz;
-            push_one(ce, E, pc);
-            const int cst = classify(ce, pc.N, pc.mode);
-            if (cst != ST_KEPT) {
-                // left the domain during its first push: it still takes its
-                // id, but is not stored
-                atomicAdd(&lost6[cnt_slot() * 6 + cst - 1], 1u);
-                ce.jx = ce.jy = CELL_DEAD;
-            }
-            stage_put(spn.se, &spn.ce->stage_count, &spn.ce->overflow, ce, (unsigned long long)pid,
-                      pw);
-            // new ion at the same place; the ion pass of this step moves it;
-            // products take the parent's weight (e_collisions.cpp:413,441)
-            PState ci = pre;
-            ci.vx = ch.ivx;
-            ci.vy = ch.ivy;
-            ci.vz = ch.ivz;
-            stage_put(spn.si, &spn.ci->stage_count, &spn.ci->overflow, ci, (unsigned long long)pid,
-                      pw);
-        }
+        if (EV_KIND(ev) == mcc::EV_IONIZE)
+            stage_ionisation(ch, pre, pid, E, pc, spn, lost6, pw);
     }
     __syncthreads();
     if (threadIdx.x < 8 && se[threadIdx.x])

@@ -383,12 +383,14 @@ __device__ __forceinline__ bool candidate(const MccConst &c, uint32_t id, uint32
 // holds the ejected electron and the new ion; in REF mode EV_IONIZE means the
 // parent is removed.  inside: the particle passes the reference's
 // "inside the domain" test (e_collisions.cpp:507-511), used in REF mode.
+// CAND: the particle has passed its candidate test (PHYS).
+template <bool CAND = false>
 __device__ __forceinline__ int collide_electron(const MccConst &c, float &vx, float &vy, float &vz,
                                                 uint32_t id, uint32_t step, bool inside, Child &ch,
                                                 const float2 *tab) {
     const uint32_t s0 = (c.electron ? 0u : 16u);
     uint32_t r[4];
-    if (c.mode == PIC_DEV_MODE_REF) {
+    if (!CAND && c.mode == PIC_DEV_MODE_REF) {
         philox4x32_10(id, step, s0 + RS_MAIN, RNG_DOMAIN_MCC, c.key0, c.key1, r);
         if (!inside) return EV_NONE;
         float v2 = vx * vx + vy * vy + vz * vz;
@@ -430,7 +432,7 @@ __device__ __forceinline__ int collide_electron(const MccConst &c, float &vx, fl
     }
     // PHYS null collision
     const float2 bound = null_bound(c, vx * vx + vy * vy + vz * vz, tab);
-    {
+    if (!CAND) {
         uint32_t rc[2];
         philox2x32_10(id, step, c.key0 ^ (c.electron ? RNG_KEY_CAND_E : RNG_KEY_CAND_I), rc);
         if (!(u01(rc[0]) < bound.x)) return EV_NONE;
@@ -515,10 +517,11 @@ __device__ __forceinline__ int collide_electron(const MccConst &c, float &vx, fl
 // Ion collision (PHYS: isotropic elastic + charge exchange against a
 // Maxwellian neutral).  REF ion charge exchange is a per-column sequential
 // accumulator and is not handled here.
+template <bool CAND = false>
 __device__ __forceinline__ int collide_ion(const MccConst &c, float &vx, float &vy, float &vz,
                                            uint32_t id, uint32_t step) {
     const uint32_t s0 = 16u;
-    if (!candidate(c, id, step, vx * vx + vy * vy + vz * vz)) return EV_NONE;
+    if (!CAND && !candidate(c, id, step, vx * vx + vy * vy + vz * vz)) return EV_NONE;
     uint32_t r[4];
     philox4x32_10(id, step, s0 + RS_MAIN, RNG_DOMAIN_MCC, c.key0, c.key1, r);
     float nx, ny, nz;

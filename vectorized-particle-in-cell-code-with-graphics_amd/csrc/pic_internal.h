@@ -162,6 +162,9 @@ struct Spawn {
 };
 
 // ---- k_particles.hip
+// particles per block of the particle passes; a species' arrays are allocated
+// in whole blocks
+#define PASS_BLOCK 1024
 // words between consecutive counters of the sort histogram (binCount): each
 // key's counter has a 128-byte line of its own, so the per-block atomics of
 // different keys do not queue on a shared line
