@@ -292,7 +292,8 @@ enum PassVariant {
     PV_COLL_E = 2,
     PV_COLL_I = 3,
     PV_SPAWN = 4,
-    PV_DEFER = 5
+    PV_DEFER = 5,
+    PV_COMPACT = 6  // sort pass without a push (drops holes): the generic body, pinned
 };
 
 template <int V>
@@ -301,7 +302,7 @@ __device__ __forceinline__ void pin_variant(PushConst &pc, mcc::MccConst &mc, Sp
     pc.mode = PIC_DEV_MODE_PHYS;
     pc.bfield = 0;
     sp.w = nullptr;
-    if (V == PV_PLAIN || V == PV_SPAWN) {
+    if (V == PV_PLAIN || V == PV_SPAWN || V == PV_COMPACT) {
         mc.on = 0;
     } else if (V == PV_DEFER) {
         mc.on = 1;
@@ -317,8 +318,8 @@ __device__ __forceinline__ void pin_variant(PushConst &pc, mcc::MccConst &mc, Sp
 template <int V>
 __device__ __forceinline__ void pin_spawn(Spawn &spn) {
     if (V != PV_GENERIC) spn.plop = 0;
-    if (V == PV_PLAIN || V == PV_SPAWN || V == PV_DEFER) spn.wall = 0;
-    if (V == PV_PLAIN) spn.lost_ids = 0;
+    if (V == PV_PLAIN || V == PV_SPAWN || V == PV_DEFER || V == PV_COMPACT) spn.wall = 0;
+    if (V == PV_PLAIN || V == PV_COMPACT) spn.lost_ids = 0;
 }
 
 // A deferred pass's candidates of one round: the wavefront appends the
@@ -853,21 +854,17 @@ __device__ __forceinline__ void scatter_round(PState &s, uint32_t pid, float w, 
 // directly.
 //
 // LDS: one arena serves three phases -- the rank table (8 KB) beside the
-// collision queue (11 KB), or the hash table alone; then the deposit window
-// (as many nodes as the arena holds); then the write staging in two halves
-// of 512 particles.  Its size follows the waves per SIMD each variant's
-// registers allow: 25 KB for the collisionless variants (6 blocks per CU),
-// 32 KB for the collisional ones (4-5 blocks per CU).  The pass is bound by
-// memory latency: with 3 instead of 4 blocks per CU it took 20 % longer.
-#ifndef SCAT_WAVES_PLAIN
-#define SCAT_WAVES_PLAIN 6
-#endif
-#ifndef SCAT_ARENA_COLL
-#define SCAT_ARENA_COLL 4096
-#endif
+// collision queue (20 KB), or the hash table alone; then the deposit window
+// (as many nodes as the arena holds, a 62 x 62 fallback window); then the
+// write staging.  31 KB let five blocks share a CU, as the variants' 89-93
+// VGPRs do (5 waves per SIMD).  Measured, 20 steps at 257^2 and 10 at 1025^2
+// of the argon discharge: 5 waves 7.19 and 35.1 ms; collisionless variants at
+// 6 in 25 KB 7.22 and 35.1; collisional ones at 4 7.20 and 35.4.
+#define SCAT_WAVES 5
+#define SCAT_ARENA 3900
 template <int V>
 constexpr int scat_arena_u64() {
-    return (V == PV_PLAIN || V == PV_SPAWN) ? 3200 : SCAT_ARENA_COLL;
+    return V == PV_GENERIC ? 4096 : V == PV_COMPACT ? 3200 : SCAT_ARENA;
 }
 static_assert(SCAT_WIN + (11 * CQ_CAP * 4) / 8 <= 3200, "table + queue");
 static_assert(8 * (256 * IPP / 2) * 4 <= 3200 * 8, "staging half");
@@ -886,7 +883,10 @@ template <int V>
 __device__ __forceinline__ void push_scatter_body(PUSH_SCATTER_PARAMS) {
     pin_variant<V>(pc, mc, src);
     pin_spawn<V>(sp);
-    if (V != PV_GENERIC) dst.w = nullptr;
+    if (V == PV_COMPACT) {
+        dst.w = nullptr;
+        do_push = deposit = 0;
+    }
     if (blockIdx.x * (blockDim.x * IPP) >= *nptr) return;  // past the live count
     constexpr int ARENA = scat_arena_u64<V>();
     __shared__ unsigned long long arena[ARENA];
@@ -1111,34 +1111,393 @@ __device__ __forceinline__ void push_scatter_body(PUSH_SCATTER_PARAMS) {
     if (threadIdx.x == 0 && shole) atomicAdd(&holes[cnt_slot()], shole);
 }
 
+// ---- the passes with pinned options (physical mode, no magnetic field, no
+// per-particle weights)
+
+// A copy of the collision constants the compiler takes for new: expressions of
+// them are then evaluated where they are used.  (Hoisted out of the queue's
+// loop they are uniform floats in some 40 VGPRs, held across it.)
+__device__ __forceinline__ mcc::MccConst fresh(mcc::MccConst c) {
+    asm volatile("" : "+s"(c.mass), "+s"(c.M), "+s"(c.q), "+s"(c.ng), "+s"(c.opal_B), "+s"(c.vtn));
+    asm volatile("" : "+s"(c.e_exc), "+s"(c.e_iz), "+s"(c.kev_amu_div), "+s"(c.nu_max), "+s"(c.gas));
+    return c;
+}
+
+// mcc's block-level collisions on the pinned passes (COLL_E, COLL_I): the
+// candidates of the block's P x 256 particles are queued in LDS and collide
+// on dense lanes; vx and vy (and vz: VZ_BACK) come back to the particles'
+// lanes, everything else -- vz into the store, the event counts, the products of an ionisation -- is
+// settled by the lane that made the collision, so none of it takes code or
+// registers in the particles' rounds.  The queue holds every particle of the
+// block (5 words each): it cannot overflow.  q: free on entry and again after
+// the next barrier.  The store's words of the block are not yet overwritten.
+#define CQ_WORDS 5
+template <int P, bool VZ_BACK>
+__device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)[P],
+                                              float (&vy)[P], float (&vz)[P],
+                                              const uint32_t (&id)[P], const SpView &sp,
+                                              uint32_t blk0, const float2 *__restrict__ E,
+                                              const PushConst &pc, const mcc::MccConst &mc0,
+                                              uint32_t step, const Spawn &spn,
+                                              uint32_t *__restrict__ lost6, uint32_t *se,
+                                              const float2 *tab, float *q) {
+    constexpr uint32_t CAP = P * 256;
+    __shared__ uint32_t wcnt[4];
+    uint32_t *qu = reinterpret_cast<uint32_t *>(q);  // v (3), id, slot
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    uint32_t pos[P], wtot = 0;
+#pragma unroll
+    for (int r = 0; r < P; r++) {
+        const bool cand =
+            live[r] && mcc::candidate(mc0, id[r], step,
+                                      vx[r] * vx[r] + vy[r] * vy[r] + vz[r] * vz[r], tab);
+        const uint64_t bal = __ballot(cand);
+        pos[r] = cand ? wtot + (uint32_t)__popcll(bal & below) : 0xFFFFFFFFu;
+        wtot += (uint32_t)__popcll(bal);
+    }
+    if (lane == 0) wcnt[w] = wtot;
+    __syncthreads();
+    uint32_t base = 0, total = 0;
+    for (int k = 0; k < 4; k++) {
+        if (k < w) base += wcnt[k];
+        total += wcnt[k];
+    }
+#pragma unroll
+    for (int r = 0; r < P; r++) {
+        if (pos[r] != 0xFFFFFFFFu) {
+            const uint32_t t = pos[r] += base;
+            q[t] = vx[r];
+            q[CAP + t] = vy[r];
+            q[2 * CAP + t] = vz[r];
+            qu[3 * CAP + t] = id[r];
+            qu[4 * CAP + t] = blk0 + threadIdx.x + r * 256;
+        }
+    }
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < total; t += 256) {
+        const mcc::MccConst mc = fresh(mc0);
+        float ux = q[t], uy = q[CAP + t], uz = q[2 * CAP + t];
+        const uint32_t pid = qu[3 * CAP + t], i = qu[4 * CAP + t];
+        mcc::Child ch{};
+        const int ev = mc.electron
+                           ? mcc::collide_electron<true>(mc, ux, uy, uz, pid, step, true, ch, tab)
+                           : mcc::collide_ion<true>(mc, ux, uy, uz, pid, step);
+        q[t] = ux;
+        q[CAP + t] = uy;
+        if (VZ_BACK)
+            q[2 * CAP + t] = uz;
+        else
+            sp.vz[i] = uz;
+        if (EV_KIND(ev) > 0) atomicAdd(&se[EV_KIND(ev)], 1u);
+        if (ev & EV_OVER_BOUND) atomicAdd(&se[6], 1u);
+        if (EV_KIND(ev) == mcc::EV_IONIZE)
+            stage_ionisation(ch, load_state(sp, i, false), pid, E, pc, spn, lost6, 1.0f);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < P; r++)
+        if (pos[r] != 0xFFFFFFFFu) {
+            vx[r] = q[pos[r]];
+            vy[r] = q[CAP + pos[r]];
+            if (VZ_BACK) vz[r] = q[2 * CAP + pos[r]];
+        }
+}
+
+// gather_one's field of two particles, every load issued before the first is
+// used; a particle that cannot move (ok false) reads node 0
+__device__ __forceinline__ void gather_two(const PState (&s)[2], const bool (&ok)[2],
+                                           const float2 *__restrict__ E, int N, float (&ex)[2],
+                                           float (&ey)[2]) {
+    float2 e00[2], e01[2], e10[2], e11[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const uint32_t b = ok[r] ? (uint32_t)(s[r].jy * N + s[r].jx) : 0u;
+        const float2 *lo = E + b, *hi = E + (b + (uint32_t)N);
+        e00[r] = lo[0];
+        e01[r] = lo[1];
+        e10[r] = hi[0];
+        e11[r] = hi[1];
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const float wj = s[r].ox, wk = s[r].oy;
+        const float a4 = (1.0f - wj) * (1.0f - wk), a3 = wj * (1.0f - wk);
+        const float a2 = wk * (1.0f - wj), a1 = wj * wk;
+        ex[r] = a4 * e00[r].x + a3 * e01[r].x + a2 * e10[r].x + a1 * e11[r].x;
+        ey[r] = a4 * e00[r].y + a3 * e01[r].y + a2 * e10[r].y + a1 * e11[r].y;
+    }
+}
+
+// reposition without branches
+__device__ __forceinline__ void reposition_sel(int j, float t, int &jn, float &on) {
+    const float k0 = floorf(t), f0 = t - k0;
+    const bool up = f0 >= 1.0f;  // t just below an integer: t - k rounded up to 1
+    const int jj = min(max(j + (int)(up ? k0 + 1.0f : k0), -CELL_FAR), CELL_FAR);
+    const bool in = t > -POS_GUARD && t < POS_GUARD;  // false for NaN
+    jn = in ? jj : (t > 0.0f ? CELL_FAR : -CELL_FAR);
+    on = (in && !up) ? f0 : 0.0f;
+}
+
+// move_one without a magnetic field; ok false: unchanged
+__device__ __forceinline__ void move_sel(PState &s, bool ok, float ex, float ey,
+                                         const PushConst &pc) {
+    float ux = s.vx + pc.cE * ex, uy = s.vy + pc.cE * ey;
+    ux = ux + pc.cE * ex;
+    uy = uy + pc.cE * ey;
+    int jx, jy;
+    float ox, oy;
+    reposition_sel(s.jx, s.ox + ux * pc.dtdx, jx, ox);
+    reposition_sel(s.jy, s.oy + uy * pc.dtdy, jy, oy);
+    s.jx = ok ? jx : s.jx;
+    s.jy = ok ? jy : s.jy;
+    s.ox = ok ? ox : s.ox;
+    s.oy = ok ? oy : s.oy;
+    s.vx = ok ? ux : s.vx;
+    s.vy = ok ? uy : s.vy;
+}
+
+__device__ __forceinline__ bool inside_cells(const PState &s, int N) {
+    return (unsigned)s.jx <= (unsigned)(N - 2) && (unsigned)s.jy <= (unsigned)(N - 2);
+}
+
+// The sort pass's pinned variants, with the push: push_scatter_body's plan in
+// push_inplace_body's form (every load first, field loads of two particles at
+// a time, straight-line rounds, collisions settled on the queue's lanes).
+// Bound by the scattered writes (1025^2, a sort every 3rd pass: 5.5 GB written
+// for 2.9 GB of particles, runs of about 16 particles per tile) and the flush
+// atomics; 2.93 -> 2.57 ms at 104.9 M electrons over the one-particle rounds.
+template <int V>
+__device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
+    pin_variant<V>(pc, mc, src);
+    pin_spawn<V>(sp);
+    constexpr bool COLL = V == PV_COLL_E || V == PV_COLL_I;
+    const uint32_t n = *nptr, blk0 = blockIdx.x * (256 * IPP);
+    if (blk0 >= n) return;  // past the live count
+    constexpr int ARENA = scat_arena_u64<V>();
+    __shared__ unsigned long long arena[ARENA];
+    __shared__ uint32_t se[8], sl[6], s_total, shole;
+    __shared__ int wmin[4], wmax[4];
+    __shared__ float2 sbins[MCC_BINS];
+    uint32_t *tcnt = reinterpret_cast<uint32_t *>(arena);  // per key: count, then staging base
+    uint32_t *tkey = tcnt + SCAT_WIN;                      // per key: slot of its rank 0
+    float *cq = reinterpret_cast<float *>(arena + SCAT_WIN);  // collision queue behind the table
+    static_assert(!COLL || SCAT_WIN + CQ_WORDS * IPP * 256 / 2 <= ARENA, "table + queue");
+    const uint32_t tid = threadIdx.x;
+    if (tid < 8) se[tid] = 0;
+    if (tid < 6) sl[tid] = 0;
+    if (tid == 0) s_total = shole = 0;
+    uint32_t c0[IPP], pid[IPP];
+    float ox[IPP], oy[IPP], vx[IPP], vy[IPP], vz[IPP];
+    {
+        const uint32_t *pc_ = src.cell + blk0, *pi = src.id + blk0;
+        const float *px = src.ox + blk0, *py = src.oy + blk0, *pu = src.vx + blk0,
+                    *pv = src.vy + blk0, *pz = src.vz + blk0;
+#pragma unroll
+        for (int r = 0; r < IPP; r++) {  // every load first
+            c0[r] = pc_[tid + r * 256];
+            pid[r] = pi[tid + r * 256];
+            vx[r] = pu[tid + r * 256];
+            vy[r] = pv[tid + r * 256];
+            vz[r] = pz[tid + r * 256];
+            ox[r] = px[tid + r * 256];
+            oy[r] = py[tid + r * 256];
+        }
+    }
+    if (COLL && mc.bins && tid < MCC_BINS) sbins[tid] = mc.bins[tid];
+    bool claim[IPP];  // the slots k_key_count counted, keyed by the cell before the step
+    uint32_t ent[IPP], rank[IPP];
+    int kmin = 0x7FFFFFFF, kmax = -1;
+#pragma unroll
+    for (int r = 0; r < IPP; r++) {
+        const int jx = cell_jx(c0[r]);
+        claim[r] = blk0 + tid + r * 256 < n && jx != CELL_HOLE;
+        ent[r] = bin_key(jx, cell_jy(c0[r]), pc.tilesX) >> pc.keyshift;
+        kmin = min(kmin, claim[r] ? (int)ent[r] : 0x7FFFFFFF);
+        kmax = max(kmax, claim[r] ? (int)ent[r] : -1);
+    }
+    kmin = wave_min(kmin);
+    kmax = wave_max(kmax);
+    if ((tid & 63) == 0) {
+        wmin[tid >> 6] = kmin;
+        wmax[tid >> 6] = kmax;
+    }
+    __syncthreads();  // counters cleared, key range known, bounds staged
+    kmin = min(min(wmin[0], wmin[1]), min(wmin[2], wmin[3]));
+    kmax = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+    const int span = kmax - kmin + 1;      // <= 0: no claims
+    const bool direct = span <= SCAT_WIN;  // uniform over the block
+    // `late`: each of the first threads holds one key's claim in flight over
+    // the collisions and the push; a wider table claims at once
+    const bool late = span <= 256;
+    uint32_t cnt0 = 0u, old0 = 0u, st0 = 0u;
+    if (direct) {
+        for (int e = tid; e < span; e += 256) tcnt[e] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPP; r++) {
+            ent[r] -= (uint32_t)kmin;
+            rank[r] = 0u;
+            if (claim[r]) rank[r] = atomicAdd(&tcnt[ent[r]], 1u);
+        }
+        __syncthreads();
+        // one claim per distinct key: the bin count runs down from its total,
+        // so the block's c particles of key k take the slots start(k) + old -
+        // c + rank, rank < c
+        for (int e = tid; e < span; e += 256) {
+            const uint32_t c = tcnt[e];
+            if (!c) continue;
+            const uint32_t old = atomicSub(&binCount[(size_t)(kmin + e) * BIN_STRIDE], c);
+            const uint32_t st = binStart[kmin + e];
+            if (late) {
+                cnt0 = c;
+                old0 = old;
+                st0 = st;
+            } else {
+                tkey[e] = st + old - c;
+                tcnt[e] = atomicAdd(&s_total, c);
+            }
+        }
+    } else {
+        // wide block (an unsorted store, or the particles appended since the
+        // last sort): ranks in the LDS hash table, one claim per distinct key,
+        // every slot (in rank) known before the collision queue takes the LDS
+        BlockHash &H = *reinterpret_cast<BlockHash *>(arena);
+        hash_clear(H);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPP; r++) ent[r] = hash_insert(H, ent[r], claim[r], rank[r]);
+        __syncthreads();
+        for (int e = tid; e < HASH_SIZE; e += 256) {
+            const uint32_t k = H.key[e], c = H.cnt[e];
+            if (k != HASH_EMPTY)
+                H.key[e] = binStart[k] + atomicSub(&binCount[(size_t)k * BIN_STRIDE], c) - c;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPP; r++)
+            if (claim[r]) rank[r] += H.key[ent[r]];
+        __syncthreads();
+    }
+    if (COLL)
+        collide_queue<IPP, true>(claim, vx, vy, vz, pid, src, blk0, E, pc, mc, step, sp, lost6, se,
+                                 mc.bins ? sbins : nullptr, cq);
+    PState s[IPP];
+    bool kept[IPP];
+    float w[IPP];
+#pragma unroll
+    for (int h = 0; h < IPP; h += 2) {
+        PState t[2];
+        bool ok[2];
+        float ex[2], ey[2];
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const int r = h + g;
+            t[g] = PState{cell_jx(c0[r]), cell_jy(c0[r]), ox[r], oy[r], vx[r], vy[r], vz[r]};
+            ok[g] = claim[r] && inside_cells(t[g], pc.N);
+        }
+        gather_two(t, ok, E, pc.N, ex, ey);
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const int r = h + g;
+            s[r] = t[g];
+            w[r] = 1.0f;
+            move_sel(s[r], ok[g], ex[g], ey[g], pc);
+            kept[r] = claim[r] && inside_cells(s[r], pc.N);
+            if (claim[r] && !kept[r]) {
+                atomicAdd(&sl[classify(s[r], pc.N, pc.mode) - 1], 1u);
+                atomicAdd(&shole, 1u);
+                if (sp.lost_ids) queue_lost(sp, pid[r], 1.0f);
+                if (COLL && sp.wall)  // waits for the surface pass
+                    stage_put(sp.wq, &sp.cw->wall_count, &sp.cw->overflow, s[r],
+                              (unsigned long long)pid[r]);
+            }
+        }
+    }
+    if (direct) {
+        if (late && cnt0) {
+            tkey[tid] = st0 + old0 - cnt0;
+            tcnt[tid] = atomicAdd(&s_total, cnt0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < IPP; r++) {  // the slot, and the place in slot order
+            const uint32_t e = claim[r] ? ent[r] : 0u;
+            ent[r] = tcnt[e] + rank[r];
+            rank[r] = tkey[e] + rank[r];
+        }
+    }
+    __syncthreads();  // the table is read; the deposit window reuses the LDS
+    if (deposit) block_deposit_n<IPP, ARENA>(kept, s, w, q, pc.N, arena);
+    __syncthreads();
+    if (direct) {
+        // the claimed slots staged in slot order, SH at a time (a claimed
+        // slot of a particle that left holds a hole)
+        constexpr uint32_t SH = ARENA / 4 < 256 * IPP ? ARENA / 4 : 256 * IPP;
+        uint32_t *stg = reinterpret_cast<uint32_t *>(arena);  // 8 words x SH, SoA
+        const uint32_t tot = s_total;
+        for (uint32_t lo = 0; lo < tot; lo += SH) {  // uniform: tot is the block's
+#pragma unroll
+            for (int r = 0; r < IPP; r++) {
+                const uint32_t l = ent[r] - lo;
+                if (claim[r] && l < SH) {
+                    stg[l] = rank[r];
+                    stg[SH + l] =
+                        kept[r] ? cell_pack(s[r].jx, s[r].jy) : cell_pack(CELL_HOLE, CELL_HOLE);
+                    stg[2 * SH + l] = __float_as_uint(s[r].ox);
+                    stg[3 * SH + l] = __float_as_uint(s[r].oy);
+                    stg[4 * SH + l] = __float_as_uint(s[r].vx);
+                    stg[5 * SH + l] = __float_as_uint(s[r].vy);
+                    stg[6 * SH + l] = __float_as_uint(s[r].vz);
+                    stg[7 * SH + l] = pid[r];
+                }
+            }
+            __syncthreads();
+            const uint32_t m = min(SH, tot - lo);
+            for (uint32_t l = tid; l < m; l += 256) {
+                const uint32_t d = stg[l];
+                if (d < cap) {
+                    dst.cell[d] = stg[SH + l];
+                    dst.ox[d] = __uint_as_float(stg[2 * SH + l]);
+                    dst.oy[d] = __uint_as_float(stg[3 * SH + l]);
+                    dst.vx[d] = __uint_as_float(stg[4 * SH + l]);
+                    dst.vy[d] = __uint_as_float(stg[5 * SH + l]);
+                    dst.vz[d] = __uint_as_float(stg[6 * SH + l]);
+                    dst.id[d] = stg[7 * SH + l];
+                }
+            }
+            __syncthreads();  // written out before the next part fills it
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < IPP; r++)
+            if (claim[r] && rank[r] < cap) {
+                PState o = s[r];
+                if (!kept[r]) o.jx = o.jy = CELL_HOLE;
+                store_state(dst, rank[r], o, pid[r]);
+            }
+    }
+    if (COLL && tid < 8 && se[tid])
+        atomicAdd(&events[cnt_slot() * 8 + tid], (unsigned long long)se[tid]);
+    if (tid < 6 && sl[tid]) atomicAdd(&lost6[cnt_slot() * 6 + tid], sl[tid]);
+    if (tid == 0 && shole) atomicAdd(&holes[cnt_slot()], shole);
+}
+
 template <int V>
 __global__ void __launch_bounds__(256) k_push_scatter(PUSH_SCATTER_PARAMS) {
     push_scatter_body<V>(PUSH_SCATTER_ARGS);
 }
-// The collisionless variants fit 6 waves per SIMD in 76 VGPRs without spills
-// (7 spill, and measured slower); left to itself the compiler gives them 110
-// (4 waves).  The collisional ones keep their 117 (4 waves).
-template <>
-__global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(SCAT_WAVES_PLAIN, SCAT_WAVES_PLAIN)))
-    k_push_scatter<PV_PLAIN>(PUSH_SCATTER_PARAMS) {
-    push_scatter_body<PV_PLAIN>(PUSH_SCATTER_ARGS);
-}
-template <>
-__global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(SCAT_WAVES_PLAIN, SCAT_WAVES_PLAIN)))
-    k_push_scatter<PV_SPAWN>(PUSH_SCATTER_PARAMS) {
-    push_scatter_body<PV_SPAWN>(PUSH_SCATTER_ARGS);
-}
-#ifdef SCAT_WAVES_COLL
-template <>
-__global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(SCAT_WAVES_COLL, SCAT_WAVES_COLL)))
-    k_push_scatter<PV_COLL_E>(PUSH_SCATTER_PARAMS) {
-    push_scatter_body<PV_COLL_E>(PUSH_SCATTER_ARGS);
-}
-#endif
-
+#define SCATTER_FAST(V)                                                        \
+    template <>                                                                \
+    __global__ void __launch_bounds__(256)                                     \
+        __attribute__((amdgpu_waves_per_eu(SCAT_WAVES, SCAT_WAVES)))           \
+        k_push_scatter<V>(PUSH_SCATTER_PARAMS) {                               \
+        push_scatter_fast<V>(PUSH_SCATTER_ARGS);                               \
+    }
+SCATTER_FAST(PV_PLAIN)
+SCATTER_FAST(PV_SPAWN)
+SCATTER_FAST(PV_COLL_E)
+SCATTER_FAST(PV_COLL_I)
 
 // one particle of the generic k_push_inplace: collide (block-wide when blk), push, store
 // in place or leave a hole, count, stage products; dep = deposit it
@@ -1270,152 +1629,6 @@ __device__ __forceinline__ void push_inplace_generic(
     if (threadIdx.x == 0 && shole) atomicAdd(&holes[cnt_slot()], shole);
 }
 
-// ---- the passes with pinned options (physical mode, no magnetic field, no
-// per-particle weights)
-
-// A copy of the collision constants the compiler takes for new: expressions of
-// them are then evaluated where they are used.  (Hoisted out of the queue's
-// loop they are uniform floats in some 40 VGPRs, held across it.)
-__device__ __forceinline__ mcc::MccConst fresh(mcc::MccConst c) {
-    asm volatile("" : "+s"(c.mass), "+s"(c.M), "+s"(c.q), "+s"(c.ng), "+s"(c.opal_B), "+s"(c.vtn));
-    asm volatile("" : "+s"(c.e_exc), "+s"(c.e_iz), "+s"(c.kev_amu_div), "+s"(c.nu_max), "+s"(c.gas));
-    return c;
-}
-
-// mcc's block-level collisions on the pinned passes (COLL_E, COLL_I): the
-// candidates of the block's P x 256 particles are queued in LDS and collide
-// on dense lanes; vx and vy come back to the particles' lanes, everything
-// else -- the new vz, the event counts, the products of an ionisation -- is
-// settled by the lane that made the collision, so none of it takes code or
-// registers in the particles' rounds.  The queue holds every particle of the
-// block (5 words each): it cannot overflow.  q: free on entry and again after
-// the next barrier.  The store's words of the block are not yet overwritten.
-#define CQ_WORDS 5
-template <int P>
-__device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)[P],
-                                              float (&vy)[P], const float (&vz)[P],
-                                              const uint32_t (&id)[P], const SpView &sp,
-                                              uint32_t blk0, const float2 *__restrict__ E,
-                                              const PushConst &pc, const mcc::MccConst &mc0,
-                                              uint32_t step, const Spawn &spn,
-                                              uint32_t *__restrict__ lost6, uint32_t *se,
-                                              const float2 *tab, float *q) {
-    constexpr uint32_t CAP = P * 256;
-    __shared__ uint32_t wcnt[4];
-    uint32_t *qu = reinterpret_cast<uint32_t *>(q);  // v (3), id, slot
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    uint32_t pos[P], wtot = 0;
-#pragma unroll
-    for (int r = 0; r < P; r++) {
-        const bool cand =
-            live[r] && mcc::candidate(mc0, id[r], step,
-                                      vx[r] * vx[r] + vy[r] * vy[r] + vz[r] * vz[r], tab);
-        const uint64_t bal = __ballot(cand);
-        pos[r] = cand ? wtot + (uint32_t)__popcll(bal & below) : 0xFFFFFFFFu;
-        wtot += (uint32_t)__popcll(bal);
-    }
-    if (lane == 0) wcnt[w] = wtot;
-    __syncthreads();
-    uint32_t base = 0, total = 0;
-    for (int k = 0; k < 4; k++) {
-        if (k < w) base += wcnt[k];
-        total += wcnt[k];
-    }
-#pragma unroll
-    for (int r = 0; r < P; r++) {
-        if (pos[r] != 0xFFFFFFFFu) {
-            const uint32_t t = pos[r] += base;
-            q[t] = vx[r];
-            q[CAP + t] = vy[r];
-            q[2 * CAP + t] = vz[r];
-            qu[3 * CAP + t] = id[r];
-            qu[4 * CAP + t] = blk0 + threadIdx.x + r * 256;
-        }
-    }
-    __syncthreads();
-    for (uint32_t t = threadIdx.x; t < total; t += 256) {
-        const mcc::MccConst mc = fresh(mc0);
-        float ux = q[t], uy = q[CAP + t], uz = q[2 * CAP + t];
-        const uint32_t pid = qu[3 * CAP + t], i = qu[4 * CAP + t];
-        mcc::Child ch{};
-        const int ev = mc.electron
-                           ? mcc::collide_electron<true>(mc, ux, uy, uz, pid, step, true, ch, tab)
-                           : mcc::collide_ion<true>(mc, ux, uy, uz, pid, step);
-        q[t] = ux;
-        q[CAP + t] = uy;
-        sp.vz[i] = uz;
-        if (EV_KIND(ev) > 0) atomicAdd(&se[EV_KIND(ev)], 1u);
-        if (ev & EV_OVER_BOUND) atomicAdd(&se[6], 1u);
-        if (EV_KIND(ev) == mcc::EV_IONIZE)
-            stage_ionisation(ch, load_state(sp, i, false), pid, E, pc, spn, lost6, 1.0f);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < P; r++)
-        if (pos[r] != 0xFFFFFFFFu) {
-            vx[r] = q[pos[r]];
-            vy[r] = q[CAP + pos[r]];
-        }
-}
-
-// gather_one's field of two particles, every load issued before the first is
-// used; a particle that cannot move (ok false) reads node 0
-__device__ __forceinline__ void gather_two(const PState (&s)[2], const bool (&ok)[2],
-                                           const float2 *__restrict__ E, int N, float (&ex)[2],
-                                           float (&ey)[2]) {
-    float2 e00[2], e01[2], e10[2], e11[2];
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-        const uint32_t b = ok[r] ? (uint32_t)(s[r].jy * N + s[r].jx) : 0u;
-        const float2 *lo = E + b, *hi = E + (b + (uint32_t)N);
-        e00[r] = lo[0];
-        e01[r] = lo[1];
-        e10[r] = hi[0];
-        e11[r] = hi[1];
-    }
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-        const float wj = s[r].ox, wk = s[r].oy;
-        const float a4 = (1.0f - wj) * (1.0f - wk), a3 = wj * (1.0f - wk);
-        const float a2 = wk * (1.0f - wj), a1 = wj * wk;
-        ex[r] = a4 * e00[r].x + a3 * e01[r].x + a2 * e10[r].x + a1 * e11[r].x;
-        ey[r] = a4 * e00[r].y + a3 * e01[r].y + a2 * e10[r].y + a1 * e11[r].y;
-    }
-}
-
-// reposition without branches
-__device__ __forceinline__ void reposition_sel(int j, float t, int &jn, float &on) {
-    const float k0 = floorf(t), f0 = t - k0;
-    const bool up = f0 >= 1.0f;  // t just below an integer: t - k rounded up to 1
-    const int jj = min(max(j + (int)(up ? k0 + 1.0f : k0), -CELL_FAR), CELL_FAR);
-    const bool in = t > -POS_GUARD && t < POS_GUARD;  // false for NaN
-    jn = in ? jj : (t > 0.0f ? CELL_FAR : -CELL_FAR);
-    on = (in && !up) ? f0 : 0.0f;
-}
-
-// move_one without a magnetic field; ok false: unchanged
-__device__ __forceinline__ void move_sel(PState &s, bool ok, float ex, float ey,
-                                         const PushConst &pc) {
-    float ux = s.vx + pc.cE * ex, uy = s.vy + pc.cE * ey;
-    ux = ux + pc.cE * ex;
-    uy = uy + pc.cE * ey;
-    int jx, jy;
-    float ox, oy;
-    reposition_sel(s.jx, s.ox + ux * pc.dtdx, jx, ox);
-    reposition_sel(s.jy, s.oy + uy * pc.dtdy, jy, oy);
-    s.jx = ok ? jx : s.jx;
-    s.jy = ok ? jy : s.jy;
-    s.ox = ok ? ox : s.ox;
-    s.oy = ok ? oy : s.oy;
-    s.vx = ok ? ux : s.vx;
-    s.vy = ok ? uy : s.vy;
-}
-
-__device__ __forceinline__ bool inside_cells(const PState &s, int N) {
-    return (unsigned)s.jx <= (unsigned)(N - 2) && (unsigned)s.jy <= (unsigned)(N - 2);
-}
-
 // LDS of an in-place pass (u64 words): the collision queue, then the deposit
 // window, then the sort histogram (which needs 16 KB).  The electrons'
 // collisional variant takes a 58 x 58 fallback window (28 KB, five blocks per
@@ -1497,7 +1710,7 @@ __device__ __forceinline__ void push_inplace_body(
     }
     __syncthreads();  // counters initialised, bounds staged
     if (COLL)
-        collide_queue<IPP>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step, spn, lost6, se,
+        collide_queue<IPP, false>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step, spn, lost6, se,
                            mc.bins ? sbins : nullptr, reinterpret_cast<float *>(lds));
     if (V == PV_DEFER) {
         // a candidate stays as it is for k_collide_q (a deferring species has
@@ -2475,10 +2688,21 @@ void launch_push_scatter(hipStream_t st, const SpView &src, const SpView &dst, c
                          uint32_t step, uint32_t *binCount, const uint32_t *binStart,
                          unsigned long long *q, int do_push, int deposit, const Spawn &spn,
                          unsigned long long *events, uint32_t *lost6, uint32_t *holes) {
-    const int v = (dst.w == nullptr) ? pass_variant(src, pc, mc, &spn) : PV_GENERIC;
-    LAUNCH_VARIANT(v, k_push_scatter, dim3(blocks_for(cap, 256 * IPP)), st, src, dst, n,
-                   (uint32_t)cap, E, pc, mc, step, binCount, binStart, q, do_push, deposit, spn,
-                   events, lost6, holes);
+    int v = (dst.w == nullptr) ? pass_variant(src, pc, mc, &spn) : PV_GENERIC;
+    if (v != PV_GENERIC && !do_push) v = PV_COMPACT;
+    const dim3 grid(blocks_for(cap, 256 * IPP)), blk(256);
+#define SCATTER(V)                                                                              \
+    hipLaunchKernelGGL(k_push_scatter<V>, grid, blk, 0, st, src, dst, n, (uint32_t)cap, E, pc, mc, \
+                       step, binCount, binStart, q, do_push, deposit, spn, events, lost6, holes)
+    switch (v) {
+    case PV_PLAIN: SCATTER(PV_PLAIN); break;
+    case PV_SPAWN: SCATTER(PV_SPAWN); break;
+    case PV_COLL_E: SCATTER(PV_COLL_E); break;
+    case PV_COLL_I: SCATTER(PV_COLL_I); break;
+    case PV_COMPACT: SCATTER(PV_COMPACT); break;
+    default: SCATTER(PV_GENERIC); break;  // a sort pass defers no collisions
+    }
+#undef SCATTER
 }
 
 void launch_push_inplace(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
