@@ -2,8 +2,8 @@
 (every option at run time), which a species with per-particle weights takes:
 the same run with every weight set to 1 must end in the same state, bit for
 bit, at particle counts around a block's edges, for the collisionless, the
-block-queued and the deferred collisional passes, and with more collision
-candidates than one round of a block's lanes."""
+electrons' and the ions' collisional passes, and with more collision candidates
+than one round of a block's lanes."""
 import numpy as np
 import pytest
 
@@ -42,8 +42,8 @@ def test_pinned_passes_match_the_generic_pass(n, kind):
     gas, pressure, wall = {
         "plain": (pic2d.GAS_ARGON, 0.0, pic2d.WALL_ABSORB),
         "spawn": (pic2d.GAS_ARGON, 0.0, pic2d.WALL_STEADY),
-        "argon": (pic2d.GAS_ARGON, 66.0, pic2d.WALL_STEADY),       # ions deferred
-        "hydrogen": (pic2d.GAS_HYDROGEN, 66.0, pic2d.WALL_STEADY),  # ions in the block queue
+        "argon": (pic2d.GAS_ARGON, 66.0, pic2d.WALL_STEADY),
+        "hydrogen": (pic2d.GAS_HYDROGEN, 66.0, pic2d.WALL_STEADY),
         # most particles are candidates: the queue holds whole blocks
         "dense": (pic2d.GAS_ARGON, 60000.0, pic2d.WALL_ABSORB),
     }[kind]

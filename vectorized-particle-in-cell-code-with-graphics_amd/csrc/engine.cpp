@@ -253,8 +253,6 @@ void species_free(Species &s) {
     for (void *p : wq)
         if (p) hipFree(p);
     if (s.rstate) hipFree(s.rstate);
-    if (s.mq) hipFree(s.mq);
-    if (s.mq_cnt) hipFree(s.mq_cnt);
     if (s.mc_bins) hipFree(s.mc_bins);
     for (int b = 0; b < 2; b++)
         if (s.qbuf[b]) hipFree(s.qbuf[b]);
@@ -455,8 +453,6 @@ Spawn make_spawn(pic_handle *h, bool plop, int si) {
     sp.plop_ref = 0;
     sp.wall = (h->wall_on && si >= 0) ? 1 : 0;
     sp.lost_ids = 0;
-    sp.mq = sp.mq_cnt = nullptr;
-    sp.mq_seg = 0;
     if (sp.wall) {
         sp.wq = h->sp[si].wq;
         sp.cw = &h->cnt[si];
@@ -760,21 +756,6 @@ int check_overflow(pic_handle *h, bool wait) {
     return PIC_OK;
 }
 
-// Physical-mode collisions run in a pass of their own ahead of the particle
-// pass when few particles are candidates (the argon ions: a fraction of a
-// percent): that pass then has the registers of a collisionless one, for 8
-// B per particle read ahead.  Where many are (the electrons: ~13 % under the
-// global bound), the candidates' velocities would cost a read and write of
-// nearly every line, and the particle pass collides them in its block queue
-// instead.  With energy-binned bounds (about 2 % candidates in a 2 eV argon
-// discharge) the deferred form was measured too: the electrons' in-place
-// pass fell from 1.69 to 1.35 ms at 1025^2, but colliding, pushing and
-// depositing the 2 M queued candidates took 0.43 ms, so they collide in the
-// pass.
-bool collide_ahead(const Species &s) {
-    return s.mc.on && s.mc.mode == PIC_DEV_MODE_PHYS && s.mc.p_null < 0.02f && !s.mc.bins;
-}
-
 // counting sort + (optional) collisions and push + deposit of one species.
 // The keys are the cells at the start of the pass; with a push, the
 // particles lost in the pass leave holes in the sorted store (counted in the
@@ -787,11 +768,6 @@ void push_species(pic_handle *h, int si, int do_push, int deposit) {
     mcc::MccConst mc = s.mc;
     if (!do_push) mc.on = 0;
     Spawn spn = pass_spawn(h, si, do_push);
-    if (do_push && collide_ahead(s) && s.mq) {
-        launch_collide(h->st, s.buf[c], &h->cnt[si].n[c], s.cap, h->E32, s.pc, mc, step, spn,
-                       &h->cnt[si].events[0][0], &h->cnt[si].lost[0][0], s.mq, s.mq_cnt);
-        mc.on = 0;
-    }
     clear_holes(h, si);  // the pass drops the old holes
     uint32_t *bins = bin_count(h, si);
     // the in-place pass before a timestep's sort pass has made its histogram
@@ -830,18 +806,9 @@ void push_species_inplace(pic_handle *h, int si) {
     Species &s = h->sp[si];
     int c = s.cur;
     Spawn spn = pass_spawn(h, si, 1);
-    // few candidates: the pass makes the candidate test only and leaves each
-    // candidate to k_collide_q (collide, push, store, deposit) after it
-    const bool defer = collide_ahead(s) && s.mq;
-    // the next pass of this species sorts: this one (and the deferred
-    // collisions after it) count its keys
+    // the next pass of this species sorts: this one counts its keys
     drop_hist(h, si);
     const bool hist = s.since_sort + 2 >= s.sort_interval && hist_fusable(h, si);
-    if (defer) {  // the queue counters are zero (k_collide_q leaves them so)
-        spn.mq = s.mq;
-        spn.mq_cnt = s.mq_cnt;
-        spn.mq_seg = collide_seg_cap(s.cap);
-    }
     int p = prof_begin(h, 6);
     launch_push_inplace(h->st, s.buf[c], &h->cnt[si].n[c], s.cap, h->E32, s.pc, s.mc,
                         (uint32_t)h->step, s.q, 1, spn, &h->cnt[si].events[0][0],
@@ -849,10 +816,6 @@ void push_species_inplace(pic_handle *h, int si) {
                         hist ? bin_count(h, si) : nullptr);
     s.hist_pending = hist;
     prof_end(h, p);
-    if (defer)
-        launch_collide_deferred(h->st, s.buf[c], h->E32, s.pc, s.mc, (uint32_t)h->step, spn,
-                                &h->cnt[si].events[0][0], &h->cnt[si].lost[0][0], s.q,
-                                &h->cnt[si].holes[0], hist ? bin_count(h, si) : nullptr);
     plop_drain(h, si, 1);
     s.holes = true;
     s.since_sort++;
@@ -1353,14 +1316,6 @@ int pic_create(const pic_params *Pin, int restart, const char *dump_dir, pic_han
     }
     if ((rc = setup_mcc(h, h->sp[0], true)) != PIC_OK || (rc = setup_mcc(h, h->sp[1], false)) != PIC_OK)
         return fail(rc);
-    for (int s = 0; s < 2; s++) {
-        Species &sp = h->sp[s];
-        if (!collide_ahead(sp)) continue;
-        if ((rc = dalloc(h, &sp.mq, (size_t)MQ_SEGS * collide_seg_cap(sp.cap))) != PIC_OK ||
-            (rc = dalloc(h, &sp.mq_cnt, (size_t)MQ_SEGS * MQ_STRIDE)) != PIC_OK)
-            return fail(rc);
-        launch_fill<uint32_t>(h->st, sp.mq_cnt, MQ_SEGS * MQ_STRIDE, 0u);
-    }
     if (h->wall_on) {
         WallConst &c = h->wc;
         c.mode = P.mode == PIC_MODE_PHYSICAL ? PIC_DEV_MODE_PHYS : PIC_DEV_MODE_REF;
@@ -2091,9 +2046,6 @@ int pic_estimate_bytes(const pic_params *pp, int64_t *bytes) {
         if (s == 1 && !wall_on && P.wall == PIC_WALL_STEADY && P.mode == PIC_MODE_PHYSICAL)
             b += std::min<int64_t>(std::max<int64_t>(65536, n0 / 8), (int64_t)1 << 26) *
                  (36 + (weighted ? 4 : 0));
-        // candidate queue of collisions run ahead (counted for both species)
-        if (P.have_collisions && P.mode == PIC_MODE_PHYSICAL)
-            b += (int64_t)MQ_SEGS * collide_seg_cap(cap) * 4 + MQ_SEGS * MQ_STRIDE * 4;
     }
     const int64_t tiles = (N + 1 + 7) / 8;
     {  // sort histogram (one counter per 128-byte line) and starts

@@ -277,23 +277,22 @@ __device__ __forceinline__ uint32_t hash_insert(BlockHash &H, uint32_t key, bool
 // Variants of the particle passes.  The generic kernel takes every option at
 // run time; the others pin options that the host has checked (physical mode,
 // no magnetic field, no per-particle weights, no pair sampling in the pass;
-// then: no collisions in the pass and nothing staged (PLAIN); no collisions
-// in the pass -- none, or run ahead in k_collide -- and lost particles
-// queuing their ids for re-injection (SPAWN); or the block-queued collisions
-// of one species (COLL_E, COLL_I); or, in place, the candidate test only,
-// each candidate left untouched for k_collide_q (DEFER)), so the compiler
-// drops the code and registers of everything else (the collisionless
-// in-place pass: 42 instead of 94 VGPRs, 8 instead of 5 waves per SIMD).  A
-// pinned value always equals the one passed in, so every variant computes
-// what the generic kernel computes.
+// then: no collisions and nothing staged (PLAIN); no collisions and lost
+// particles queuing their ids for re-injection (SPAWN); or the block-queued
+// collisions of one species (COLL_E, COLL_I)), so the compiler drops the code
+// and registers of everything else.  A pinned value always equals the one
+// passed in, so every variant computes what the generic kernel computes.
+// The argon ions (0.5 % candidates) used to leave theirs to a pass of their
+// own, to keep the collision code's registers out of the ions' pass; with the
+// products settled on the queue's lanes COLL_I takes 72 VGPRs like SPAWN, and
+// that pass (18 us at 257^2, 125 us at 1025^2) is gone.
 enum PassVariant {
     PV_GENERIC = 0,
     PV_PLAIN = 1,
     PV_COLL_E = 2,
     PV_COLL_I = 3,
     PV_SPAWN = 4,
-    PV_DEFER = 5,
-    PV_COMPACT = 6  // sort pass without a push (drops holes): the generic body, pinned
+    PV_COMPACT = 5  // sort pass without a push (drops holes): the generic body, pinned
 };
 
 template <int V>
@@ -304,9 +303,6 @@ __device__ __forceinline__ void pin_variant(PushConst &pc, mcc::MccConst &mc, Sp
     sp.w = nullptr;
     if (V == PV_PLAIN || V == PV_SPAWN || V == PV_COMPACT) {
         mc.on = 0;
-    } else if (V == PV_DEFER) {
-        mc.on = 1;
-        mc.mode = PIC_DEV_MODE_PHYS;
     } else {
         mc.on = 1;
         mc.mode = PIC_DEV_MODE_PHYS;
@@ -318,24 +314,8 @@ __device__ __forceinline__ void pin_variant(PushConst &pc, mcc::MccConst &mc, Sp
 template <int V>
 __device__ __forceinline__ void pin_spawn(Spawn &spn) {
     if (V != PV_GENERIC) spn.plop = 0;
-    if (V == PV_PLAIN || V == PV_SPAWN || V == PV_DEFER || V == PV_COMPACT) spn.wall = 0;
+    if (V == PV_PLAIN || V == PV_SPAWN || V == PV_COMPACT) spn.wall = 0;
     if (V == PV_PLAIN || V == PV_COMPACT) spn.lost_ids = 0;
-}
-
-// A deferred pass's candidates of one round: the wavefront appends the
-// store indices of its candidates to its block's queue segment (one atomic
-// per wavefront).  Called by every lane.
-__device__ __forceinline__ void defer_queue(const Spawn &spn, bool cand, uint32_t i) {
-    const uint64_t bal = __ballot(cand);
-    if (!bal) return;  // uniform over the wavefront
-    const int lane = threadIdx.x & 63, lead = __ffsll((unsigned long long)bal) - 1;
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t seg = blockIdx.x % MQ_SEGS;
-    uint32_t b = 0u;
-    if (lane == lead) b = atomicAdd(&spn.mq_cnt[seg * MQ_STRIDE], (uint32_t)__popcll(bal));
-    b = (uint32_t)__shfl((int)b, lead, 64);
-    const uint32_t t = b + (uint32_t)__popcll(bal & below);
-    if (cand && t < spn.mq_seg) spn.mq[(size_t)seg * spn.mq_seg + t] = i;
 }
 
 // a particle lost through a wall queues its id and weight for k_plop_drain
@@ -1129,10 +1109,11 @@ __device__ __forceinline__ mcc::MccConst fresh(mcc::MccConst c) {
 // lanes, everything else -- vz into the store, the event counts, the products of an ionisation -- is
 // settled by the lane that made the collision, so none of it takes code or
 // registers in the particles' rounds.  The queue holds every particle of the
-// block (5 words each): it cannot overflow.  q: free on entry and again after
+// block (5 words each): it cannot overflow.  Without VZ_IN (no energy bins, tab
+// null: the bound does not depend on the speed) only candidates' vz is read.  q: free on entry and again after
 // the next barrier.  The store's words of the block are not yet overwritten.
 #define CQ_WORDS 5
-template <int P, bool VZ_BACK>
+template <int P, bool VZ_IN, bool VZ_BACK>
 __device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)[P],
                                               float (&vy)[P], float (&vz)[P],
                                               const uint32_t (&id)[P], const SpView &sp,
@@ -1149,9 +1130,8 @@ __device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)
     uint32_t pos[P], wtot = 0;
 #pragma unroll
     for (int r = 0; r < P; r++) {
-        const bool cand =
-            live[r] && mcc::candidate(mc0, id[r], step,
-                                      vx[r] * vx[r] + vy[r] * vy[r] + vz[r] * vz[r], tab);
+        const float v2 = VZ_IN ? vx[r] * vx[r] + vy[r] * vy[r] + vz[r] * vz[r] : 0.0f;
+        const bool cand = live[r] && mcc::candidate(mc0, id[r], step, v2, tab);
         const uint64_t bal = __ballot(cand);
         pos[r] = cand ? wtot + (uint32_t)__popcll(bal & below) : 0xFFFFFFFFu;
         wtot += (uint32_t)__popcll(bal);
@@ -1163,13 +1143,14 @@ __device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)
         if (k < w) base += wcnt[k];
         total += wcnt[k];
     }
+    if (total == 0) return;  // uniform
 #pragma unroll
     for (int r = 0; r < P; r++) {
         if (pos[r] != 0xFFFFFFFFu) {
             const uint32_t t = pos[r] += base;
             q[t] = vx[r];
             q[CAP + t] = vy[r];
-            q[2 * CAP + t] = vz[r];
+            if (VZ_IN) q[2 * CAP + t] = vz[r];
             qu[3 * CAP + t] = id[r];
             qu[4 * CAP + t] = blk0 + threadIdx.x + r * 256;
         }
@@ -1177,8 +1158,8 @@ __device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)
     __syncthreads();
     for (uint32_t t = threadIdx.x; t < total; t += 256) {
         const mcc::MccConst mc = fresh(mc0);
-        float ux = q[t], uy = q[CAP + t], uz = q[2 * CAP + t];
         const uint32_t pid = qu[3 * CAP + t], i = qu[4 * CAP + t];
+        float ux = q[t], uy = q[CAP + t], uz = VZ_IN ? q[2 * CAP + t] : sp.vz[i];
         mcc::Child ch{};
         const int ev = mc.electron
                            ? mcc::collide_electron<true>(mc, ux, uy, uz, pid, step, true, ch, tab)
@@ -1380,7 +1361,7 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
         __syncthreads();
     }
     if (COLL)
-        collide_queue<IPP, true>(claim, vx, vy, vz, pid, src, blk0, E, pc, mc, step, sp, lost6, se,
+        collide_queue<IPP, true, true>(claim, vx, vy, vz, pid, src, blk0, E, pc, mc, step, sp, lost6, se,
                                  mc.bins ? sbins : nullptr, cq);
     PState s[IPP];
     bool kept[IPP];
@@ -1667,7 +1648,6 @@ __device__ __forceinline__ void push_inplace_body(
     pin_variant<V>(pc, mc, sp);
     pin_spawn<V>(spn);
     constexpr bool COLL = V == PV_COLL_E || V == PV_COLL_I;
-    constexpr bool ID = COLL || V == PV_DEFER;
     const uint32_t n = *nptr, blk0 = bid * (256 * IPP);
     // the grid covers the capacity: blocks past the live count leave at once
     // (uniformly, before any barrier); bid: this block's index in the species
@@ -1691,36 +1671,27 @@ __device__ __forceinline__ void push_inplace_body(
 #pragma unroll
         for (int r = 0; r < IPP; r++) {  // every load first
             c0[r] = pc_[tid + r * 256];
-            if (ID) pid[r] = pi[tid + r * 256];
+            if (COLL) pid[r] = pi[tid + r * 256];
             vx[r] = pu[tid + r * 256];
             vy[r] = pv[tid + r * 256];
-            if (COLL) vz[r] = pz[tid + r * 256];
+            if (V == PV_COLL_E) vz[r] = pz[tid + r * 256];
             ox[r] = px[tid + r * 256];
             oy[r] = py[tid + r * 256];
         }
     }
     // the electrons' null-collision bounds in LDS (loaded beside the state)
     __shared__ float2 sbins[MCC_BINS];
-    if (COLL && mc.bins && tid < MCC_BINS) sbins[tid] = mc.bins[tid];
-    bool live[IPP], cand[IPP];
+    if (V == PV_COLL_E && mc.bins && tid < MCC_BINS) sbins[tid] = mc.bins[tid];
+    bool live[IPP];
 #pragma unroll
     for (int r = 0; r < IPP; r++) {
         live[r] = blk0 + tid + r * 256 < n && cell_jx(c0[r]) != CELL_HOLE;
-        cand[r] = false;
     }
     __syncthreads();  // counters initialised, bounds staged
     if (COLL)
-        collide_queue<IPP, false>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step, spn, lost6, se,
-                           mc.bins ? sbins : nullptr, reinterpret_cast<float *>(lds));
-    if (V == PV_DEFER) {
-        // a candidate stays as it is for k_collide_q (a deferring species has
-        // no energy bins: its bound is global)
-#pragma unroll
-        for (int r = 0; r < IPP; r++) {
-            cand[r] = live[r] && mcc::candidate(mc, pid[r], step, 0.0f, nullptr);
-            defer_queue(spn, cand[r], blk0 + tid + r * 256);
-        }
-    }
+        collide_queue<IPP, V == PV_COLL_E, false>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step, spn, lost6, se,
+                           V == PV_COLL_E && mc.bins ? sbins : nullptr,
+                           reinterpret_cast<float *>(lds));
     PState s[IPP];
     bool dep[IPP];
     float w[IPP];
@@ -1744,8 +1715,7 @@ __device__ __forceinline__ void push_inplace_body(
             s[r] = t[g];
             w[r] = 1.0f;
             move_sel(s[r], ok[g], ex[g], ey[g], pc);
-            const bool move = live[r] && !cand[r];
-            dep[r] = move && inside_cells(s[r], pc.N);
+            dep[r] = live[r] && inside_cells(s[r], pc.N);
             if (dep[r]) {
                 // a word whose bits did not change (the cell of a particle
                 // that stayed in its cell) is not written again, and a
@@ -1756,7 +1726,7 @@ __device__ __forceinline__ void push_inplace_body(
                 py[tid + r * 256] = s[r].oy;
                 pu[tid + r * 256] = s[r].vx;
                 pv[tid + r * 256] = s[r].vy;
-            } else if (move) {
+            } else if (live[r]) {
                 pc_[tid + r * 256] = cell_pack(CELL_HOLE, CELL_HOLE);
                 const int st = classify(s[r], pc.N, pc.mode);
                 atomicAdd(&sl[st - 1], 1u);
@@ -1813,6 +1783,7 @@ __global__ void __launch_bounds__(256) k_push_inplace<PV_GENERIC>(PUSH_INPLACE_P
 // and 6 (a few spills): 7.63 and 37.0; 8 and 7 (ten): 8.05 and 37.9.
 #define INPL_WAVES_PLAIN 7
 #define INPL_WAVES_COLL 5
+#define INPL_WAVES_COLL_I 7
 template <>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
     k_push_inplace<PV_PLAIN>(PUSH_INPLACE_PARAMS) {
@@ -1826,20 +1797,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_W
                                 hist, blockIdx.x);
 }
 template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
-    k_push_inplace<PV_DEFER>(PUSH_INPLACE_PARAMS) {
-    push_inplace_body<PV_DEFER>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
-                                hist, blockIdx.x);
-}
-
-template <>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_COLL, INPL_WAVES_COLL)))
     k_push_inplace<PV_COLL_E>(PUSH_INPLACE_PARAMS) {
     push_inplace_body<PV_COLL_E>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
                                 hist, blockIdx.x);
 }
 template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_COLL, INPL_WAVES_COLL)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_COLL_I, INPL_WAVES_COLL_I)))
     k_push_inplace<PV_COLL_I>(PUSH_INPLACE_PARAMS) {
     push_inplace_body<PV_COLL_I>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
                                 hist, blockIdx.x);
@@ -1857,142 +1821,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_W
     else
         push_inplace_body<PV_PLAIN>(b.sp, b.n, E, b.pc, b.mc, step, b.q, deposit, b.spn,
                                     b.events, b.lost6, b.holes, b.hist, blockIdx.x - nba);
-}
-
-// Physical-mode null-collision MCC of one species as passes of their own,
-// ahead of the particle pass of the same step (collisions precede the push,
-// e_collisions.cpp:480-597 and ion_collisions.cpp:255-308 before
-// move_particles), for a species with few candidates (the argon ions: about
-// 0.5 %).  Keeping the collision code out of the particle pass gives that
-// pass the registers (and occupancy) of the collisionless one.  The draws
-// are the per-particle streams of collide_electron / collide_ion, so every
-// result equals the per-lane one.
-//
-// Pass 1, k_cand: every particle's candidate test from its id (one
-// Philox2x32 word; reads the cell and the id, 8 B).  A block appends its
-// candidates' store indices to one of MQ_SEGS queue segments (by block
-// index) with one atomic on that segment's counter, each counter on a
-// 128-byte line of its own: no counter takes more than 1/MQ_SEGS of the
-// blocks (atomics on one address queue behind each other: with 64 counters
-// this pass took 50 us for the C2 ions).  A segment holds every particle of
-// its blocks, so it cannot overflow.
-#define CIPP 8
-__global__ void __launch_bounds__(256)
-    k_cand(SpView sp, const uint32_t *__restrict__ nptr, mcc::MccConst mc, uint32_t step,
-           uint32_t *__restrict__ mq, uint32_t seg_cap, uint32_t *__restrict__ mq_cnt) {
-    const uint32_t n = *nptr;
-    if (blockIdx.x * (256 * CIPP) >= n) return;  // past the live count
-    __shared__ uint32_t wcnt[4], sbase;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t base = blockIdx.x * (256 * CIPP) + threadIdx.x;
-    uint32_t pos[CIPP], cl[CIPP], idv[CIPP];
-#pragma unroll
-    for (int r = 0; r < CIPP; r++) {  // every load first, none waiting on another
-        const uint32_t i = base + r * 256;
-        cl[r] = i < n ? sp.cell[i] : cell_pack(CELL_HOLE, CELL_HOLE);
-        idv[r] = i < n ? sp.id[i] : 0u;
-    }
-    uint32_t wtot = 0;
-#pragma unroll
-    for (int r = 0; r < CIPP; r++) {
-        const bool cand = cell_jx(cl[r]) != CELL_HOLE && mcc::candidate(mc, idv[r], step, 0.0f);
-        const uint64_t bal = __ballot(cand);
-        pos[r] = cand ? wtot + (uint32_t)__popcll(bal & below) : 0xFFFFFFFFu;
-        wtot += (uint32_t)__popcll(bal);
-    }
-    if (lane == 0) wcnt[w] = wtot;
-    __syncthreads();
-    uint32_t off = 0, total = 0;
-    for (int k = 0; k < 4; k++) {
-        if (k < w) off += wcnt[k];
-        total += wcnt[k];
-    }
-    const uint32_t seg = blockIdx.x % MQ_SEGS;
-    if (threadIdx.x == 0) sbase = total ? atomicAdd(&mq_cnt[seg * MQ_STRIDE], total) : 0u;
-    __syncthreads();
-    uint32_t *q = mq + (size_t)seg * seg_cap;
-#pragma unroll
-    for (int r = 0; r < CIPP; r++) {
-        const uint32_t t = sbase + off + pos[r];
-        if (pos[r] != 0xFFFFFFFFu && t < seg_cap) q[t] = base + r * 256;
-    }
-}
-
-// Pass 2, k_collide_q: the queued candidates collide on dense lanes (a
-// stride loop over each segment), their velocities read and written back by
-// store index (12 B each way).  An ionisation stages the ejected electron
-// (born at the parent's position and pushed this step) and the new ion, as
-// the particle passes do.  `defer`: the queue comes from a deferred in-place
-// pass, which left its candidates as they were: each is then also pushed,
-// stored in place or left as a hole (loss counted, lost id queued for
-// re-injection), and deposited with global atomics -- what the pass does
-// for the others.
-__global__ void __launch_bounds__(256)
-    k_collide_q(SpView sp, const float2 *__restrict__ E, PushConst pc, mcc::MccConst mc,
-                uint32_t step, Spawn spn, const uint32_t *__restrict__ mq, uint32_t seg_cap,
-                uint32_t *__restrict__ mq_cnt, unsigned long long *__restrict__ events,
-                uint32_t *__restrict__ lost6, int defer, unsigned long long *__restrict__ q,
-                uint32_t *__restrict__ holes, uint32_t *__restrict__ hist) {
-    __shared__ uint32_t se[8];
-    if (threadIdx.x < 8) se[threadIdx.x] = 0;
-    __syncthreads();
-    const uint32_t seg = blockIdx.x % MQ_SEGS, chunk = blockIdx.x / MQ_SEGS;
-    const uint32_t nch = gridDim.x / MQ_SEGS;
-    const uint32_t cnt = min(mq_cnt[seg * MQ_STRIDE], seg_cap);
-    const uint32_t *queue = mq + (size_t)seg * seg_cap;
-    for (uint32_t t = chunk * 256 + threadIdx.x; t < cnt; t += nch * 256) {
-        const uint32_t i = queue[t];
-        const uint32_t pid = sp.id[i];
-        float vx = sp.vx[i], vy = sp.vy[i], vz = sp.vz[i];
-        mcc::Child ch{};
-        const int ev = mc.electron ? mcc::collide_electron(mc, vx, vy, vz, pid, step, true, ch)
-                                   : mcc::collide_ion(mc, vx, vy, vz, pid, step);
-        if (EV_KIND(ev) > 0) atomicAdd(&se[EV_KIND(ev)], 1u);
-        if (ev & EV_OVER_BOUND) atomicAdd(&se[6], 1u);
-        const PState pre = load_state(sp, i, false);
-        const float pw = load_w(sp, i);
-        if (defer) {
-            PState s = pre;
-            s.vx = vx;
-            s.vy = vy;
-            s.vz = vz;
-            push_one(s, E, pc);
-            const int st = classify(s, pc.N, pc.mode);
-            if (st == ST_KEPT) {
-                sp.cell[i] = cell_pack(s.jx, s.jy);
-                sp.ox[i] = s.ox;
-                sp.oy[i] = s.oy;
-                if (deposit_ok(s, pc.N, pc.mode))
-                    dep_global(q, pc.N, s.jx, s.jy, fx_weights_w(s.ox, s.oy, pw));
-                // the histogram of the next sort pass, which the deferring
-                // in-place pass counted for every other particle
-                if (hist)
-                    atomicAdd(&hist[(size_t)(bin_key(s.jx, s.jy, pc.tilesX) >> pc.keyshift) *
-                                    BIN_STRIDE],
-                              1u);
-            } else {
-                sp.cell[i] = cell_pack(CELL_HOLE, CELL_HOLE);
-                atomicAdd(&lost6[cnt_slot() * 6 + st - 1], 1u);
-                atomicAdd(&holes[cnt_slot()], 1u);
-                if (spn.lost_ids && st >= ST_LEFT && st <= ST_TOP) queue_lost(spn, pid, pw);
-            }
-            vx = s.vx;
-            vy = s.vy;
-            vz = s.vz;
-        }
-        sp.vx[i] = vx;
-        sp.vy[i] = vy;
-        sp.vz[i] = vz;
-        if (EV_KIND(ev) == mcc::EV_IONIZE)
-            stage_ionisation(ch, pre, pid, E, pc, spn, lost6, pw);
-    }
-    __syncthreads();
-    if (threadIdx.x < 8 && se[threadIdx.x])
-        atomicAdd(&events[cnt_slot() * 8 + threadIdx.x], (unsigned long long)se[threadIdx.x]);
-    // one block per segment (the launches below): the segment's counter is
-    // read; clear it for the next queue
-    if (threadIdx.x == 0 && nch == 1) mq_cnt[seg * MQ_STRIDE] = 0u;
 }
 
 // Re-injection for the ions lost through a wall in the particle pass just
@@ -2663,7 +2491,6 @@ static int pass_variant(const SpView &sp, const PushConst &pc, const mcc::MccCon
         return (spn && spn->lost_ids) ? PV_SPAWN : PV_PLAIN;
     }
     if (mc.mode != PIC_DEV_MODE_PHYS) return PV_GENERIC;
-    if (spn && spn->mq) return spn->wall ? PV_GENERIC : PV_DEFER;
     return mc.electron ? PV_COLL_E : PV_COLL_I;
 }
 
@@ -2673,7 +2500,6 @@ static int pass_variant(const SpView &sp, const PushConst &pc, const mcc::MccCon
     case PV_COLL_E: hipLaunchKernelGGL(kern<PV_COLL_E>, grid, dim3(256), 0, __VA_ARGS__); break; \
     case PV_COLL_I: hipLaunchKernelGGL(kern<PV_COLL_I>, grid, dim3(256), 0, __VA_ARGS__); break; \
     case PV_SPAWN: hipLaunchKernelGGL(kern<PV_SPAWN>, grid, dim3(256), 0, __VA_ARGS__); break; \
-    case PV_DEFER: hipLaunchKernelGGL(kern<PV_DEFER>, grid, dim3(256), 0, __VA_ARGS__); break; \
     default: hipLaunchKernelGGL(kern<PV_GENERIC>, grid, dim3(256), 0, __VA_ARGS__); break;   \
     }
 
@@ -2726,32 +2552,6 @@ void launch_push_inplace_pair(hipStream_t st, const InplaceArgs &a, const Inplac
     const uint32_t nb = nba + (uint32_t)blocks_for(b.cap, 256 * IPP);
     hipLaunchKernelGGL(k_push_inplace_pair, dim3(nb), dim3(256), 0, st, a, b, nba, E, step,
                        deposit);
-}
-
-uint32_t collide_seg_cap(int64_t cap) {
-    const int64_t blocks = blocks_for(cap, 256 * CIPP);
-    return (uint32_t)((blocks + MQ_SEGS - 1) / MQ_SEGS * (256 * CIPP));
-}
-
-void launch_collide(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
-                    const float2 *E, const PushConst &pc, const mcc::MccConst &mc, uint32_t step,
-                    const Spawn &spn, unsigned long long *events, uint32_t *lost6, uint32_t *mq,
-                    uint32_t *mq_cnt) {
-    const uint32_t seg_cap = collide_seg_cap(cap);
-    // the counters are zero: set so at allocation, cleared by k_collide_q
-    hipLaunchKernelGGL(k_cand, dim3(blocks_for(cap, 256 * CIPP)), dim3(256), 0, st, sp, n, mc, step,
-                       mq, seg_cap, mq_cnt);
-    hipLaunchKernelGGL(k_collide_q, dim3(MQ_SEGS), dim3(256), 0, st, sp, E, pc, mc, step, spn,
-                       mq, seg_cap, mq_cnt, events, lost6, 0, (unsigned long long *)nullptr,
-                       (uint32_t *)nullptr, (uint32_t *)nullptr);
-}
-
-void launch_collide_deferred(hipStream_t st, const SpView &sp, const float2 *E,
-                             const PushConst &pc, const mcc::MccConst &mc, uint32_t step,
-                             const Spawn &spn, unsigned long long *events, uint32_t *lost6,
-                             unsigned long long *q, uint32_t *holes, uint32_t *hist) {
-    hipLaunchKernelGGL(k_collide_q, dim3(MQ_SEGS), dim3(256), 0, st, sp, E, pc, mc, step, spn,
-                       spn.mq, spn.mq_seg, spn.mq_cnt, events, lost6, 1, q, holes, hist);
 }
 
 void launch_plop_drain(hipStream_t st, const StageView &wq, SpCounters *cw, const Spawn &sp,

@@ -155,10 +155,6 @@ struct Spawn {
     // re-injection after the pass: a particle lost through a wall queues only
     // its id and weight in wq (k_plop_drain samples the pair)
     int lost_ids;
-    // deferred collisions (in-place pass): a candidate is queued here by
-    // store index, untouched, for k_collide_q to collide, push and deposit
-    uint32_t *mq, *mq_cnt;
-    uint32_t mq_seg;
 };
 
 // ---- k_particles.hip
@@ -198,19 +194,6 @@ struct InplaceArgs {
 bool inplace_pair_ok(const InplaceArgs &a, const InplaceArgs &b);
 void launch_push_inplace_pair(hipStream_t st, const InplaceArgs &a, const InplaceArgs &b,
                               const float2 *E, uint32_t step, int deposit);
-// candidate queue of the collisions run ahead: MQ_SEGS segments of
-// collide_seg_cap(cap) indices, one counter per segment every MQ_STRIDE words
-#define MQ_SEGS 1024
-#define MQ_STRIDE 32
-uint32_t collide_seg_cap(int64_t cap);
-void launch_collide(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
-                    const float2 *E, const PushConst &pc, const mcc::MccConst &mc, uint32_t step,
-                    const Spawn &spn, unsigned long long *events, uint32_t *lost6, uint32_t *mq,
-                    uint32_t *mq_cnt);
-void launch_collide_deferred(hipStream_t st, const SpView &sp, const float2 *E,
-                             const PushConst &pc, const mcc::MccConst &mc, uint32_t step,
-                             const Spawn &spn, unsigned long long *events, uint32_t *lost6,
-                             unsigned long long *q, uint32_t *holes, uint32_t *hist = nullptr);
 void launch_plop_drain(hipStream_t st, const StageView &wq, SpCounters *cw, const Spawn &sp,
                        const mcc::MccConst &mc, uint32_t step, int N);
 void launch_mcc(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
