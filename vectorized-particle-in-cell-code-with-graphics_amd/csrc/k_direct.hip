@@ -75,18 +75,63 @@ __device__ __forceinline__ void fft8(double2 (&v)[8]) {
 __device__ __forceinline__ int fpad(int i) { return i + (i >> 3); }
 constexpr int fft_lds(int logl) { return (1 << logl) + (1 << (logl - 3)); }  // double2 per FFT
 
+// thread t's twiddles, loaded beside the data (a load between two exchanges
+// would put the cache's latency on the chain of every pass; with the barriers
+// that fft_sync saves a 65^2 step takes 743 us for eight frames, it took 761):
+// w[p-1] of the radix-8 pass p, l[m] of butterfly m of the last pass
+template <int LOGL> struct Twid {
+    static constexpr int A = LOGL / 3, B = LOGL % 3, M = B ? 8 >> B : 0;
+    double2 w[A > 1 ? A - 1 : 1], l[M ? M : 1];
+    __device__ __forceinline__ void load(int t, const double2 *__restrict__ tw) {
+        constexpr int L = 1 << LOGL;
+#pragma unroll
+        for (int p = 1; p < A; p++) w[p - 1] = tw[(t & ((1 << (3 * p)) - 1)) * (L >> (3 * p + 3))];
+#pragma unroll
+        for (int m = 0; m < M; m++) l[m] = tw[t + L / 8 * m];
+    }
+    __device__ __forceinline__ double2 pass(int p) const { return w[p - 1]; }
+    __device__ __forceinline__ double2 last(int m) const { return l[m]; }
+};
+// the longest transform has 1024 threads and 128 registers for each: its
+// twiddles are loaded where they are used
+template <> struct Twid<13> {
+    const double2 *tw;
+    int t;
+    __device__ __forceinline__ void load(int t_, const double2 *tw_) { t = t_, tw = tw_; }
+    __device__ __forceinline__ double2 pass(int p) const {
+        return tw[(t & ((1 << (3 * p)) - 1)) << (10 - 3 * p)];
+    }
+    __device__ __forceinline__ double2 last(int m) const { return tw[t + 1024 * m]; }
+};
+
+// the threads of an FFT meet: its NT threads lie in one wavefront, whose LDS
+// operations complete in order (the compiler must keep them so), or the
+// workgroup waits
+template <bool WAVE>
+__device__ __forceinline__ void fft_sync() {
+    if (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
+
 // forward FFT of length L = 2^LOGL (Stockham, radix 8 with a last pass of 2
 // or 4), thread t of its NT = L/8 threads; buf: fft_lds(LOGL) of LDS; tw[k] =
-// exp(-2 pi i k / L).  Every thread of the workgroup calls it.
+// exp(-2 pi i k / L).  Every thread of the workgroup calls it.  For NT up to
+// 64 a wavefront holds whole FFTs and no exchange takes a barrier.
 template <int LOGL>
 __device__ __forceinline__ void fft_fwd(double2 (&v)[8], int t, double2 *buf,
-                                        const double2 *__restrict__ tw) {
+                                        const Twid<LOGL> &tw) {
     constexpr int L = 1 << LOGL, NT = L / 8, A = LOGL / 3, B = LOGL % 3;
+    constexpr bool WAVE = NT <= 64;
 #pragma unroll
     for (int p = 0; p < A; p++) {
         const int ns = 1 << (3 * p), k = t & (ns - 1);
         if (p > 0) {
-            const double2 w1 = tw[k * (L / (8 * ns))], w2 = cmul(w1, w1), w3 = cmul(w2, w1),
+            const double2 w1 = tw.pass(p), w2 = cmul(w1, w1), w3 = cmul(w2, w1),
                           w4 = cmul(w2, w2);
             v[1] = cmul(v[1], w1);
             v[2] = cmul(v[2], w2);
@@ -99,10 +144,10 @@ __device__ __forceinline__ void fft_fwd(double2 (&v)[8], int t, double2 *buf,
         fft8(v);
         if (p == A - 1 && B == 0) break;  // natural order: t + NT s
         const int base = (t - k) * 8 + k;
-        if (p > 0) __syncthreads();  // the last exchange has been read
+        if (p > 0) fft_sync<WAVE>();  // the last exchange has been read
 #pragma unroll
         for (int r = 0; r < 8; r++) buf[fpad(base + r * ns)] = v[r];
-        __syncthreads();
+        fft_sync<WAVE>();
 #pragma unroll
         for (int s = 0; s < 8; s++) v[s] = buf[fpad(t + NT * s)];
     }
@@ -110,7 +155,7 @@ __device__ __forceinline__ void fft_fwd(double2 (&v)[8], int t, double2 *buf,
         constexpr int R = 1 << B, M = 8 / R;
 #pragma unroll
         for (int m = 0; m < M; m++) {
-            const double2 w1 = tw[t + NT * m];
+            const double2 w1 = tw.last(m);
             v[m + M] = cmul(v[m + M], w1);
             if constexpr (R == 4) {
                 const double2 w2 = cmul(w1, w1);
@@ -155,10 +200,12 @@ __global__ void __launch_bounds__(FPB * (1 << LOGN) / 4)
     const int ra = 2 * ((int)blockIdx.x * FPB + f) + 1;
     const bool two = ra + 1 < n;
     double2 v[8];
+    Twid<LOGN + 1> w;
+    w.load(t, tw);
     const double *__restrict__ a = BACK ? src + (long)(ra - 1) * n - 1 : src + (long)ra * N;
     constexpr int ls = BACK ? n : N;
     load_odd<LOGN>(v, t, [&](int q) { return double2{a[q], two ? a[q + ls] : 0.0}; });
-    fft_fwd<LOGN + 1>(v, t, buf + f * fft_lds(LOGN + 1), tw);
+    fft_fwd<LOGN + 1>(v, t, buf + f * fft_lds(LOGN + 1), w);
     double *__restrict__ o = BACK ? dst + (long)ra * N : dst + (long)(ra - 1) * n - 1;
     constexpr int os = BACK ? N : n;
 #pragma unroll
@@ -192,6 +239,9 @@ __global__ void __launch_bounds__(FPB * (1 << LOGN) / 4)
     const int p = b * FPB + f;
     const bool two = 2 * p + 2 < n;
     double2 v[8];
+    Twid<LOGN + 1> w;
+    w.load(t, tw);
+    const double la = lam[2 * p + 1], lb = lam[2 * p + 2];
     double2 *__restrict__ c = reinterpret_cast<double2 *>(T) + p;
     load_odd<LOGN>(v, t, [&](int q) {
         double2 z = c[(long)(q - 1) * (n / 2)];
@@ -199,8 +249,7 @@ __global__ void __launch_bounds__(FPB * (1 << LOGN) / 4)
         return z;
     });
     double2 *bf = buf + f * fft_lds(LOGN + 1);
-    fft_fwd<LOGN + 1>(v, t, bf, tw);
-    const double la = lam[2 * p + 1], lb = lam[2 * p + 2];
+    fft_fwd<LOGN + 1>(v, t, bf, w);
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const int k = t + NT * s;
@@ -208,8 +257,8 @@ __global__ void __launch_bounds__(FPB * (1 << LOGN) / 4)
         v[s].y *= scale / (lk + la);  // the imaginary part is the first column's
         v[s].x *= scale / (lk + lb);
     }
-    __syncthreads();  // the forward transform's last exchange has been read
-    fft_fwd<LOGN + 1>(v, t, bf, tw);
+    fft_sync<NT <= 64>();  // the forward transform's last exchange has been read
+    fft_fwd<LOGN + 1>(v, t, bf, w);
 #pragma unroll
     for (int s = 0; s < 4; s++) {
         const int q = t + NT * s;
@@ -238,11 +287,20 @@ __global__ void __launch_bounds__((1 << (2 * LOGN)) / 8 < 64 ? 64 : (1 << (2 * L
     __syncthreads();
     double2 v[8];
     double2 *bf = buf + p * fft_lds(LOGN + 1);
+    Twid<LOGN + 1> w;
+    w.load(t, tw);
+    const double la = lam[2 * p + 1], lb = lam[2 * p + 2];
+    double lk[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        const int k = t + NT * s;
+        lk[s] = lam[k <= n ? k : 2 * n - k];
+    }
     auto rows = [&]() {  // the zero column and row n of X stay zero
         load_odd<LOGN>(v, t, [&](int q) {
             return double2{X[(2 * p + 1) * LD + q], X[(2 * p + 2) * LD + q]};
         });
-        fft_fwd<LOGN + 1>(v, on ? t : 0, bf, tw);
+        fft_fwd<LOGN + 1>(v, t, bf, w);
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             const int q = t + NT * s;
@@ -257,17 +315,14 @@ __global__ void __launch_bounds__((1 << (2 * LOGN)) / 8 < 64 ? 64 : (1 << (2 * L
     load_odd<LOGN>(v, t, [&](int q) {
         return double2{X[q * LD + 2 * p + 1], X[q * LD + 2 * p + 2]};
     });
-    fft_fwd<LOGN + 1>(v, t, bf, tw);
-    const double la = lam[2 * p + 1], lb = lam[2 * p + 2];
+    fft_fwd<LOGN + 1>(v, t, bf, w);
 #pragma unroll
     for (int s = 0; s < 8; s++) {
-        const int k = t + NT * s;
-        const double lk = lam[k <= n ? k : 2 * n - k];
-        v[s].y *= scale / (lk + la);
-        v[s].x *= scale / (lk + lb);
+        v[s].y *= scale / (lk[s] + la);
+        v[s].x *= scale / (lk[s] + lb);
     }
-    __syncthreads();
-    fft_fwd<LOGN + 1>(v, t, bf, tw);
+    fft_sync<true>();
+    fft_fwd<LOGN + 1>(v, t, bf, w);
 #pragma unroll
     for (int s = 0; s < 4; s++) {
         const int q = t + NT * s;
