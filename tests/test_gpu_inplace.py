@@ -1,9 +1,10 @@
-"""The in-place particle passes with pinned options against the generic pass
-(every option at run time), which a species with per-particle weights takes:
-the same run with every weight set to 1 must end in the same state, bit for
-bit, at particle counts around a block's edges, for the collisionless, the
-electrons' and the ions' collisional passes, and with more collision candidates
-than one round of a block's lanes."""
+"""The particle passes with pinned options against the generic passes (every
+option at run time), which a run with a magnetic field takes: a field too weak
+to change a bit of any velocity must end in the same state, bit for bit, at
+particle counts around a block's edges, for the collisionless, the electrons'
+and the ions' collisional passes, with and without per-particle weights,
+through in-place and sort passes, and with more collision candidates than one
+round of a block's lanes."""
 import numpy as np
 import pytest
 
@@ -15,22 +16,27 @@ pytestmark = pytest.mark.gpu
 
 def by_id(sim, s):
     d = sim.get_state(s)
+    d["w"] = sim.get_weights(s)
     o = np.argsort(d["id"])
     return {k: v[o] for k, v in d.items()}
 
 
-def run(n, gas, pressure, wall, weighted, steps=4, te=4.0):
+def run(n, gas, pressure, wall, weights, bfield=0.0, sort=16, steps=4, te=4.0,
+        emit=False):
     p = workloads.discharge(16, 4, te=te)
     p.init_particle_no = n
     if pressure:
         workloads.with_gas(p, gas, pressure)
         p.gas = gas
     p.wall = wall
-    p.sort_interval = 16
+    if emit:
+        p.e_impact_see = p.ion_impact_see = p.reflection = p.backscatter = 1
+    p.sort_interval = sort
+    p.magnetic_field, p.angle = bfield, 0.0
     with pic2d.Pic(p) as sim:
-        if weighted:
+        if weights is not None:
             for s in (0, 1):
-                sim.set_weights(s, np.ones(n, dtype=np.float32))
+                sim.set_weights(s, weights[s][sim.get_state(s)["id"]])
         sim.advance(steps)
         return ([by_id(sim, s) for s in (0, 1)], [sim.get_qfixed(s) for s in (0, 1)],
                 [sim.loss_counts(s) for s in (0, 1)], [sim.collision_counts(s) for s in (0, 1)])
@@ -48,11 +54,35 @@ def test_pinned_passes_match_the_generic_pass(n, kind):
         "dense": (pic2d.GAS_ARGON, 60000.0, pic2d.WALL_ABSORB),
     }[kind]
     print(f"in-place {kind} n={n}", flush=True)
-    a, b = (run(n, gas, pressure, wall, w) for w in (False, True))
+    compare(run(n, gas, pressure, wall, None),
+            run(n, gas, pressure, wall, [np.ones(n, dtype=np.float32)] * 2), kind, n)
+
+
+def compare(a, b, kind, n):
     for s in (0, 1):
-        for k in ("id", "cell", "ox", "oy", "vx", "vy", "vz"):
+        for k in ("id", "cell", "ox", "oy", "vx", "vy", "vz", "w"):
             assert np.array_equal(a[0][s][k], b[0][s][k]), (s, k)
         for q in (1, 2, 3):
             assert np.array_equal(a[q][s], b[q][s]), (s, q)
     if kind == "dense" and n == 5000:
         assert a[3][0].sum() > n  # a quarter of the electrons a step at least
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1025, 5000])
+@pytest.mark.parametrize("kind", ["absorb", "steady", "emit", "argon", "argon_emit", "dense"])
+@pytest.mark.parametrize("sort", [16, 2])
+def test_weighted_passes_match_the_generic_pass(n, kind, sort):
+    gas, pressure, wall, emit = {
+        "absorb": (pic2d.GAS_ARGON, 0.0, pic2d.WALL_ABSORB, False),
+        "steady": (pic2d.GAS_ARGON, 0.0, pic2d.WALL_STEADY, False),
+        "emit": (pic2d.GAS_ARGON, 0.0, pic2d.WALL_ABSORB, True),
+        "argon": (pic2d.GAS_ARGON, 66.0, pic2d.WALL_STEADY, False),
+        "argon_emit": (pic2d.GAS_ARGON, 66.0, pic2d.WALL_ABSORB, True),
+        "dense": (pic2d.GAS_ARGON, 60000.0, pic2d.WALL_ABSORB, False),
+    }[kind]
+    rng = np.random.default_rng(n)
+    w = [rng.integers(0, 9, n).astype(np.float32) / 4 for _ in range(2)]
+    print(f"weighted {kind} n={n} sort={sort}", flush=True)
+    kw = dict(sort=sort, te=40.0 if emit else 4.0, emit=emit)
+    compare(run(n, gas, pressure, wall, w, **kw), run(n, gas, pressure, wall, w, bfield=1e-30, **kw),
+            kind, n)

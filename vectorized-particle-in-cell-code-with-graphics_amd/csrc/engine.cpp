@@ -216,11 +216,15 @@ void prof_flush(pic_handle *h) {
 }
 
 // ------------------------------------------------------------ species
+// whole blocks of the particle passes: they load a block's words without
+// testing each against the count
+size_t whole_blocks(int64_t cap) {
+    return ((size_t)cap + PASS_BLOCK - 1) / PASS_BLOCK * PASS_BLOCK;
+}
+
 int species_alloc(pic_handle *h, Species &s, int64_t cap) {
     s.cap = cap;
-    // whole blocks of the particle passes: they load a block's words without
-    // testing each against the count
-    const size_t pad = ((size_t)cap + PASS_BLOCK - 1) / PASS_BLOCK * PASS_BLOCK;
+    const size_t pad = whole_blocks(cap);
     for (int b = 0; b < 2; b++) {
         CHECK(dalloc(h, &s.buf[b].cell, pad));
         CHECK(dalloc(h, &s.buf[b].ox, pad));
@@ -623,7 +627,7 @@ void update_scale(pic_handle *h, Species &s) {
 int enable_weights(pic_handle *h, Species &s) {
     if (s.weighted) return PIC_OK;
     for (int b = 0; b < 2; b++) {
-        CHECK(dalloc(h, &s.buf[b].w, (size_t)s.cap));
+        CHECK(dalloc(h, &s.buf[b].w, whole_blocks(s.cap)));
         launch_fill<float>(h->st, s.buf[b].w, (long)s.cap, (float)s.weight);
     }
     CHECK(dalloc(h, &s.stage.w, (size_t)s.stage.cap));

@@ -276,11 +276,11 @@ __device__ __forceinline__ uint32_t hash_insert(BlockHash &H, uint32_t key, bool
 
 // Variants of the particle passes.  The generic kernel takes every option at
 // run time; the others pin options that the host has checked (physical mode,
-// no magnetic field, no per-particle weights, no pair sampling in the pass;
-// then: no collisions and nothing staged (PLAIN); no collisions and lost
-// particles queuing their ids for re-injection (SPAWN); or the block-queued
-// collisions of one species (COLL_E, COLL_I)), so the compiler drops the code
-// and registers of everything else.  A pinned value always equals the one
+// no magnetic field, no pair sampling in the pass, per-particle weights with
+// PV_W and none without; then: no collisions and nothing staged (PLAIN); no
+// collisions and lost particles queuing for re-injection or the surface pass
+// (SPAWN); or the block-queued collisions of one species (COLL_E, COLL_I)),
+// so the compiler drops the code and registers of everything else.  A pinned value always equals the one
 // passed in, so every variant computes what the generic kernel computes.
 // The argon ions (0.5 % candidates) used to leave theirs to a pass of their
 // own, to keep the collision code's registers out of the ions' pass; with the
@@ -292,21 +292,26 @@ enum PassVariant {
     PV_COLL_E = 2,
     PV_COLL_I = 3,
     PV_SPAWN = 4,
-    PV_COMPACT = 5  // sort pass without a push (drops holes): the generic body, pinned
+    PV_COMPACT = 5,  // sort pass without a push (drops holes): the generic body, pinned
+    PV_W = 8         // flag on PLAIN, SPAWN, COLL_E, COLL_I: per-particle weights
 };
+constexpr int pv_base(int v) { return v & 7; }
+constexpr bool pv_weighted(int v) { return (v & PV_W) != 0; }
+constexpr bool pv_coll_e(int v) { return pv_base(v) == PV_COLL_E; }
+constexpr bool pv_coll_i(int v) { return pv_base(v) == PV_COLL_I; }
 
 template <int V>
 __device__ __forceinline__ void pin_variant(PushConst &pc, mcc::MccConst &mc, SpView &sp) {
     if (V == PV_GENERIC) return;
     pc.mode = PIC_DEV_MODE_PHYS;
     pc.bfield = 0;
-    sp.w = nullptr;
-    if (V == PV_PLAIN || V == PV_SPAWN || V == PV_COMPACT) {
+    if (!pv_weighted(V)) sp.w = nullptr;
+    if (!pv_coll_e(V) && !pv_coll_i(V)) {
         mc.on = 0;
     } else {
         mc.on = 1;
         mc.mode = PIC_DEV_MODE_PHYS;
-        mc.electron = (V == PV_COLL_E) ? 1 : 0;
+        mc.electron = pv_coll_e(V) ? 1 : 0;
     }
 }
 // no variant but the generic one samples re-injected pairs in the pass (the
@@ -314,8 +319,7 @@ __device__ __forceinline__ void pin_variant(PushConst &pc, mcc::MccConst &mc, Sp
 template <int V>
 __device__ __forceinline__ void pin_spawn(Spawn &spn) {
     if (V != PV_GENERIC) spn.plop = 0;
-    if (V == PV_PLAIN || V == PV_SPAWN || V == PV_COMPACT) spn.wall = 0;
-    if (V == PV_PLAIN || V == PV_COMPACT) spn.lost_ids = 0;
+    if (pv_base(V) == PV_PLAIN || V == PV_COMPACT) spn.wall = spn.lost_ids = 0;
 }
 
 // a particle lost through a wall queues its id and weight for k_plop_drain
@@ -1091,8 +1095,7 @@ __device__ __forceinline__ void push_scatter_body(PUSH_SCATTER_PARAMS) {
     if (threadIdx.x == 0 && shole) atomicAdd(&holes[cnt_slot()], shole);
 }
 
-// ---- the passes with pinned options (physical mode, no magnetic field, no
-// per-particle weights)
+// ---- the passes with pinned options (physical mode, no magnetic field)
 
 // A copy of the collision constants the compiler takes for new: expressions of
 // them are then evaluated where they are used.  (Hoisted out of the queue's
@@ -1173,7 +1176,7 @@ __device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)
         if (EV_KIND(ev) > 0) atomicAdd(&se[EV_KIND(ev)], 1u);
         if (ev & EV_OVER_BOUND) atomicAdd(&se[6], 1u);
         if (EV_KIND(ev) == mcc::EV_IONIZE)
-            stage_ionisation(ch, load_state(sp, i, false), pid, E, pc, spn, lost6, 1.0f);
+            stage_ionisation(ch, load_state(sp, i, false), pid, E, pc, spn, lost6, load_w(sp, i));
     }
     __syncthreads();
 #pragma unroll
@@ -1252,7 +1255,7 @@ template <int V>
 __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
     pin_variant<V>(pc, mc, src);
     pin_spawn<V>(sp);
-    constexpr bool COLL = V == PV_COLL_E || V == PV_COLL_I;
+    constexpr bool COLL = pv_coll_e(V) || pv_coll_i(V), WGT = pv_weighted(V);
     const uint32_t n = *nptr, blk0 = blockIdx.x * (256 * IPP);
     if (blk0 >= n) return;  // past the live count
     constexpr int ARENA = scat_arena_u64<V>();
@@ -1269,7 +1272,7 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
     if (tid < 6) sl[tid] = 0;
     if (tid == 0) s_total = shole = 0;
     uint32_t c0[IPP], pid[IPP];
-    float ox[IPP], oy[IPP], vx[IPP], vy[IPP], vz[IPP];
+    float ox[IPP], oy[IPP], vx[IPP], vy[IPP], vz[IPP], w[IPP];
     {
         const uint32_t *pc_ = src.cell + blk0, *pi = src.id + blk0;
         const float *px = src.ox + blk0, *py = src.oy + blk0, *pu = src.vx + blk0,
@@ -1283,6 +1286,7 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
             vz[r] = pz[tid + r * 256];
             ox[r] = px[tid + r * 256];
             oy[r] = py[tid + r * 256];
+            w[r] = WGT ? src.w[blk0 + tid + r * 256] : 1.0f;
         }
     }
     if (COLL && mc.bins && tid < MCC_BINS) sbins[tid] = mc.bins[tid];
@@ -1365,7 +1369,6 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
                                  mc.bins ? sbins : nullptr, cq);
     PState s[IPP];
     bool kept[IPP];
-    float w[IPP];
 #pragma unroll
     for (int h = 0; h < IPP; h += 2) {
         PState t[2];
@@ -1382,16 +1385,15 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
         for (int g = 0; g < 2; g++) {
             const int r = h + g;
             s[r] = t[g];
-            w[r] = 1.0f;
             move_sel(s[r], ok[g], ex[g], ey[g], pc);
             kept[r] = claim[r] && inside_cells(s[r], pc.N);
             if (claim[r] && !kept[r]) {
                 atomicAdd(&sl[classify(s[r], pc.N, pc.mode) - 1], 1u);
                 atomicAdd(&shole, 1u);
-                if (sp.lost_ids) queue_lost(sp, pid[r], 1.0f);
-                if (COLL && sp.wall)  // waits for the surface pass
+                if (sp.lost_ids) queue_lost(sp, pid[r], w[r]);
+                if (sp.wall)  // waits for the surface pass
                     stage_put(sp.wq, &sp.cw->wall_count, &sp.cw->overflow, s[r],
-                              (unsigned long long)pid[r]);
+                              (unsigned long long)pid[r], w[r]);
             }
         }
     }
@@ -1414,8 +1416,9 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
     if (direct) {
         // the claimed slots staged in slot order, SH at a time (a claimed
         // slot of a particle that left holds a hole)
-        constexpr uint32_t SH = ARENA / 4 < 256 * IPP ? ARENA / 4 : 256 * IPP;
-        uint32_t *stg = reinterpret_cast<uint32_t *>(arena);  // 8 words x SH, SoA
+        constexpr uint32_t SW = WGT ? 9 : 8;  // words of a slot, SoA
+        constexpr uint32_t SH = 2 * ARENA / SW < 256 * IPP ? 2 * ARENA / SW : 256 * IPP;
+        uint32_t *stg = reinterpret_cast<uint32_t *>(arena);
         const uint32_t tot = s_total;
         for (uint32_t lo = 0; lo < tot; lo += SH) {  // uniform: tot is the block's
 #pragma unroll
@@ -1431,6 +1434,7 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
                     stg[5 * SH + l] = __float_as_uint(s[r].vy);
                     stg[6 * SH + l] = __float_as_uint(s[r].vz);
                     stg[7 * SH + l] = pid[r];
+                    if (WGT) stg[8 * SH + l] = __float_as_uint(w[r]);
                 }
             }
             __syncthreads();
@@ -1445,6 +1449,7 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
                     dst.vy[d] = __uint_as_float(stg[5 * SH + l]);
                     dst.vz[d] = __uint_as_float(stg[6 * SH + l]);
                     dst.id[d] = stg[7 * SH + l];
+                    if (WGT) dst.w[d] = __uint_as_float(stg[8 * SH + l]);
                 }
             }
             __syncthreads();  // written out before the next part fills it
@@ -1456,6 +1461,7 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
                 PState o = s[r];
                 if (!kept[r]) o.jx = o.jy = CELL_HOLE;
                 store_state(dst, rank[r], o, pid[r]);
+                if (WGT) dst.w[rank[r]] = w[r];
             }
     }
     if (COLL && tid < 8 && se[tid])
@@ -1479,6 +1485,10 @@ SCATTER_FAST(PV_PLAIN)
 SCATTER_FAST(PV_SPAWN)
 SCATTER_FAST(PV_COLL_E)
 SCATTER_FAST(PV_COLL_I)
+SCATTER_FAST((PV_PLAIN | PV_W))
+SCATTER_FAST((PV_SPAWN | PV_W))
+SCATTER_FAST((PV_COLL_E | PV_W))
+SCATTER_FAST((PV_COLL_I | PV_W))
 
 // one particle of the generic k_push_inplace: collide (block-wide when blk), push, store
 // in place or leave a hole, count, stage products; dep = deposit it
@@ -1617,7 +1627,7 @@ __device__ __forceinline__ void push_inplace_generic(
 // sorted.
 template <int V>
 constexpr int inplace_lds_u64() {
-    return V == PV_COLL_E ? 3584 : V == PV_COLL_I ? 2560 : BLOCK_LDS_U64;
+    return pv_coll_e(V) ? 3584 : pv_coll_i(V) ? 2560 : BLOCK_LDS_U64;
 }
 
 // In-place timestep of one species between sort passes: the same collide +
@@ -1647,7 +1657,7 @@ __device__ __forceinline__ void push_inplace_body(
     uint32_t *__restrict__ holes, uint32_t *__restrict__ hist, uint32_t bid) {
     pin_variant<V>(pc, mc, sp);
     pin_spawn<V>(spn);
-    constexpr bool COLL = V == PV_COLL_E || V == PV_COLL_I;
+    constexpr bool COLL = pv_coll_e(V) || pv_coll_i(V), WGT = pv_weighted(V);
     const uint32_t n = *nptr, blk0 = bid * (256 * IPP);
     // the grid covers the capacity: blocks past the live count leave at once
     // (uniformly, before any barrier); bid: this block's index in the species
@@ -1663,7 +1673,7 @@ __device__ __forceinline__ void push_inplace_body(
     if (tid < 8) se[tid] = 0;
     if (tid == 0) shole = 0;
     uint32_t c0[IPP], pid[IPP];
-    float ox[IPP], oy[IPP], vx[IPP], vy[IPP], vz[IPP];
+    float ox[IPP], oy[IPP], vx[IPP], vy[IPP], vz[IPP], w[IPP];
     {
         const uint32_t *pc_ = sp.cell + blk0, *pi = sp.id + blk0;
         const float *px = sp.ox + blk0, *py = sp.oy + blk0, *pu = sp.vx + blk0,
@@ -1674,14 +1684,15 @@ __device__ __forceinline__ void push_inplace_body(
             if (COLL) pid[r] = pi[tid + r * 256];
             vx[r] = pu[tid + r * 256];
             vy[r] = pv[tid + r * 256];
-            if (V == PV_COLL_E) vz[r] = pz[tid + r * 256];
+            if (pv_coll_e(V)) vz[r] = pz[tid + r * 256];
             ox[r] = px[tid + r * 256];
             oy[r] = py[tid + r * 256];
+            w[r] = WGT ? sp.w[blk0 + tid + r * 256] : 1.0f;
         }
     }
     // the electrons' null-collision bounds in LDS (loaded beside the state)
     __shared__ float2 sbins[MCC_BINS];
-    if (V == PV_COLL_E && mc.bins && tid < MCC_BINS) sbins[tid] = mc.bins[tid];
+    if (pv_coll_e(V) && mc.bins && tid < MCC_BINS) sbins[tid] = mc.bins[tid];
     bool live[IPP];
 #pragma unroll
     for (int r = 0; r < IPP; r++) {
@@ -1689,12 +1700,12 @@ __device__ __forceinline__ void push_inplace_body(
     }
     __syncthreads();  // counters initialised, bounds staged
     if (COLL)
-        collide_queue<IPP, V == PV_COLL_E, false>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step, spn, lost6, se,
-                           V == PV_COLL_E && mc.bins ? sbins : nullptr,
-                           reinterpret_cast<float *>(lds));
+        collide_queue<IPP, pv_coll_e(V), false>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step,
+                                                spn, lost6, se,
+                                                pv_coll_e(V) && mc.bins ? sbins : nullptr,
+                                                reinterpret_cast<float *>(lds));
     PState s[IPP];
     bool dep[IPP];
-    float w[IPP];
     uint32_t *pc_ = sp.cell + blk0;
     float *px = sp.ox + blk0, *py = sp.oy + blk0, *pu = sp.vx + blk0, *pv = sp.vy + blk0;
 #pragma unroll
@@ -1713,7 +1724,6 @@ __device__ __forceinline__ void push_inplace_body(
         for (int g = 0; g < 2; g++) {
             const int r = h + g;
             s[r] = t[g];
-            w[r] = 1.0f;
             move_sel(s[r], ok[g], ex[g], ey[g], pc);
             dep[r] = live[r] && inside_cells(s[r], pc.N);
             if (dep[r]) {
@@ -1733,12 +1743,12 @@ __device__ __forceinline__ void push_inplace_body(
                 atomicAdd(&shole, 1u);
                 // the id and vz are read again only here
                 const uint32_t i = blk0 + tid + r * 256;
-                if (spn.lost_ids) queue_lost(spn, sp.id[i], 1.0f);
-                if (COLL && spn.wall) {  // waits for the surface pass
+                if (spn.lost_ids) queue_lost(spn, sp.id[i], w[r]);
+                if (spn.wall) {  // waits for the surface pass
                     PState post = s[r];
                     post.vz = sp.vz[i];
                     stage_put(spn.wq, &spn.cw->wall_count, &spn.cw->overflow, post,
-                              (unsigned long long)sp.id[i]);
+                              (unsigned long long)sp.id[i], w[r]);
                 }
             }
         }
@@ -1768,10 +1778,7 @@ __device__ __forceinline__ void push_inplace_body(
         Spawn spn, unsigned long long *__restrict__ events, uint32_t *__restrict__ lost6,     \
         uint32_t *__restrict__ holes, uint32_t *__restrict__ hist
 template <int V>
-__global__ void __launch_bounds__(256) k_push_inplace(PUSH_INPLACE_PARAMS) {
-    push_inplace_body<V>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes, hist,
-                         blockIdx.x);
-}
+__global__ void __launch_bounds__(256) k_push_inplace(PUSH_INPLACE_PARAMS);
 template <>
 __global__ void __launch_bounds__(256) k_push_inplace<PV_GENERIC>(PUSH_INPLACE_PARAMS) {
     push_inplace_generic(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes, hist,
@@ -1784,30 +1791,22 @@ __global__ void __launch_bounds__(256) k_push_inplace<PV_GENERIC>(PUSH_INPLACE_P
 #define INPL_WAVES_PLAIN 7
 #define INPL_WAVES_COLL 5
 #define INPL_WAVES_COLL_I 7
-template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
-    k_push_inplace<PV_PLAIN>(PUSH_INPLACE_PARAMS) {
-    push_inplace_body<PV_PLAIN>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
-                                hist, blockIdx.x);
-}
-template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
-    k_push_inplace<PV_SPAWN>(PUSH_INPLACE_PARAMS) {
-    push_inplace_body<PV_SPAWN>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
-                                hist, blockIdx.x);
-}
-template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_COLL, INPL_WAVES_COLL)))
-    k_push_inplace<PV_COLL_E>(PUSH_INPLACE_PARAMS) {
-    push_inplace_body<PV_COLL_E>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
-                                hist, blockIdx.x);
-}
-template <>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_COLL_I, INPL_WAVES_COLL_I)))
-    k_push_inplace<PV_COLL_I>(PUSH_INPLACE_PARAMS) {
-    push_inplace_body<PV_COLL_I>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes,
-                                hist, blockIdx.x);
-}
+#define INPL_WAVES_W 6  // four weights more in registers
+#define INPLACE_FAST(V, WAVES)                                                                 \
+    template <>                                                                                \
+    __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))  \
+        k_push_inplace<V>(PUSH_INPLACE_PARAMS) {                                               \
+        push_inplace_body<V>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes, \
+                             hist, blockIdx.x);                                                \
+    }
+INPLACE_FAST(PV_PLAIN, INPL_WAVES_PLAIN)
+INPLACE_FAST(PV_SPAWN, INPL_WAVES_PLAIN)
+INPLACE_FAST(PV_COLL_E, INPL_WAVES_COLL)
+INPLACE_FAST(PV_COLL_I, INPL_WAVES_COLL_I)
+INPLACE_FAST((PV_PLAIN | PV_W), INPL_WAVES_W)
+INPLACE_FAST((PV_SPAWN | PV_W), INPL_WAVES_W)
+INPLACE_FAST((PV_COLL_E | PV_W), INPL_WAVES_COLL)
+INPLACE_FAST((PV_COLL_I | PV_W), INPL_WAVES_W)
 
 // Both species' collisionless in-place passes in one launch (the first nba
 // blocks advance a, the rest b): the kernel of each species pass as it is,
@@ -2484,24 +2483,12 @@ void launch_inject(hipStream_t st, const StageView &sv, SpCounters *cnt, const f
 // the variant whose pinned options match the pass's (PV_GENERIC otherwise)
 static int pass_variant(const SpView &sp, const PushConst &pc, const mcc::MccConst &mc,
                         const Spawn *spn) {
-    if (pc.mode != PIC_DEV_MODE_PHYS || pc.bfield != 0 || sp.w != nullptr || (spn && spn->plop))
-        return PV_GENERIC;
-    if (!mc.on) {
-        if (spn && spn->wall) return PV_GENERIC;  // the wall queue takes the whole state
-        return (spn && spn->lost_ids) ? PV_SPAWN : PV_PLAIN;
-    }
+    if (pc.mode != PIC_DEV_MODE_PHYS || pc.bfield != 0 || (spn && spn->plop)) return PV_GENERIC;
+    const int w = sp.w != nullptr ? PV_W : 0;
+    if (!mc.on) return ((spn && (spn->lost_ids || spn->wall)) ? PV_SPAWN : PV_PLAIN) | w;
     if (mc.mode != PIC_DEV_MODE_PHYS) return PV_GENERIC;
-    return mc.electron ? PV_COLL_E : PV_COLL_I;
+    return (mc.electron ? PV_COLL_E : PV_COLL_I) | w;
 }
-
-#define LAUNCH_VARIANT(v, kern, grid, ...)                                                  \
-    switch (v) {                                                                           \
-    case PV_PLAIN: hipLaunchKernelGGL(kern<PV_PLAIN>, grid, dim3(256), 0, __VA_ARGS__); break; \
-    case PV_COLL_E: hipLaunchKernelGGL(kern<PV_COLL_E>, grid, dim3(256), 0, __VA_ARGS__); break; \
-    case PV_COLL_I: hipLaunchKernelGGL(kern<PV_COLL_I>, grid, dim3(256), 0, __VA_ARGS__); break; \
-    case PV_SPAWN: hipLaunchKernelGGL(kern<PV_SPAWN>, grid, dim3(256), 0, __VA_ARGS__); break; \
-    default: hipLaunchKernelGGL(kern<PV_GENERIC>, grid, dim3(256), 0, __VA_ARGS__); break;   \
-    }
 
 void launch_key_count(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
                       const PushConst &pc, uint32_t *binCount, int do_push) {
@@ -2514,8 +2501,8 @@ void launch_push_scatter(hipStream_t st, const SpView &src, const SpView &dst, c
                          uint32_t step, uint32_t *binCount, const uint32_t *binStart,
                          unsigned long long *q, int do_push, int deposit, const Spawn &spn,
                          unsigned long long *events, uint32_t *lost6, uint32_t *holes) {
-    int v = (dst.w == nullptr) ? pass_variant(src, pc, mc, &spn) : PV_GENERIC;
-    if (v != PV_GENERIC && !do_push) v = PV_COMPACT;
+    int v = pass_variant(src, pc, mc, &spn);
+    if (v != PV_GENERIC && !do_push) v = src.w ? PV_GENERIC : PV_COMPACT;
     const dim3 grid(blocks_for(cap, 256 * IPP)), blk(256);
 #define SCATTER(V)                                                                              \
     hipLaunchKernelGGL(k_push_scatter<V>, grid, blk, 0, st, src, dst, n, (uint32_t)cap, E, pc, mc, \
@@ -2525,8 +2512,12 @@ void launch_push_scatter(hipStream_t st, const SpView &src, const SpView &dst, c
     case PV_SPAWN: SCATTER(PV_SPAWN); break;
     case PV_COLL_E: SCATTER(PV_COLL_E); break;
     case PV_COLL_I: SCATTER(PV_COLL_I); break;
+    case PV_PLAIN | PV_W: SCATTER(PV_PLAIN | PV_W); break;
+    case PV_SPAWN | PV_W: SCATTER(PV_SPAWN | PV_W); break;
+    case PV_COLL_E | PV_W: SCATTER(PV_COLL_E | PV_W); break;
+    case PV_COLL_I | PV_W: SCATTER(PV_COLL_I | PV_W); break;
     case PV_COMPACT: SCATTER(PV_COMPACT); break;
-    default: SCATTER(PV_GENERIC); break;  // a sort pass defers no collisions
+    default: SCATTER(PV_GENERIC); break;
     }
 #undef SCATTER
 }
@@ -2536,9 +2527,22 @@ void launch_push_inplace(hipStream_t st, const SpView &sp, const uint32_t *n, in
                          uint32_t step, unsigned long long *q, int deposit, const Spawn &spn,
                          unsigned long long *events, uint32_t *lost6, uint32_t *holes,
                          uint32_t *hist) {
-    const int v = pass_variant(sp, pc, mc, &spn);
-    LAUNCH_VARIANT(v, k_push_inplace, dim3(blocks_for(cap, 256 * IPP)), st, sp, n, E, pc, mc, step,
-                   q, deposit, spn, events, lost6, holes, hist);
+    const dim3 grid(blocks_for(cap, 256 * IPP)), blk(256);
+#define INPLACE(V)                                                                             \
+    hipLaunchKernelGGL(k_push_inplace<V>, grid, blk, 0, st, sp, n, E, pc, mc, step, q, deposit, \
+                       spn, events, lost6, holes, hist)
+    switch (pass_variant(sp, pc, mc, &spn)) {
+    case PV_PLAIN: INPLACE(PV_PLAIN); break;
+    case PV_SPAWN: INPLACE(PV_SPAWN); break;
+    case PV_COLL_E: INPLACE(PV_COLL_E); break;
+    case PV_COLL_I: INPLACE(PV_COLL_I); break;
+    case PV_PLAIN | PV_W: INPLACE(PV_PLAIN | PV_W); break;
+    case PV_SPAWN | PV_W: INPLACE(PV_SPAWN | PV_W); break;
+    case PV_COLL_E | PV_W: INPLACE(PV_COLL_E | PV_W); break;
+    case PV_COLL_I | PV_W: INPLACE(PV_COLL_I | PV_W); break;
+    default: INPLACE(PV_GENERIC); break;
+    }
+#undef INPLACE
 }
 
 bool inplace_pair_ok(const InplaceArgs &a, const InplaceArgs &b) {
