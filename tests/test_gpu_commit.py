@@ -1,0 +1,44 @@
+"""The commit of staged particles at the counts where its sort changes form (a
+wavefront, one, two and four values a thread, the sort in memory): the first c of a
+step's injected particles do not depend on how many are injected, so each
+commit must append what the largest one appends first, in the same order."""
+import numpy as np
+import pytest
+
+import pic2d
+import workloads
+
+pytestmark = pytest.mark.gpu
+
+LARGEST = 5000
+
+
+def appended(c, species):
+    p = workloads.discharge(16, 4)
+    p.number_to_inject = c
+    with pic2d.Pic(p) as sim:
+        n = sim.particle_size(species)
+        sim.inject_particles(species)
+        d = sim.get_state(species)
+        return {k: v[n:] for k, v in d.items()}
+
+
+@pytest.fixture(scope="module")
+def largest():
+    return [appended(LARGEST, s) for s in (0, 1)]
+
+
+@pytest.mark.parametrize("c", [1, 2, 63, 64, 65, 128, 129, 1000, 1024, 1025, 2048, 2049, 4096, 4097])
+def test_commit_order(c, largest):
+    print(f"commit c={c}", flush=True)
+    for s in (0, 1):
+        d = appended(c, s)
+        assert len(d["id"]) == c and np.array_equal(np.diff(d["id"]), np.ones(c - 1))
+        for k in ("id", "cell", "ox", "oy", "vx", "vy", "vz"):
+            assert np.array_equal(d[k], largest[s][k][:c]), (s, k)
+
+
+def test_largest_commit_is_in_key_order(largest):
+    for s in (0, 1):
+        assert np.array_equal(np.diff(largest[s]["id"]), np.ones(LARGEST - 1))
+        assert len(np.unique(largest[s]["vx"])) > LARGEST // 2

@@ -494,7 +494,7 @@ bool plop_on(pic_handle *h) {
 
 // Spawn of a fused particle pass of species si.  With the physical-mode
 // steady walls the ion pass queues its ions lost through a wall in the wall
-// queue (unused by these walls otherwise) and plop_drain stages their
+// queue (unused by these walls otherwise) and the step's last commit stages their
 // re-injected pairs after the pass.
 Spawn pass_spawn(pic_handle *h, int si, int do_push) {
     Spawn sp = make_spawn(h, false, do_push ? si : -1);
@@ -504,12 +504,6 @@ Spawn pass_spawn(pic_handle *h, int si, int do_push) {
         sp.cw = &h->cnt[1];
     }
     return sp;
-}
-
-void plop_drain(pic_handle *h, int si, int do_push) {
-    if (!(do_push && si == 1 && plop_on(h))) return;
-    launch_plop_drain(h->st, h->sp[1].wq, &h->cnt[1], make_spawn(h, true, si), h->sp[1].mc,
-                      (uint32_t)h->step, h->N);
 }
 
 // the reference's steady-state walls (pairing of outside electrons and ions)
@@ -597,25 +591,30 @@ struct HistScope {
     }
 };
 
-// append species `src`'s staged particles to species `dst_s`'s current buffer
-void commit(pic_handle *h, int src, int dst_s, int deposit) {
-    drop_hist(h, dst_s);  // (not on the fused step's path: count its keys again)
-    Species &d = h->sp[dst_s];
-    launch_commit(h->st, h->sp[src].stage, &h->cnt[src], d.buf[d.cur], &h->cnt[dst_s].n[d.cur],
-                  d.cap, &h->cnt[dst_s], deposit, h->N, d.pc.mode, d.q);
+// commit of species s's staged particles to its current buffer
+CommitArgs commit_args(pic_handle *h, int s, int deposit) {
+    Species &d = h->sp[s];
+    // appended particles join the histogram of a pending sort pass
+    return CommitArgs{d.stage, &h->cnt[s], d.buf[d.cur], &h->cnt[s].n[d.cur], (uint32_t)d.cap,
+                      &h->cnt[s], deposit, d.pc.mode, d.q,
+                      d.hist_pending ? bin_count(h, s) : nullptr, d.pc.tilesX, d.pc.keyshift};
 }
 
-// commit(h, 1, 1, dep_i) and commit(h, 0, 0, dep_e) in one launch
-void commit_both(pic_handle *h, int dep_i, int dep_e) {
-    auto args = [&](int s, int dep) {
-        Species &d = h->sp[s];
-        // appended particles join the histogram of a pending sort pass
-        return CommitArgs{d.stage, &h->cnt[s], d.buf[d.cur], &h->cnt[s].n[d.cur], (uint32_t)d.cap,
-                          &h->cnt[s], dep, d.pc.mode, d.q,
-                          d.hist_pending ? bin_count(h, s) : nullptr, d.pc.tilesX,
-                          d.pc.keyshift};
-    };
-    launch_commit_pair(h->st, args(1, dep_i), args(0, dep_e), h->N);
+void commit(pic_handle *h, int s, int deposit) {
+    drop_hist(h, s);  // (not on the fused step's path: count its keys again)
+    launch_commit(h->st, commit_args(h, s, deposit), h->N);
+}
+
+// commit(h, 1, dep_i) and commit(h, 0, dep_e) in one launch; drain: with the
+// pairs re-injected for the ions lost in the ion pass just run
+void commit_both(pic_handle *h, int dep_i, int dep_e, bool drain = false) {
+    PlopArgs pl{};
+    if (drain) {
+        const Spawn sp = make_spawn(h, true, 1);
+        pl = PlopArgs{1, (uint32_t)h->step, sp.se_sigma, sp.si_sigma, h->sp[1].wq, &h->cnt[1],
+                      h->sp[1].mc};
+    }
+    launch_commit_pair(h->st, commit_args(h, 1, dep_i), commit_args(h, 0, dep_e), pl, h->N);
 }
 
 void update_scale(pic_handle *h, Species &s) {
@@ -638,21 +637,25 @@ int enable_weights(pic_handle *h, Species &s) {
     return PIC_OK;
 }
 
-// inject_more_particles (particle.cpp:491-510) into the species' staging
-// buffer; push: move and wall-test them with this step's field first
-void inject(pic_handle *h, int si, int push) {
-    Species &s = h->sp[si];
+// inject_more_particles (particle.cpp:491-510) into the staging buffers of the
+// species s0 .. s1; push_e: electrons are moved and wall-tested with this
+// step's field first
+void inject(pic_handle *h, int s0, int s1, int push_e) {
     const pic_params &P = h->P;
     if (P.number_to_inject <= 0) return;
     // particleVec() value-initialises the weight to 0 (particleVec.h:26-35):
     // the reference's injected particles carry no charge; physical mode
     // gives them weight 1
     const float w = P.mode == PIC_MODE_REF ? 0.0f : 1.0f;
-    const double vt = si == 0 ? P.vte : P.vti;
-    launch_inject(h->st, s.stage, &h->cnt[si], h->E32, s.pc, s.mc.key0, s.mc.key1,
-                  (uint32_t)h->step, (uint32_t)P.number_to_inject, w, h->dx, P.length, vt,
-                  (uint32_t)si, push, &h->cnt[si].lost[0][0]);
-    s.injected += P.number_to_inject;
+    InjectArgs a[2];
+    for (int si = s0; si <= s1; si++) {
+        Species &s = h->sp[si];
+        a[si - s0] = InjectArgs{s.stage,      &h->cnt[si], s.pc, s.mc.key0, s.mc.key1, (uint32_t)si,
+                                si == 0 && push_e, si == 0 ? P.vte : P.vti};
+        s.injected += P.number_to_inject;
+    }
+    launch_inject(h->st, a, s1 - s0 + 1, h->E32, (uint32_t)h->step, (uint32_t)P.number_to_inject, w,
+                  h->dx, P.length);
 }
 
 // contain_particle_growth (particle.cpp:640-653) on the current buffer;
@@ -798,7 +801,6 @@ void push_species(pic_handle *h, int si, int do_push, int deposit) {
     if (deposit && cold)
         launch_deposit(h->st, s.buf[1 - c], &h->cnt[si].n[1 - c], s.cap, h->N, s.pc.mode, s.q);
     prof_end(h, p3);
-    plop_drain(h, si, do_push);
     s.cur = 1 - c;
     s.holes = do_push != 0;
     s.since_sort = 0;
@@ -820,7 +822,6 @@ void push_species_inplace(pic_handle *h, int si) {
                         hist ? bin_count(h, si) : nullptr);
     s.hist_pending = hist;
     prof_end(h, p);
-    plop_drain(h, si, 1);
     s.holes = true;
     s.since_sort++;
 }
@@ -1099,8 +1100,7 @@ int fused_step(pic_handle *h) {
     }
     // particle source after the electron collisions, before the gather
     // (pic.cpp:1071-1082): electrons are staged already moved, ions unmoved
-    inject(h, 0, 1);
-    inject(h, 1, 0);
+    inject(h, 0, 1, 1);
     const bool ions_move = h->step % h->P.dt_dti == 0;
     if (!(ions_move && push_pair_inplace(h))) {
         advance_species(h, 0);
@@ -1123,7 +1123,7 @@ int fused_step(pic_handle *h) {
     }
     if (h->spawning && (plop_on(h) || h->wall_on)) {
         // pairs re-injected for ions lost this step; ion-impact secondaries
-        commit_both(h, 1, 1);
+        commit_both(h, 1, 1, ions_move && plop_on(h));
     }
     if (ref_steady(h)) steady_boundary(h);
     // pic.cpp:1130-1141: electrons, then ions, before the charge is used
@@ -1976,8 +1976,8 @@ int pic_inject_particles(pic_handle *h, int32_t s) {
     CHECK(check_species(h, s));
     if (h->P.number_to_inject <= 0) return PIC_OK;
     compact_species(h, s);
-    inject(h, s, 0);
-    commit(h, s, s, 0);
+    inject(h, s, s, 0);
+    commit(h, s, 0);
     h->sp[s].since_sort = 1 << 20;  // appended unsorted: the next pass sorts
     return PIC_OK;
 }

@@ -315,14 +315,14 @@ __device__ __forceinline__ void pin_variant(PushConst &pc, mcc::MccConst &mc, Sp
     }
 }
 // no variant but the generic one samples re-injected pairs in the pass (the
-// fused step queues lost ions for k_plop_drain); PLAIN stages nothing at all
+// fused step queues lost ions for the commit); PLAIN stages nothing at all
 template <int V>
 __device__ __forceinline__ void pin_spawn(Spawn &spn) {
     if (V != PV_GENERIC) spn.plop = 0;
     if (pv_base(V) == PV_PLAIN || V == PV_COMPACT) spn.wall = spn.lost_ids = 0;
 }
 
-// a particle lost through a wall queues its id and weight for k_plop_drain
+// a particle lost through a wall queues its id and weight for the commit
 __device__ __forceinline__ void queue_lost(const Spawn &spn, uint32_t id, float w) {
     const uint32_t slot = atomicAdd(&spn.cw->wall_count, 1u);
     if (slot >= spn.wq.cap) {
@@ -1822,33 +1822,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_W
                                     b.events, b.lost6, b.holes, b.hist, blockIdx.x - nba);
 }
 
-// Re-injection for the ions lost through a wall in the particle pass just
-// run (physical mode, steady walls): the pass queued each such ion (key = id,
-// with its weight) in the wall queue, which these walls do not otherwise
-// use, and here every queued ion stages the electron-ion pair drawn from its
-// own stream (mcc::plop_pair), keyed (1 << 32 | id), with its weight -- what
-// the pass itself staged before.  The pair sampler (three Philox blocks, six
-// logs and cosines) then stays out of the pass and its registers.  One
-// workgroup: a step loses few ions.  The queue is left empty.
-__global__ void __launch_bounds__(1024)
-    k_plop_drain(StageView wq, SpCounters *__restrict__ cw, Spawn sp, mcc::MccConst mc,
-                 uint32_t step, int N) {
-    uint32_t n = cw->wall_count;
-    if (n > wq.cap) n = wq.cap;
-    for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) {
-        const uint32_t pid = (uint32_t)wq.key[e];
-        const float w = wq.w ? wq.w[e] : 1.0f;
-        PState pe, pi;
-        mcc::plop_pair(mc, pid, step, N, sp.se_sigma, sp.si_sigma, sp.plop_ref, pe, pi);
-        const unsigned long long k = (1ull << 32) | pid;
-        // the re-injected pair replaces the lost ion: it carries its weight
-        stage_put(sp.se, &sp.ce->stage_count, &sp.ce->overflow, pe, k, w);
-        stage_put(sp.si, &sp.ci->stage_count, &sp.ci->overflow, pi, k, w);
-    }
-    __syncthreads();  // every thread has read the count
-    if (threadIdx.x == 0) cw->wall_count = 0;
-}
-
 // ------------------------------------------------------- per-phase path
 __global__ void __launch_bounds__(256)
     k_gather(SpView sp, const uint32_t *__restrict__ nptr, const float2 *__restrict__ E,
@@ -2039,49 +2012,111 @@ __global__ void __launch_bounds__(256)
         atomicAdd(&lost6[cnt_slot() * 6 + threadIdx.x], sl[threadIdx.x]);
 }
 
-// Sort (key, val) pairs [0, c) ascending by key in one workgroup: bitonic
-// network over the next power of two, padded with ~0 keys (the arrays hold
-// at least that many entries: the staging capacity is a power of two).
-#define SORT_LDS 4096  // pairs sorted in LDS (48 KB); larger batches sort in place
+// ---- commit of the staged particles
+// v of the lane J away (a power of two below 64; every lane is active)
+template <int J>
+__device__ __forceinline__ unsigned long long lane_xor(unsigned long long v) {
+    int lo = (int)(uint32_t)v, hi = (int)(uint32_t)(v >> 32);
+#define DPP2(ctrl)                                               \
+    lo = __builtin_amdgcn_mov_dpp(lo, ctrl, 0xF, 0xF, true);     \
+    hi = __builtin_amdgcn_mov_dpp(hi, ctrl, 0xF, 0xF, true)
+    if (J == 1) {
+        DPP2(0xB1);  // quad_perm 1 0 3 2
+    } else if (J == 2) {
+        DPP2(0x4E);  // quad_perm 2 3 0 1
+    } else if (J == 4) {
+        DPP2(0x141);  // row_half_mirror: lane ^ 7
+        DPP2(0x1B);   // quad_perm 3 2 1 0: lane ^ 3
+    } else if (J == 8) {
+        DPP2(0x128);  // row_ror 8
+    } else {
+        return __shfl_xor(v, J, 64);
+    }
+#undef DPP2
+    return (unsigned long long)(uint32_t)hi << 32 | (uint32_t)lo;
+}
+
+// one step of a bitonic network between lanes: the lower element keeps the
+// smaller key where `up`
+template <int J>
+__device__ __forceinline__ void lane_step(unsigned long long &v, bool up) {
+    const unsigned long long o = lane_xor<J>(v);
+    const bool low = (threadIdx.x & J) == 0;
+    v = (low == up) == (o < v) ? o : v;
+}
+template <int J>
+__device__ __forceinline__ void lane_merge(unsigned long long &v, bool up) {
+    lane_step<J>(v, up);
+    if constexpr (J > 1) lane_merge<J / 2>(v, up);
+}
+template <int K>
+__device__ __forceinline__ void lane_sort(unsigned long long &v) {
+    if constexpr (K > 2) lane_sort<K / 2>(v);
+    lane_merge<K / 2>(v, (threadIdx.x & K) == 0);
+}
+
+// Sort the P <= 1024 M values (a power of two, at least 64; distinct but for
+// padding) ascending, thread t of 1024 holding values t + 1024 m: a bitonic
+// network whose steps below 64 are lane exchanges, between 64 and 512 LDS
+// exchanges (x: P words) and from 1024 on in registers.
+template <int M>
+__device__ __forceinline__ void block_sort_regs(unsigned long long (&v)[M], uint32_t P,
+                                                unsigned long long *x) {
+    const uint32_t t = threadIdx.x;
+    const bool on = (t & ~63u) < P;  // whole waves
+    if (on)
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            lane_sort<32>(v[m]);
+            lane_merge<32>(v[m], (t & 64u) == 0);
+        }
+    for (uint32_t k = 128; k <= P; k <<= 1) {
+#pragma unroll
+        for (uint32_t j = 512u * M; j >= 1024; j >>= 1) {
+            if (j >= k) continue;
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                const int o = m ^ (int)(j >> 10);
+                if (o < M && o > m) {
+                    const bool up = ((t + 1024u * m) & k) == 0;
+                    const unsigned long long a = v[m], b = v[o];
+                    v[m] = (a < b) == up ? a : b;
+                    v[o] = (a < b) == up ? b : a;
+                }
+            }
+        }
+        for (uint32_t j = min(k >> 1, 512u); j >= 64; j >>= 1) {
+            if (on)
+#pragma unroll
+                for (int m = 0; m < M; m++) x[t + 1024 * m] = v[m];
+            __syncthreads();
+            if (on)
+#pragma unroll
+                for (int m = 0; m < M; m++) {
+                    const unsigned long long o = x[(t + 1024 * m) ^ j];
+                    const bool up = ((t + 1024u * m) & k) == 0;
+                    v[m] = ((t & j) == 0) == up ? (o < v[m] ? o : v[m]) : (o < v[m] ? v[m] : o);
+                }
+            __syncthreads();
+        }
+        if (on)
+#pragma unroll
+            for (int m = 0; m < M; m++) lane_merge<32>(v[m], ((t + 1024u * m) & k) == 0);
+    }
+}
+
+// Sort (key, val) pairs [0, c) ascending by key in one workgroup, in place: the
+// same network over the next power of two, padded with ~0 keys (the arrays
+// hold at least that many entries: the staging capacity is a power of two).
 __device__ void block_sort_pairs(unsigned long long *key, uint32_t *val, uint32_t c) {
     uint32_t P = 1;
     while (P < c) P <<= 1;
-    if (P <= SORT_LDS) {
-        // the same network on an LDS copy: no global round trip per stage
-        __shared__ unsigned long long sk[SORT_LDS];
-        __shared__ uint32_t sv[SORT_LDS];
-        for (uint32_t t = threadIdx.x; t < P; t += blockDim.x) {
-            sk[t] = t < c ? key[t] : ~0ull;
-            sv[t] = t < c ? val[t] : 0u;
-        }
-        __syncthreads();
-        for (uint32_t k = 2; k <= P; k <<= 1) {
-            for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-                for (uint32_t t = threadIdx.x; t < P; t += blockDim.x) {
-                    uint32_t o = t ^ j;
-                    if (o > t) {
-                        unsigned long long a = sk[t], b = sk[o];
-                        bool up = (t & k) == 0;
-                        if ((a > b) == up) {
-                            sk[t] = b;
-                            sk[o] = a;
-                            uint32_t x = sv[t];
-                            sv[t] = sv[o];
-                            sv[o] = x;
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-        }
-        for (uint32_t t = threadIdx.x; t < c; t += blockDim.x) {
-            key[t] = sk[t];
-            val[t] = sv[t];
-        }
-        __syncthreads();
-        return;
+    for (uint32_t t = threadIdx.x; t < P; t += blockDim.x) {
+        if (t < c)
+            val[t] = t;
+        else
+            key[t] = ~0ull;
     }
-    for (uint32_t t = c + threadIdx.x; t < P; t += blockDim.x) key[t] = ~0ull;
     __syncthreads();
     for (uint32_t k = 2; k <= P; k <<= 1) {
         for (uint32_t j = k >> 1; j > 0; j >>= 1) {
@@ -2104,96 +2139,161 @@ __device__ void block_sort_pairs(unsigned long long *key, uint32_t *val, uint32_
     }
 }
 
-// Commit the staged particles of one species: bitonic sort of (key, index)
-// in one workgroup, then append in key order to dst with consecutive new
-// ids, optionally depositing their charge.  Sorting makes the result
-// independent of the order in which the staging atomics fired.
-__device__ __forceinline__ void commit_body(StageView sv, SpCounters *__restrict__ scnt, SpView dst,
-                                            uint32_t *__restrict__ n_dst, uint32_t cap_dst,
-                                            SpCounters *__restrict__ dcnt, int deposit, int N,
-                                            int mode, unsigned long long *__restrict__ q,
-                                            uint32_t *__restrict__ hist = nullptr,
-                                            int tilesX = 0, int keyshift = 0) {
-    __shared__ uint32_t s_c, s_base, s_nid;
-    if (threadIdx.x == 0) {
-        uint32_t c = scnt->stage_count;
-        s_c = c < sv.cap ? c : sv.cap;
-        s_base = *n_dst;
-        s_nid = dcnt->next_id;
+// The staged entry k (key kk) of rank r: given its id and, unless it was
+// staged as CELL_DEAD (it takes an id but is not stored), the next slot.
+// Every thread of the workgroup calls it; `stored` counts the slots taken.
+__device__ __forceinline__ void commit_entry(const CommitArgs &a, int N, bool in, uint32_t r,
+                                             uint32_t k, unsigned long long kk, uint32_t base,
+                                             uint32_t nid, uint32_t &stored) {
+    PState p{};
+    float w = 1.0f;
+    bool live = false;
+    if (in) {
+        const uint32_t cc = a.sv.cell[k];
+        p = PState{cell_jx(cc), cell_jy(cc), a.sv.ox[k], a.sv.oy[k],
+                   a.sv.vx[k],  a.sv.vy[k],  a.sv.vz[k]};
+        if (a.sv.w) w = a.sv.w[k];
+        live = cc != cell_pack(CELL_DEAD, CELL_DEAD);
     }
-    __syncthreads();
-    const uint32_t c = s_c;
-    if (c == 0) return;
-    for (uint32_t t = threadIdx.x; t < c; t += blockDim.x) sv.idx[t] = t;
-    __syncthreads();
-    block_sort_pairs(sv.key, sv.idx, c);
-    // entries staged as CELL_DEAD take an id but are not stored: exclusive
-    // scan of the stored flags gives each stored entry its slot
-    __shared__ uint32_t chunk_total;
-    const uint32_t base = s_base, nid = s_nid;
-    const uint32_t dead = cell_pack(CELL_DEAD, CELL_DEAD);
-    uint32_t stored_before = 0;
-    for (uint32_t r0 = 0; r0 < c; r0 += blockDim.x) {
-        uint32_t r = r0 + threadIdx.x;
-        bool live = r < c && sv.cell[sv.idx[r]] != dead;
-        uint32_t tot;
-        uint32_t ex = block_excl_scan_1024(live ? 1u : 0u, &tot);
-        if (threadIdx.x == 0) chunk_total = tot;
-        __syncthreads();
-        if (live) {
-            uint32_t k = sv.idx[r];
-            uint32_t slot = base + stored_before + ex;
-            if (slot < cap_dst) {
-                PState p;
-                uint32_t cc = sv.cell[k];
-                p.jx = cell_jx(cc);
-                p.jy = cell_jy(cc);
-                p.ox = sv.ox[k];
-                p.oy = sv.oy[k];
-                p.vx = sv.vx[k];
-                p.vy = sv.vy[k];
-                p.vz = sv.vz[k];
-                // reflected and backscattered particles (sources 4, 5) keep their id
-                const unsigned long long kk = sv.key[r];
-                const uint32_t src = (uint32_t)(kk >> 32);
-                store_state(dst, slot, p, (src == 4u || src == 5u) ? (uint32_t)kk : nid + r);
-                const float w = sv.w ? sv.w[k] : 1.0f;
-                if (dst.w) dst.w[slot] = w;
-                if (deposit && deposit_ok(p, N, mode))
-                    dep_global(q, N, p.jx, p.jy, fx_weights_w(p.ox, p.oy, w));
-                // the store's histogram for a pending sort pass counts it too
-                if (hist)
-                    atomicAdd(&hist[(size_t)(bin_key(p.jx, p.jy, tilesX) >> keyshift) * BIN_STRIDE],
-                              1u);
-            }
+    uint32_t tot;
+    const uint32_t slot = base + stored + block_excl_scan_1024(live ? 1u : 0u, &tot);
+    stored += tot;
+    if (!live || slot >= a.cap_dst) return;
+    // reflected and backscattered particles (sources 4, 5) keep their id
+    const uint32_t src = (uint32_t)(kk >> 32);
+    store_state(a.dst, slot, p, (src == 4u || src == 5u) ? (uint32_t)kk : nid + r);
+    if (a.dst.w) a.dst.w[slot] = w;
+    if (a.deposit && deposit_ok(p, N, a.mode))
+        dep_global(a.q, N, p.jx, p.jy, fx_weights_w(p.ox, p.oy, w));
+    // the store's histogram for a pending sort pass counts it too
+    if (a.hist)
+        atomicAdd(&a.hist[(size_t)(bin_key(p.jx, p.jy, a.tilesX) >> a.keyshift) * BIN_STRIDE], 1u);
+}
+
+// c <= 1024 M staged entries: sorted by (key, place in the stage) packed in
+// one word (sources stay below 2^8, so a key has at most 40 bits, a place 12)
+template <int M>
+__device__ __forceinline__ uint32_t commit_regs(const CommitArgs &a, int N, uint32_t c,
+                                                uint32_t loaded, unsigned long long first,
+                                                uint32_t base, uint32_t nid,
+                                                unsigned long long *x) {
+    const uint32_t t = threadIdx.x;
+    uint32_t P = M == 1 ? 64u : 1024u * M;
+    while (P < c) P <<= 1;
+    unsigned long long v[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+        const uint32_t e = t + 1024u * m;
+        v[m] = e < c ? (m == 0 && e < loaded ? first : a.sv.key[e]) << 12 | e : ~0ull;
+    }
+    block_sort_regs<M>(v, P, x);
+    uint32_t stored = 0;
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+        const uint32_t r = t + 1024u * m;
+        if (1024u * m < c)  // uniform
+            commit_entry(a, N, r < c, r, (uint32_t)v[m] & 4095u, v[m] >> 12, base, nid, stored);
+    }
+    return stored;
+}
+
+// Commit the staged particles of one species: sort by (key, index) in one
+// workgroup, then append in key order to dst with consecutive new ids,
+// optionally depositing their charge.  Sorting makes the result independent
+// of the order in which the staging atomics fired.
+//
+// Re-injection (pl.on; physical mode, steady walls): the ion pass queued each
+// ion lost through a wall (key = id, with its weight) in the wall queue, which
+// these walls do not otherwise use; here every queued ion stages the
+// electron-ion pair drawn from its own stream (mcc::plop_pair), keyed
+// (1 << 32 | id), with its weight, each species' workgroup its own half.  The
+// pair sampler (three Philox blocks, six logs and cosines) then stays out of
+// the pass and its registers.  The second workgroup to have read the queue's
+// count empties it.
+//
+// Bound by latency: a chain of loads, the sort and the append.  Up to 4096
+// entries the sort keeps them in registers, with a barrier only for the steps
+// that cross a wavefront (12 of 55 at 1024 entries); the first keys load beside
+// the counts.  Argon at 257^2 and 1025^2, mean of a step's two commits: 9.5 and
+// 14.3 us with the re-injection, against 10.6 and 19.3 for a sort in LDS plus
+// 6.9 and 7.8 for a launch of the re-injection's own.
+__device__ __forceinline__ void commit_body(const CommitArgs &a, int N, const PlopArgs &pl,
+                                            bool electrons) {
+    __shared__ uint32_t s_raw, s_base, s_nid, s_lost;
+    __shared__ unsigned long long x[4096];
+    const uint32_t t = threadIdx.x;
+    if (t == 0) {
+        s_raw = a.scnt->stage_count;
+        s_base = *a.n_dst;
+        s_nid = a.dcnt->next_id;
+        uint32_t lost = 0;
+        if (pl.on) {
+            lost = (uint32_t)__builtin_amdgcn_readfirstlane((int)pl.cw->wall_count);
+            asm volatile("" : "+s"(lost) : : "memory");  // read before the ticket is taken
+            if (atomicAdd(&pl.cw->wall_ticket, 1u) == 1u) pl.cw->wall_count = pl.cw->wall_ticket = 0;
         }
-        stored_before += chunk_total;
-        __syncthreads();
+        s_lost = lost;
     }
-    if (threadIdx.x == 0) {
-        uint32_t room = base < cap_dst ? cap_dst - base : 0u;
-        uint32_t written = stored_before < room ? stored_before : room;
-        *n_dst = base + written;
-        dcnt->next_id = nid + c;
-        uint32_t dropped = (stored_before - written) + (scnt->stage_count - c);
-        if (dropped) dcnt->overflow += dropped;
-        scnt->stage_count = 0;
+    const unsigned long long first = t < a.sv.cap ? a.sv.key[t] : 0ull;  // while the counts load
+    __syncthreads();
+    const uint32_t raw = s_raw, base = s_base, nid = s_nid, lost = min(s_lost, pl.wq.cap);
+    if (raw + lost == 0) return;
+    for (uint32_t e = t; e < lost; e += blockDim.x) {
+        const uint32_t pid = (uint32_t)pl.wq.key[e], k = raw + e;
+        PState pe, pi;
+        mcc::plop_pair(pl.mc, pid, pl.step, N, pl.se_sigma, pl.si_sigma, 0, pe, pi);
+        if (k >= a.sv.cap) continue;
+        a.sv.cell[k] = cell_pack(pe.jx, pe.jy);
+        a.sv.ox[k] = pe.ox;
+        a.sv.oy[k] = pe.oy;
+        a.sv.vx[k] = electrons ? pe.vx : pi.vx;
+        a.sv.vy[k] = electrons ? pe.vy : pi.vy;
+        a.sv.vz[k] = electrons ? pe.vz : pi.vz;
+        a.sv.key[k] = (1ull << 32) | pid;
+        // the re-injected pair replaces the lost ion: it carries its weight
+        if (a.sv.w) a.sv.w[k] = pl.wq.w ? pl.wq.w[e] : 1.0f;
+    }
+    if (lost) __syncthreads();
+    const uint32_t c = min(raw + lost, a.sv.cap), loaded = min(raw, a.sv.cap);
+    uint32_t stored = 0;
+    if (c <= 1024) {
+        stored = commit_regs<1>(a, N, c, loaded, first, base, nid, x);
+    } else if (c <= 2048) {
+        stored = commit_regs<2>(a, N, c, loaded, first, base, nid, x);
+    } else if (c <= 4096) {
+        stored = commit_regs<4>(a, N, c, loaded, first, base, nid, x);
+    } else {
+        block_sort_pairs(a.sv.key, a.sv.idx, c);
+        for (uint32_t r0 = 0; r0 < c; r0 += blockDim.x) {
+            const uint32_t r = r0 + t;
+            const bool in = r < c;
+            commit_entry(a, N, in, r, in ? a.sv.idx[r] : 0u, in ? a.sv.key[r] : 0ull, base, nid,
+                         stored);
+        }
+    }
+    if (t == 0) {
+        const uint32_t room = base < a.cap_dst ? a.cap_dst - base : 0u;
+        const uint32_t written = stored < room ? stored : room;
+        *a.n_dst = base + written;
+        a.dcnt->next_id = nid + c;
+        // a pair that found the stage full counts like one that stage_put refused
+        const uint32_t full = raw + lost - max(raw, c);
+        const uint32_t dropped = (stored - written) + (raw + lost - c) + full;
+        if (dropped) a.dcnt->overflow += dropped;
+        a.scnt->stage_count = 0;
     }
 }
 
+__global__ void __launch_bounds__(1024) k_commit(CommitArgs a, int N) {
+    commit_body(a, N, PlopArgs{}, false);
+}
+
+// two independent commits (the ions', then the electrons': disjoint staging,
+// stores, counters and charge), workgroup b takes the b-th
 __global__ void __launch_bounds__(1024)
-    k_commit(StageView sv, SpCounters *__restrict__ scnt, SpView dst, uint32_t *__restrict__ n_dst,
-             uint32_t cap_dst, SpCounters *__restrict__ dcnt, int deposit, int N, int mode,
-             unsigned long long *__restrict__ q) {
-    commit_body(sv, scnt, dst, n_dst, cap_dst, dcnt, deposit, N, mode, q);
-}
-
-// two independent commits (different species: disjoint staging, stores,
-// counters and charge), workgroup b takes the b-th
-__global__ void __launch_bounds__(1024) k_commit_pair(CommitArgs a, CommitArgs b, int N) {
-    const CommitArgs &c = blockIdx.x == 0 ? a : b;
-    commit_body(c.sv, c.scnt, c.dst, c.n_dst, c.cap_dst, c.dcnt, c.deposit, N, c.mode, c.q, c.hist,
-                c.tilesX, c.keyshift);
+    k_commit_pair(CommitArgs a, CommitArgs b, PlopArgs pl, int N) {
+    const bool electrons = blockIdx.x != 0;
+    commit_body(electrons ? b : a, N, pl, electrons);
 }
 
 // ---------------------------------------------- reference steady-state walls
@@ -2435,13 +2535,14 @@ __device__ __forceinline__ float inject_vel(const uint32_t r[4], double vt) {
     return (float)(vt * cos(6.283185307179586 * R2) * sqrt(fabs(log(R1))));
 }
 
-__global__ void __launch_bounds__(256)
-    k_inject(StageView sv, SpCounters *__restrict__ cnt, const float2 *__restrict__ E, PushConst pc,
-             uint32_t key0, uint32_t key1, uint32_t step, uint32_t n_inj, float w, double dx,
-             double L, double vt, uint32_t species, int push, uint32_t *__restrict__ lost6) {
+// one launch for a step's source of both species (blockIdx.y)
+__global__ void __launch_bounds__(64)
+    k_inject(InjectArgs a0, InjectArgs a1, const float2 *__restrict__ E, uint32_t step,
+             uint32_t n_inj, float w, double dx, double L) {
+    const InjectArgs &A = blockIdx.y ? a1 : a0;
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n_inj) return;
-    const uint32_t s0 = species * 16u + RS_INJECT;
+    const uint32_t s0 = A.species * 16u + RS_INJECT, key0 = A.key0, key1 = A.key1;
     uint32_t a[4], b[4], c[4], d[4];
     philox4x32_10(k, step, s0, RNG_DOMAIN_MCC, key0, key1, a);
     philox4x32_10(k, step, s0 + 256u, RNG_DOMAIN_MCC, key0, key1, b);
@@ -2451,18 +2552,18 @@ __global__ void __launch_bounds__(256)
     PState s;
     inject_pos(fma(u01d(a[0], a[1]), span, dx), dx, s.jx, s.ox);
     inject_pos(fma(u01d(a[2], a[3]), span, dx), dx, s.jy, s.oy);
-    s.vx = inject_vel(b, vt);
-    s.vy = inject_vel(c, vt);
-    s.vz = inject_vel(d, vt);
+    s.vx = inject_vel(b, A.vt);
+    s.vy = inject_vel(c, A.vt);
+    s.vz = inject_vel(d, A.vt);
     int st = ST_KEPT;
-    if (push) {
-        push_one(s, E, pc);
-        st = classify(s, pc.N, pc.mode);
+    if (A.push) {
+        push_one(s, E, A.pc);
+        st = classify(s, A.pc.N, A.pc.mode);
     }
     if (st == ST_KEPT)
-        stage_put(sv, &cnt->stage_count, &cnt->overflow, s, (2ull << 32) | k, w);
+        stage_put(A.sv, &A.cnt->stage_count, &A.cnt->overflow, s, (2ull << 32) | k, w);
     else
-        atomicAdd(&lost6[cnt_slot() * 6 + st - 1], 1u);
+        atomicAdd(&A.cnt->lost[cnt_slot()][st - 1], 1u);
 }
 
 // ------------------------------------------------------------ launchers
@@ -2471,13 +2572,11 @@ static inline unsigned blocks_for(int64_t n, int t) {
     return (unsigned)(b > 0 ? b : 1);
 }
 
-void launch_inject(hipStream_t st, const StageView &sv, SpCounters *cnt, const float2 *E,
-                   const PushConst &pc, uint32_t key0, uint32_t key1, uint32_t step, uint32_t n_inj,
-                   float w, double dx, double L, double vt, uint32_t species, int push,
-                   uint32_t *lost6) {
+void launch_inject(hipStream_t st, const InjectArgs *a, int ns, const float2 *E, uint32_t step,
+                   uint32_t n_inj, float w, double dx, double L) {
     if (n_inj == 0) return;
-    hipLaunchKernelGGL(k_inject, dim3(blocks_for(n_inj, 256)), dim3(256), 0, st, sv, cnt, E, pc, key0,
-                       key1, step, n_inj, w, dx, L, vt, species, push, lost6);
+    hipLaunchKernelGGL(k_inject, dim3(blocks_for(n_inj, 64), (unsigned)ns), dim3(64), 0, st, a[0],
+                       a[ns - 1], E, step, n_inj, w, dx, L);
 }
 
 // the variant whose pinned options match the pass's (PV_GENERIC otherwise)
@@ -2558,11 +2657,6 @@ void launch_push_inplace_pair(hipStream_t st, const InplaceArgs &a, const Inplac
                        deposit);
 }
 
-void launch_plop_drain(hipStream_t st, const StageView &wq, SpCounters *cw, const Spawn &sp,
-                       const mcc::MccConst &mc, uint32_t step, int N) {
-    hipLaunchKernelGGL(k_plop_drain, dim3(1), dim3(1024), 0, st, wq, cw, sp, mc, step, N);
-}
-
 void launch_mcc(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
                 const PushConst &pc, const mcc::MccConst &mc, uint32_t step, const Spawn &spn,
                 unsigned long long *events) {
@@ -2570,15 +2664,13 @@ void launch_mcc(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap
                        spn, events);
 }
 
-void launch_commit_pair(hipStream_t st, const CommitArgs &a, const CommitArgs &b, int N) {
-    hipLaunchKernelGGL(k_commit_pair, dim3(2), dim3(1024), 0, st, a, b, N);
+void launch_commit_pair(hipStream_t st, const CommitArgs &a, const CommitArgs &b,
+                        const PlopArgs &pl, int N) {
+    hipLaunchKernelGGL(k_commit_pair, dim3(2), dim3(1024), 0, st, a, b, pl, N);
 }
 
-void launch_commit(hipStream_t st, const StageView &sv, SpCounters *scnt, const SpView &dst,
-                   uint32_t *n_dst, int64_t cap_dst, SpCounters *dcnt, int deposit, int N, int mode,
-                   unsigned long long *q) {
-    hipLaunchKernelGGL(k_commit, dim3(1), dim3(1024), 0, st, sv, scnt, dst, n_dst,
-                       (uint32_t)cap_dst, dcnt, deposit, N, mode, q);
+void launch_commit(hipStream_t st, const CommitArgs &a, int N) {
+    hipLaunchKernelGGL(k_commit, dim3(1), dim3(1024), 0, st, a, N);
 }
 
 void launch_gather(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,

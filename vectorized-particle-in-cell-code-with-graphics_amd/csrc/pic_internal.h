@@ -33,7 +33,7 @@ struct SpCounters {
     uint32_t next_id;        // id of the next particle created
     uint32_t overflow;       // particles dropped for lack of capacity
     uint32_t stage_count;    // entries in the staging buffer
-    uint32_t pad_;
+    uint32_t wall_ticket;    // readers of wall_count so far; zero between launches
     // left, right, bottom, top, removed by collision, -
     uint32_t lost[CNT_SLOTS][6];
     uint32_t holes[CNT_SLOTS];  // empty slots left by in-place steps (current buffer)
@@ -153,7 +153,7 @@ struct Spawn {
     StageView wq;
     SpCounters *cw;
     // re-injection after the pass: a particle lost through a wall queues only
-    // its id and weight in wq (k_plop_drain samples the pair)
+    // its id and weight in wq (the commit samples the pair)
     int lost_ids;
 };
 
@@ -194,8 +194,6 @@ struct InplaceArgs {
 bool inplace_pair_ok(const InplaceArgs &a, const InplaceArgs &b);
 void launch_push_inplace_pair(hipStream_t st, const InplaceArgs &a, const InplaceArgs &b,
                               const float2 *E, uint32_t step, int deposit);
-void launch_plop_drain(hipStream_t st, const StageView &wq, SpCounters *cw, const Spawn &sp,
-                       const mcc::MccConst &mc, uint32_t step, int N);
 void launch_mcc(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
                 const PushConst &pc, const mcc::MccConst &mc, uint32_t step, const Spawn &spn,
                 unsigned long long *events);
@@ -213,11 +211,21 @@ struct CommitArgs {
     uint32_t *hist;
     int tilesX, keyshift;
 };
-// both species' commits in one launch (one workgroup each)
-void launch_commit_pair(hipStream_t st, const CommitArgs &a, const CommitArgs &b, int N);
-void launch_commit(hipStream_t st, const StageView &sv, SpCounters *scnt, const SpView &dst,
-                   uint32_t *n_dst, int64_t cap_dst, SpCounters *dcnt, int deposit, int N, int mode,
-                   unsigned long long *q);
+// re-injection of the ions queued as lost in the ion pass (on: the queue of the
+// ions' counters cw is drained)
+struct PlopArgs {
+    int on;
+    uint32_t step;
+    float se_sigma, si_sigma;
+    StageView wq;
+    SpCounters *cw;
+    mcc::MccConst mc;
+};
+// both species' commits in one launch, the ions' (a) and the electrons' (b) in
+// one workgroup each
+void launch_commit_pair(hipStream_t st, const CommitArgs &a, const CommitArgs &b,
+                        const PlopArgs &pl, int N);
+void launch_commit(hipStream_t st, const CommitArgs &a, int N);
 void launch_scan(hipStream_t st, const uint32_t *count, uint32_t *start, uint32_t nbins_pad,
                  uint32_t *partial, uint32_t *n_out);
 uint32_t scan_pad(uint32_t nbins);
@@ -263,10 +271,16 @@ struct ReduceState {
 void launch_reduce(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
                    const ReduceConst &rc, ReduceState *state, SpCounters *cnt, uint32_t step,
                    unsigned long long *q, int N, int mode);
-void launch_inject(hipStream_t st, const StageView &sv, SpCounters *cnt, const float2 *E,
-                   const PushConst &pc, uint32_t key0, uint32_t key1, uint32_t step, uint32_t n_inj,
-                   float w, double dx, double L, double vt, uint32_t species, int push,
-                   uint32_t *lost6);
+struct InjectArgs {
+    StageView sv;
+    SpCounters *cnt;
+    PushConst pc;
+    uint32_t key0, key1, species;
+    int push;
+    double vt;
+};
+void launch_inject(hipStream_t st, const InjectArgs *a, int ns, const float2 *E, uint32_t step,
+                   uint32_t n_inj, float w, double dx, double L);
 
 // ---- k_wall.hip: secondary emission, reflection, backscatter (boundary.cpp:281-529, 687-756)
 struct WallConst {
