@@ -58,27 +58,30 @@ __global__ void __launch_bounds__(128)
 // Levels up to 17^2 (64 threads) are visited by the first wavefront alone,
 // without barriers.
 //
-// What bounds it: latency, a serial chain of about 6 dependent LDS round trips
-// per level visit.  Before this form (one node per thread and sweep, index
-// divisions, all five operands from LDS) a V-cycle from 65^2 took 45 us and
-// the full multigrid 170 us.
+// What bounds it: latency, per level visit some 100 instructions of one
+// wavefront and 6 dependent LDS round trips.  So the level is a template
+// argument (a thread's plane index is its own plus its block row, and every
+// LDS address that plus a constant), its nodes and right-hand side stay in
+// registers between the two legs, and the grid spacings are exact powers of
+// four apart: 9.5 us for a V-cycle from 65^2 and 35 us for the full multigrid
+// there.  With runtime levels (the index arithmetic of every visit) they took
+// 11.5 and 50 us, with one node per thread and sweep 45 and 170 us.
 #define FMG_TOP 5
 
 struct CoarseMem {
     double planes[4 * (33 * 33 + 17 * 17 + 9 * 9 + 5 * 5 + 3 * 3) + 40];
-    double res[2 * 33 * 33 + 40];             // black residuals of the visited level
+    double res[2 * 33 * 33 + 40];  // black residuals of the visited level
     double cres[33 * 33 + 17 * 17 + 9 * 9 + 5 * 5 + 3 * 3];  // V-cycle rhs, levels 0..4
     double sol[33 * 33 + 17 * 17 + 9 * 9 + 5 * 5 + 3 * 3];   // solutions, levels 0..4
     double rhs[65 * 65 + 33 * 33 + 17 * 17 + 9 * 9 + 5 * 5 + 3 * 3];  // levels 0..5
-    double h2[FMG_TOP + 1], h2i[FMG_TOP + 1];
 };
 
 // sum of (2^k + 1)^2 for k = 1 .. l-1, the start of level l's plane quartet / 4
-__device__ __forceinline__ int plane_start(int l) {
+__host__ __device__ constexpr int plane_start(int l) {
     return ((1 << (2 * l)) - 4) / 3 + 2 * ((1 << l) - 2) + (l - 1);
 }
 // sum of lvl_size(k)^2 for k < l
-__device__ __forceinline__ int flat_start(int l) { return plane_start(l + 1); }
+__host__ __device__ constexpr int flat_start(int l) { return plane_start(l + 1); }
 
 template <bool WAVE>
 __device__ __forceinline__ void level_sync() {
@@ -93,154 +96,167 @@ __device__ __forceinline__ void level_sync() {
     }
 }
 
-// thread's place on a level
-struct Blk {
-    int nb, ld, k;   // blocks per side, plane row, own plane index
-    bool on, ia, ib, ic;  // owns a block; A, B, C are inside (D always is)
-    double *pA, *pB, *pC, *pD;
+struct Node4 {
+    double a, b, c, d;
 };
-__device__ __forceinline__ Blk blk_of(CoarseMem &m, int l) {
-    Blk q;
-    q.nb = 1 << l;
-    q.ld = q.nb + 1;
-    const int t = (int)threadIdx.x, b = t >> l, c = t & (q.nb - 1);
-    q.on = b < q.nb;
-    q.k = q.on ? b * q.ld + c : 0;
-    q.ia = q.on && b > 0 && c > 0;
-    q.ib = q.on && b > 0;
-    q.ic = q.on && c > 0;
-    // 34 doubles ahead: index -1 and -ld of a wall block are never used but
+
+// a level and the thread's place on it
+template <int L>
+struct Lvl {
+    static constexpr int NB = 1 << L;       // blocks per side
+    static constexpr int LD = NB + 1;       // plane row (and row of the level below)
+    static constexpr int S = LD * LD;       // plane
+    static constexpr int N = 2 * NB + 1;    // row of a row-major array
+    static constexpr double H = 1.0 / (1 << (2 * L));  // (spacing / level 0's)^2
+    int k, o;             // place in a plane, of node A in a row-major array
+    bool on, ia, ib, ic;  // owns a block; A, B, C are inside (D always is)
+    __device__ __forceinline__ Lvl() {
+        const int t = (int)threadIdx.x;
+        on = t < NB * NB;
+        const int u = on ? t : 0, b = u >> L, c = u & (NB - 1);
+        k = u + b;
+        o = 2 * (k + (u & ~(NB - 1)));
+        ia = on && b > 0 && c > 0;
+        ib = on && b > 0;
+        ic = on && c > 0;
+    }
+    // 34 doubles ahead: index -1 and -LD of a wall block are never used but
     // stay inside the array
-    q.pA = m.planes + 34 + 4 * plane_start(l);
-    const int s = q.ld * q.ld;
-    q.pB = q.pA + s;
-    q.pC = q.pB + s;
-    q.pD = q.pC + s;
-    return q;
-}
+    __device__ __forceinline__ double *plane(CoarseMem &m, int p) const {
+        return m.planes + 34 + 4 * plane_start(L) + p * S + k;
+    }
+    __device__ __forceinline__ Node4 own4(const double *f) const {
+        return Node4{f[o], f[o + 1], f[o + N], f[o + N + 1]};
+    }
+};
 
-// own four nodes of a row-major array of level l
-__device__ __forceinline__ void own4(const double *f, int l, double &a, double &b, double &c,
-                                     double &d) {
-    const int n = lvl_size(l), t = (int)threadIdx.x, nb = 1 << l;
-    const double *p = f + (2 * (t >> l)) * n + 2 * (t & (nb - 1));
-    a = p[0];
-    b = p[1];
-    c = p[n];
-    d = p[n + 1];
-}
+struct Spacing {
+    double h2, h2i;  // level 0's squared spacing and its reciprocal
+    double length;
+};
 
-// smoothing of level l on f (zero: from a zero iterate, else from the planes),
-// the residual restricted into cres of level l - 1
-template <bool WAVE>
-__device__ __forceinline__ void coarse_pre(CoarseMem &m, int l, const double *f, bool zero) {
-    const Blk q = blk_of(m, l);
-    const double h2 = m.h2[l], h2i = m.h2i[l];
-    double fa = 0, fb = 0, fc = 0, fd = 0, a = 0, b = 0, c = 0, d = 0;
+// smoothing of level L on rhs (zero: from a zero iterate, else from the
+// planes), the thread's nodes in u, the residual restricted into cres of level
+// L - 1
+template <int L, bool WAVE>
+__device__ __forceinline__ void coarse_pre(CoarseMem &m, const Spacing &sp, const double *rhs,
+                                           Node4 &u, bool zero) {
+    constexpr int LD = Lvl<L>::LD;
+    const Lvl<L> q;
+    const double h2 = sp.h2 * Lvl<L>::H, h2i = sp.h2i * (1.0 / Lvl<L>::H);
+    double *pA = q.plane(m, 0), *pB = q.plane(m, 1), *pC = q.plane(m, 2), *pD = q.plane(m, 3);
+    double *rB = m.res + 34 + q.k, *rC = rB + Lvl<L>::S;
     double cu = 0, bl = 0, bd = 0, cr = 0;
-    const int k = q.k;
+    const Node4 f = q.own4(rhs);
+    u = Node4{0, 0, 0, 0};
+    if (!zero && q.on) {
+        u = Node4{*pA, *pB, *pC, *pD};
+        cu = pC[-LD];
+        bl = pB[-1];
+        bd = pB[LD];
+        cr = pC[1];
+    }
     if (q.on) {
-        own4(f, l, fa, fb, fc, fd);
-        if (!zero) {
-            a = q.pA[k];
-            b = q.pB[k];
-            c = q.pC[k];
-            d = q.pD[k];
-            cu = q.pC[k - q.ld];
-            bl = q.pB[k - 1];
-            bd = q.pB[k + q.ld];
-            cr = q.pC[k + 1];
-        }
         // red: south, north, east, west of A are C, C above, B, B left
-        if (q.ia) a = 0.25 * (c + cu + b + bl - h2 * fa);
-        d = 0.25 * (bd + b + cr + c - h2 * fd);
-        q.pA[k] = a;
-        q.pD[k] = d;
+        const double a = 0.25 * (u.c + cu + u.b + bl - h2 * f.a);
+        u.a = q.ia ? a : u.a;
+        u.d = 0.25 * (bd + u.b + cr + u.c - h2 * f.d);
+        *pA = u.a;
+        *pD = u.d;
     }
     level_sync<WAVE>();
     double rb = 0, rc = 0;
-    double *rB = m.res + 34, *rC = rB + q.ld * q.ld;
     if (q.on) {
-        const double du = q.pD[k - q.ld], ar = q.pA[k + 1], ad = q.pA[k + q.ld], dl = q.pD[k - 1];
-        if (q.ib) {
-            b = 0.25 * (d + du + ar + a - h2 * fb);
-            rb = -h2i * (d + du + ar + a - 4.0 * b) + fb;
-        }
-        if (q.ic) {
-            c = 0.25 * (ad + a + d + dl - h2 * fc);
-            rc = -h2i * (ad + a + d + dl - 4.0 * c) + fc;
-        }
-        q.pB[k] = b;
-        q.pC[k] = c;
-        rB[k] = rb;
-        rC[k] = rc;
+        const double du = pD[-LD], ar = pA[1], ad = pA[LD], dl = pD[-1];
+        const double sb = u.d + du + ar + u.a, sc = ad + u.a + u.d + dl;
+        const double b = 0.25 * (sb - h2 * f.b), c = 0.25 * (sc - h2 * f.c);
+        u.b = q.ib ? b : u.b;
+        u.c = q.ic ? c : u.c;
+        rb = q.ib ? -h2i * (sb - 4.0 * b) + f.b : 0.0;
+        rc = q.ic ? -h2i * (sc - 4.0 * c) + f.c : 0.0;
+        *pB = u.b;
+        *pC = u.c;
+        *rB = rb;
+        *rC = rc;
     }
     level_sync<WAVE>();
     if (q.ia) {
-        const double ra = -h2i * (c + q.pC[k - q.ld] + b + q.pB[k - 1] - 4.0 * a) + fa;
-        const int t = (int)threadIdx.x;
-        m.cres[flat_start(l - 1) + (t >> l) * q.ld + (t & (q.nb - 1))] =
-            0.5 * ra + 0.125 * (rc + rC[k - q.ld] + rb + rB[k - 1]);
+        const double ra = -h2i * (u.c + pC[-LD] + u.b + pB[-1] - 4.0 * u.a) + f.a;
+        m.cres[flat_start(L - 1) + q.k] = 0.5 * ra + 0.125 * (rc + rC[-LD] + rb + rB[-1]);
     }
     level_sync<WAVE>();
 }
 
-// prolongation of level l - 1's solution to the planes of level l: added to
-// the iterate, or (start) as the iterate
-template <bool WAVE>
-__device__ __forceinline__ void coarse_interp(CoarseMem &m, int l, bool start, double &a,
-                                              double &b, double &c, double &d, const Blk &q) {
-    const double *s = m.sol + flat_start(l - 1) + q.k;  // its rows are ld long too
-    const double c00 = s[0], c01 = s[1], c10 = s[q.ld], c11 = s[q.ld + 1];
+// prolongation of level L - 1's solution to the thread's nodes
+template <int L>
+__device__ __forceinline__ Node4 coarse_interp(CoarseMem &m, const Lvl<L> &q) {
+    constexpr int LD = Lvl<L>::LD;
+    const double *s = m.sol + flat_start(L - 1) + q.k;  // its rows are LD long too
+    const double c00 = s[0], c01 = s[1], c10 = s[LD], c11 = s[LD + 1];
     const double vc = 0.5 * (c10 + c00), vb = 0.5 * (c01 + c00);
-    const double vd = 0.5 * (0.5 * (c11 + c01) + vc);
-    if (start) {
-        a = q.ia ? c00 : 0.0;
-        b = q.ib ? vb : 0.0;
-        c = q.ic ? vc : 0.0;
-        d = vd;
-    } else {
-        a = q.ia ? q.pA[q.k] + c00 : 0.0;
-        b = q.ib ? q.pB[q.k] + vb : 0.0;
-        c = q.ic ? q.pC[q.k] + vc : 0.0;
-        d = q.pD[q.k] + vd;
-    }
+    return Node4{c00, vb, vc, 0.5 * (0.5 * (c11 + c01) + vc)};
 }
 
-// prolongation-add and smoothing of level l; the result to the planes and to
-// sol (out null) or to the row-major array out
-template <bool WAVE>
-__device__ __forceinline__ void coarse_post(CoarseMem &m, int l, const double *f, double *out) {
-    const Blk q = blk_of(m, l);
-    const double h2 = m.h2[l];
-    double fa = 0, fb = 0, fc = 0, fd = 0, a = 0, b = 0, c = 0, d = 0;
-    const int k = q.k;
+// level L's iterate from level L - 1's solution, to the planes
+template <int L>
+__device__ __forceinline__ void coarse_start(CoarseMem &m) {
+    const Lvl<L> q;
     if (q.on) {
-        own4(f, l, fa, fb, fc, fd);
-        coarse_interp<WAVE>(m, l, false, a, b, c, d, q);
-        q.pB[k] = b;
-        q.pC[k] = c;
+        const Node4 v = coarse_interp<L>(m, q);
+        *q.plane(m, 0) = q.ia ? v.a : 0.0;
+        *q.plane(m, 1) = q.ib ? v.b : 0.0;
+        *q.plane(m, 2) = q.ic ? v.c : 0.0;
+        *q.plane(m, 3) = v.d;
+    }
+    __syncthreads();
+}
+
+// prolongation-add to the nodes u and smoothing of level L; the result to the
+// planes and to sol (out null) or the row-major array out
+template <int L, bool WAVE>
+__device__ __forceinline__ void coarse_post(CoarseMem &m, const Spacing &sp, const double *rhs,
+                                            Node4 u, double *out) {
+    constexpr int LD = Lvl<L>::LD, N = Lvl<L>::N;
+    const Lvl<L> q;
+    const double h2 = sp.h2 * Lvl<L>::H;
+    double *pA = q.plane(m, 0), *pB = q.plane(m, 1), *pC = q.plane(m, 2), *pD = q.plane(m, 3);
+    const Node4 f = q.own4(rhs);
+    if (q.on) {
+        const Node4 v = coarse_interp<L>(m, q);
+        u = Node4{q.ia ? u.a + v.a : 0.0, q.ib ? u.b + v.b : 0.0, q.ic ? u.c + v.c : 0.0,
+                  u.d + v.d};
+        *pB = u.b;
+        *pC = u.c;
     }
     level_sync<WAVE>();
     if (q.on) {
-        if (q.ia) a = 0.25 * (c + q.pC[k - q.ld] + b + q.pB[k - 1] - h2 * fa);
-        d = 0.25 * (q.pB[k + q.ld] + b + q.pC[k + 1] + c - h2 * fd);
-        q.pA[k] = a;
-        q.pD[k] = d;
+        const double a = 0.25 * (u.c + pC[-LD] + u.b + pB[-1] - h2 * f.a);
+        u.a = q.ia ? a : u.a;
+        u.d = 0.25 * (pB[LD] + u.b + pC[1] + u.c - h2 * f.d);
+        *pA = u.a;
+        *pD = u.d;
     }
     level_sync<WAVE>();
     if (q.on) {
-        const double du = q.pD[k - q.ld], ar = q.pA[k + 1], ad = q.pA[k + q.ld], dl = q.pD[k - 1];
-        if (q.ib) b = 0.25 * (d + du + ar + a - h2 * fb);
-        if (q.ic) c = 0.25 * (ad + a + d + dl - h2 * fc);
-        q.pB[k] = b;
-        q.pC[k] = c;
-        const int n = lvl_size(l), t = (int)threadIdx.x;
-        double *o = (out ? out : m.sol + flat_start(l)) + (2 * (t >> l)) * n + 2 * (t & (q.nb - 1));
-        o[0] = a;
-        o[1] = b;
-        o[n] = c;
-        o[n + 1] = d;
+        const double du = pD[-LD], ar = pA[1], ad = pA[LD], dl = pD[-1];
+        const double b = 0.25 * (u.d + du + ar + u.a - h2 * f.b);
+        const double c = 0.25 * (ad + u.a + u.d + dl - h2 * f.c);
+        u.b = q.ib ? b : u.b;
+        u.c = q.ic ? c : u.c;
+        *pB = u.b;
+        *pC = u.c;
+        if (out) {
+            out[q.o] = u.a;
+            out[q.o + 1] = u.b;
+            out[q.o + N] = u.c;
+            out[q.o + N + 1] = u.d;
+        } else {
+            double *s = m.sol + flat_start(L) + q.o;
+            s[0] = u.a;
+            s[1] = u.b;
+            s[N] = u.c;
+            s[N + 1] = u.d;
+        }
     }
     level_sync<WAVE>();
 }
@@ -251,22 +267,36 @@ __device__ __forceinline__ void coarse_slvsml(CoarseMem &m, double rhs, double l
     m.sol[4] = -h * h * rhs / 4.0;
 }
 
-// one V(1,1) cycle at level j >= 1 on f (mglin.cpp:176-196)
-__device__ __forceinline__ void coarse_vcycle(CoarseMem &m, int j, const double *f, bool zero,
-                                              double length, double *out) {
-    int l = j;
-    for (; l > 3; l--) coarse_pre<false>(m, l, l == j ? f : m.cres + flat_start(l), zero || l < j);
+// one V(1,1) cycle at level j >= 1 (mglin.cpp:176-196) on rhs, from a zero
+// iterate (zero) or the planes; the levels below follow in line, those above j
+// are skipped
+__device__ __forceinline__ void coarse_vcycle(CoarseMem &m, int j, const Spacing &sp, bool zero,
+                                              double *out) {
+    Node4 u5, u4;
+#define FMG_RHS(L) ((j == L ? m.rhs : m.cres) + flat_start(L))
+#define FMG_DOWN(L, WAVE, U) \
+    if (j >= L) coarse_pre<L, WAVE>(m, sp, FMG_RHS(L), U, zero || j > L);
+#define FMG_UP(L, WAVE, U) \
+    if (j >= L) coarse_post<L, WAVE>(m, sp, FMG_RHS(L), U, j == L ? out : nullptr);
+    FMG_DOWN(5, false, u5)
+    FMG_DOWN(4, false, u4)
     if (threadIdx.x < 64) {
-        for (int w = l; w >= 1; w--)
-            coarse_pre<true>(m, w, w == j ? f : m.cres + flat_start(w), zero || w < j);
-        if (threadIdx.x == 0) coarse_slvsml(m, m.cres[4], length);
+        Node4 u3, u2, u1;
+        FMG_DOWN(3, true, u3)
+        FMG_DOWN(2, true, u2)
+        FMG_DOWN(1, true, u1)
+        if (threadIdx.x == 0) coarse_slvsml(m, m.cres[4], sp.length);
         level_sync<true>();
-        for (int w = 1; w <= l; w++)
-            coarse_post<true>(m, w, w == j ? f : m.cres + flat_start(w), w == j ? out : nullptr);
+        FMG_UP(1, true, u1)
+        FMG_UP(2, true, u2)
+        FMG_UP(3, true, u3)
     }
     __syncthreads();
-    for (l++; l <= j; l++)
-        coarse_post<false>(m, l, l == j ? f : m.cres + flat_start(l), l == j ? out : nullptr);
+    FMG_UP(4, false, u4)
+    FMG_UP(5, false, u5)
+#undef FMG_RHS
+#undef FMG_DOWN
+#undef FMG_UP
 }
 
 // full: full multigrid from rhs_in (level lc) -> u_out; else one V-cycle from
@@ -282,11 +312,10 @@ __global__ void __launch_bounds__(1024)
     for (int k = tid; k < (int)(sizeof(m.planes) / 8); k += nt) m.planes[k] = 0.0;
     for (int k = tid; k < (int)(sizeof(m.sol) / 8); k += nt) m.sol[k] = 0.0;
     for (int k = tid; k < (int)(sizeof(m.res) / 8); k += nt) m.res[k] = 0.0;
-    if (tid <= lc) {
-        const double h = length / (lvl_size(tid) - 1), h2 = h * h;
-        m.h2[tid] = h2;
-        m.h2i[tid] = 1.0 / h2;
-    }
+    // level l's spacing is 2^-l of level 0's: its square and the square's
+    // reciprocal are those of level 0 times a power of four, exactly
+    const double h0 = length / 2.0, h00 = h0 * h0;
+    const Spacing sp{h00, 1.0 / h00, length};
     // the walls of u_out; the blocks write the rest (and the first row and
     // column again)
     for (int k = tid; k < n; k += nt) u_out[k * n + n - 1] = u_out[(n - 1) * n + k] = 0.0;
@@ -296,35 +325,30 @@ __global__ void __launch_bounds__(1024)
         for (int k = tid; k < nn; k += nt) u_out[k] = k == 4 ? -h * h * top[4] / 4.0 : 0.0;
         return;
     }
-    if (!full) {
-        coarse_vcycle(m, lc, top, true, length, u_out);
-        return;
-    }
-    for (int l = lc - 1; l >= 0; l--) {
-        const int nc = lvl_size(l);
-        for (int t = tid; t < 1 << (2 * l + 2); t += nt) {  // rows and columns 1 .. nc - 2
-            const int ic = t >> (l + 1), jc = t & ((1 << (l + 1)) - 1);
-            if (ic > 0 && jc > 0)
-                m.rhs[flat_start(l) + ic * nc + jc] =
-                    rstrct_node(m.rhs + flat_start(l + 1), nc, ic, jc);
+    if (full) {
+        for (int l = lc - 1; l >= 0; l--) {
+            const int nc = lvl_size(l);
+            for (int t = tid; t < 1 << (2 * l + 2); t += nt) {  // rows and columns 1 .. nc - 2
+                const int ic = t >> (l + 1), jc = t & ((1 << (l + 1)) - 1);
+                if (ic > 0 && jc > 0)
+                    m.rhs[flat_start(l) + ic * nc + jc] =
+                        rstrct_node(m.rhs + flat_start(l + 1), nc, ic, jc);
+            }
+            __syncthreads();
         }
+        if (tid == 0) coarse_slvsml(m, m.rhs[4], length);
         __syncthreads();
     }
-    if (tid == 0) coarse_slvsml(m, m.rhs[4], length);
-    __syncthreads();
-    for (int j = 1; j <= lc; j++) {
-        const Blk q = blk_of(m, j);
-        if (q.on) {
-            double a, b, c, d;
-            coarse_interp<false>(m, j, true, a, b, c, d, q);
-            q.pA[q.k] = a;
-            q.pB[q.k] = b;
-            q.pC[q.k] = c;
-            q.pD[q.k] = d;
-        }
-        __syncthreads();
-        for (int c = 0; c < ncycle; c++)
-            coarse_vcycle(m, j, m.rhs + flat_start(j), false, length, j == lc ? u_out : nullptr);
+    for (int j = full ? 1 : lc; j <= lc; j++) {
+        if (full) switch (j) {
+            case 1: coarse_start<1>(m); break;
+            case 2: coarse_start<2>(m); break;
+            case 3: coarse_start<3>(m); break;
+            case 4: coarse_start<4>(m); break;
+            default: coarse_start<5>(m); break;
+            }
+        for (int c = 0; c < (full ? ncycle : 1); c++)
+            coarse_vcycle(m, j, sp, !full, j == lc ? u_out : nullptr);
     }
 }
 
