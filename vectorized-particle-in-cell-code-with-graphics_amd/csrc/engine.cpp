@@ -267,7 +267,7 @@ void species_free(Species &s) {
     for (void *p : st)
         if (p) hipFree(p);
     const pic::SteadyBufs &c = s.steady;
-    void *sb[] = {c.hist, c.start, c.cursor, c.id_in, c.idx_in, c.id_out, c.idx_out};
+    void *sb[] = {c.hist, c.start, c.id_in, c.idx_in, c.id_out, c.idx_out};
     for (void *p : sb)
         if (p) hipFree(p);
     s = Species();
@@ -543,7 +543,6 @@ int alloc_steady(pic_handle *h, Species &s, uint32_t nb) {
     b.nb = nb;
     CHECK(dalloc(h, &b.hist, 2 * (size_t)nb));
     CHECK(dalloc(h, &b.start, 2 * (size_t)nb + 1));
-    CHECK(dalloc(h, &b.cursor, 2 * (size_t)nb));
     if (hipMemsetAsync(b.hist, 0, sizeof(uint32_t) * 2 * nb, h->st) != hipSuccess)
         return seterr(h, PIC_ERR_DEVICE, "hipMemsetAsync failed");
     CHECK(dalloc(h, &b.id_in, (size_t)s.cap));

@@ -2342,31 +2342,40 @@ __global__ void __launch_bounds__(256) k_steady_hist(SteadyArgs a, int N, int ax
     atomicAdd(&b.hist[steady_bucket(side, a.sp[s].id[i], steady_idmax(a.cnt[s]), b.nb)], 1u);
 }
 
-// exclusive scan of a species' 2 nb bucket counts into start[0..2 nb] (and
-// the scatter cursors); the counts are cleared for the next pass
+// exclusive scan of a species' 2 nb bucket counts into start[0..2 nb].  A thread
+// takes eight buckets in a row (2 nb is a power of two, at least 32), so two
+// species of 262 144 particles (8192 buckets each) are one round: 4.0 us,
+// against 12.4 with a bucket a thread and eight rounds.
 __global__ void __launch_bounds__(1024) k_steady_scan(SteadyArgs a) {
     const SteadyBufs &b = a.b[blockIdx.x];
     const uint32_t nt = 2 * b.nb;
-    __shared__ uint32_t carry_s;
     uint32_t carry = 0;
-    for (uint32_t r0 = 0; r0 < nt; r0 += blockDim.x) {
-        const uint32_t r = r0 + threadIdx.x;
-        const uint32_t v = r < nt ? b.hist[r] : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_excl_scan_1024(v, &tot);
-        if (r < nt) {
-            b.start[r] = carry + ex;
-            b.cursor[r] = carry + ex;
-            b.hist[r] = 0u;
+    for (uint32_t r0 = 0; r0 < nt; r0 += blockDim.x * 8) {
+        const uint32_t r = r0 + threadIdx.x * 8;
+        const bool in = r < nt;
+        uint4 u{0, 0, 0, 0}, v = u;
+        if (in) {
+            const uint4 *h = reinterpret_cast<const uint4 *>(b.hist + r);
+            u = h[0];
+            v = h[1];
         }
-        if (threadIdx.x == 0) carry_s = carry + tot;
-        __syncthreads();
-        carry = carry_s;
-        __syncthreads();
+        uint32_t tot;
+        const uint32_t ex = carry + block_excl_scan_1024(u.x + u.y + u.z + u.w + v.x + v.y + v.z +
+                                                             v.w,
+                                                         &tot);
+        if (in) {
+            uint4 *o = reinterpret_cast<uint4 *>(b.start + r);
+            const uint4 p{ex, ex + u.x, ex + u.x + u.y, ex + u.x + u.y + u.z};
+            const uint32_t e = p.w + u.w;
+            o[0] = p;
+            o[1] = uint4{e, e + v.x, e + v.x + v.y, e + v.x + v.y + v.z};
+        }
+        carry += tot;
     }
     if (threadIdx.x == 0) b.start[nt] = carry;
 }
 
+// each bucket's count runs back to zero as its entries take their places
 __global__ void __launch_bounds__(256) k_steady_scatter(SteadyArgs a, int N, int axis) {
     const int s = blockIdx.y;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2375,19 +2384,18 @@ __global__ void __launch_bounds__(256) k_steady_scatter(SteadyArgs a, int N, int
     if (side < 0) return;
     const SteadyBufs &b = a.b[s];
     const uint32_t id = a.sp[s].id[i];
-    const uint32_t pos = atomicAdd(&b.cursor[steady_bucket(side, id, steady_idmax(a.cnt[s]), b.nb)], 1u);
+    const uint32_t k = steady_bucket(side, id, steady_idmax(a.cnt[s]), b.nb);
+    const uint32_t pos = b.start[k] + atomicSub(&b.hist[k], 1u) - 1u;
     b.id_in[pos] = id;
     b.idx_in[pos] = i;
 }
 
-// one workgroup per bucket: its entries in id order (ids are unique within a
-// species); up to STEADY_LDS entries by a bitonic network in LDS, larger
-// buckets by counting each entry's rank
+// The entries [lo, lo + k) of a bucket in id order (ids are unique within a
+// species), one workgroup: up to STEADY_LDS entries by a bitonic network in
+// LDS, larger buckets by counting each entry's rank
 #define STEADY_LDS 2048
-__global__ void __launch_bounds__(256) k_steady_sort(SteadyArgs a) {
-    const SteadyBufs &b = a.b[blockIdx.y];
-    const uint32_t lo = b.start[blockIdx.x], k = b.start[blockIdx.x + 1] - lo;
-    if (k == 0) return;
+__device__ __forceinline__ void steady_sort_block(const SteadyBufs &b, uint32_t lo, uint32_t k,
+                                                  uint32_t *sk, uint32_t *sv) {
     if (k > STEADY_LDS) {
         for (uint32_t j = threadIdx.x; j < k; j += blockDim.x) {
             const uint32_t v = b.id_in[lo + j];
@@ -2398,7 +2406,6 @@ __global__ void __launch_bounds__(256) k_steady_sort(SteadyArgs a) {
         }
         return;
     }
-    __shared__ uint32_t sk[STEADY_LDS], sv[STEADY_LDS];
     uint32_t P = 1;
     while (P < k) P <<= 1;
     for (uint32_t t = threadIdx.x; t < P; t += blockDim.x) {
@@ -2427,6 +2434,70 @@ __global__ void __launch_bounds__(256) k_steady_sort(SteadyArgs a) {
     for (uint32_t t = threadIdx.x; t < k; t += blockDim.x) {
         b.id_out[lo + t] = sk[t];
         b.idx_out[lo + t] = sv[t];
+    }
+    __syncthreads();  // read before the next bucket fills them
+}
+
+// up to 64 entries [lo, lo + k) in id order, one wavefront: each lane counts
+// the smaller ids
+__device__ __forceinline__ void steady_sort_wave(const SteadyBufs &b, uint32_t lo, uint32_t k) {
+    const uint32_t lane = threadIdx.x & 63;
+    const bool on = lane < k;
+    const uint32_t v = on ? b.id_in[lo + lane] : ~0u, x = on ? b.idx_in[lo + lane] : 0u;
+    uint32_t r = 0;
+    for (uint32_t t = 0; t < k; t++)
+        r += (uint32_t)__builtin_amdgcn_readlane((int)v, (int)t) < v ? 1u : 0u;
+    if (on) {
+        b.id_out[lo + r] = v;
+        b.idx_out[lo + r] = x;
+    }
+}
+
+// The buckets' entries in id order.  The buckets are sized for a store that
+// has all left, and few particles leave in a step, so most are empty: a
+// wavefront takes STEADY_BPW buckets of one side.  All their entries together
+// when they are at most 64 (a later bucket of a side holds greater ids),
+// otherwise one bucket after the other, and those above 64 entries by the
+// whole workgroup.  2 x 262 144 particles: 5.0 us, a workgroup per bucket
+// took 6.6.
+#define STEADY_BPW 32
+__global__ void __launch_bounds__(256) k_steady_sort(SteadyArgs a) {
+    const SteadyBufs &b = a.b[blockIdx.y];
+    __shared__ uint32_t sk[STEADY_LDS], sv[STEADY_LDS];
+    __shared__ uint32_t big[4 * STEADY_BPW], nbig;
+    if (threadIdx.x == 0) nbig = 0u;
+    __syncthreads();
+    const uint32_t per_side = (b.nb + STEADY_BPW - 1) / STEADY_BPW;  // waves of a side
+    const uint32_t wave = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (wave < 2 * per_side) {
+        const uint32_t side = wave / per_side;
+        const uint32_t f = side * b.nb + (wave - side * per_side) * STEADY_BPW;
+        const uint32_t m = min((uint32_t)STEADY_BPW, (side + 1) * b.nb - f);
+        const uint32_t s0 = b.start[f + min(lane, m)];  // lane m and up: the end
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)s0, 0);
+        const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)s0, 63) - lo;
+        if (k <= 64) {
+            if (k) steady_sort_wave(b, lo, k);
+        } else {
+            const uint32_t kl = __shfl_down(s0, 1, 64) - s0;
+            uint64_t todo = __ballot(lane < m && kl > 0);
+            while (todo) {
+                const int t = __ffsll((unsigned long long)todo) - 1;
+                todo &= todo - 1;
+                const uint32_t l = (uint32_t)__builtin_amdgcn_readlane((int)s0, t);
+                const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)kl, t);
+                if (c <= 64)
+                    steady_sort_wave(b, l, c);
+                else if (lane == 0)
+                    big[atomicAdd(&nbig, 1u)] = f + (uint32_t)t;
+            }
+        }
+    }
+    __syncthreads();
+    const uint32_t nl = nbig;
+    for (uint32_t t = 0; t < nl; t++) {
+        const uint32_t f = big[t], l = b.start[f];
+        steady_sort_block(b, l, b.start[f + 1] - l, sk, sv);
     }
 }
 
@@ -2715,7 +2786,8 @@ void launch_steady(hipStream_t st, const SteadyArgs &a, const mcc::MccConst &mc,
         hipLaunchKernelGGL(k_steady_scan, dim3(2), dim3(1024), 0, st, a);
         hipLaunchKernelGGL(k_steady_scatter, dim3(blocks_for(cap, 256), 2), dim3(256), 0, st, a, N,
                            axis);
-        hipLaunchKernelGGL(k_steady_sort, dim3(2 * a.b[0].nb, 2), dim3(256), 0, st, a);
+        const uint32_t waves = 2 * ((a.b[0].nb + STEADY_BPW - 1) / STEADY_BPW);
+        hipLaunchKernelGGL(k_steady_sort, dim3((waves + 3) / 4, 2), dim3(256), 0, st, a);
         hipLaunchKernelGGL(k_steady_pair, dim3(blocks_for(pairs, 256)), dim3(256), 0, st, a, mc,
                            step, N, se, si, qe, qi, mode);
     }

@@ -52,11 +52,11 @@ __device__ __forceinline__ uint32_t cnt_slot() { return blockIdx.x & (CNT_SLOTS 
 // (so the layout and the new ids are deterministic), appends them to a
 // particle buffer and optionally deposits their charge.
 // Candidates of the reference's steady walls for one species and one axis:
-// bucket counts, bucket starts (2 nb + 1) and scatter cursors over nb id
+// bucket counts (zero between passes) and bucket starts (2 nb + 1) over nb id
 // ranges per side; the candidates (id, index into the store) in bucket
 // order, then sorted by id within each bucket.  cap = the species' store.
 struct SteadyBufs {
-    uint32_t *hist, *start, *cursor;
+    uint32_t *hist, *start;
     uint32_t *id_in, *idx_in, *id_out, *idx_out;
     uint32_t nb;
 };
