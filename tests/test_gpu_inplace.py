@@ -68,7 +68,7 @@ def compare(a, b, kind, n):
         assert a[3][0].sum() > n  # a quarter of the electrons a step at least
 
 
-@pytest.mark.parametrize("n", [1, 1023, 1025, 5000])
+@pytest.mark.parametrize("n", [1, 1023, 1025, 5000, 263000])  # (the last: four particles a thread)
 @pytest.mark.parametrize("kind", ["absorb", "steady", "emit", "argon", "argon_emit", "dense"])
 @pytest.mark.parametrize("sort", [16, 2])
 def test_weighted_passes_match_the_generic_pass(n, kind, sort):

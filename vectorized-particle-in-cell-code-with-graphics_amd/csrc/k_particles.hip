@@ -196,6 +196,13 @@ __device__ __forceinline__ bool collide_take(bool blk, int qs, PState &s, int &e
 // block's particles of one key take consecutive slots.  Every particle's rank
 // within its key comes from the LDS counter of its entry.
 #define IPP (PASS_BLOCK / 256)
+// The in-place passes of a store of at most INPL_SMALL_MAX particles (with IPP
+// per thread less than a block for each of 256 CUs) take IPP_SMALL per thread:
+// there a pass is the latency of one block's chain, not throughput.  2 x
+// 262 144 particles in reference mode 2.55 -> 2.30 ms for ten steps, 33^2 148
+// -> 142 us; at 410 000 particles (65^2) 737 -> 796 us, two per thread 734.
+#define IPP_SMALL 1
+#define INPL_SMALL_MAX (256 * PASS_BLOCK)
 #define HASH_BITS 11
 #define HASH_SIZE (1 << HASH_BITS)  // >= 2 x 256 x IPP
 #define HASH_EMPTY 0xFFFFFFFFu
@@ -1188,14 +1195,15 @@ __device__ __forceinline__ void collide_queue(const bool (&live)[P], float (&vx)
         }
 }
 
-// gather_one's field of two particles, every load issued before the first is
+// gather_one's field of G particles, every load issued before the first is
 // used; a particle that cannot move (ok false) reads node 0
-__device__ __forceinline__ void gather_two(const PState (&s)[2], const bool (&ok)[2],
-                                           const float2 *__restrict__ E, int N, float (&ex)[2],
-                                           float (&ey)[2]) {
-    float2 e00[2], e01[2], e10[2], e11[2];
+template <int G>
+__device__ __forceinline__ void gather_field(const PState (&s)[G], const bool (&ok)[G],
+                                           const float2 *__restrict__ E, int N, float (&ex)[G],
+                                           float (&ey)[G]) {
+    float2 e00[G], e01[G], e10[G], e11[G];
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
+    for (int r = 0; r < G; r++) {
         const uint32_t b = ok[r] ? (uint32_t)(s[r].jy * N + s[r].jx) : 0u;
         const float2 *lo = E + b, *hi = E + (b + (uint32_t)N);
         e00[r] = lo[0];
@@ -1204,7 +1212,7 @@ __device__ __forceinline__ void gather_two(const PState (&s)[2], const bool (&ok
         e11[r] = hi[1];
     }
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
+    for (int r = 0; r < G; r++) {
         const float wj = s[r].ox, wk = s[r].oy;
         const float a4 = (1.0f - wj) * (1.0f - wk), a3 = wj * (1.0f - wk);
         const float a2 = wk * (1.0f - wj), a1 = wj * wk;
@@ -1380,7 +1388,7 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
             t[g] = PState{cell_jx(c0[r]), cell_jy(c0[r]), ox[r], oy[r], vx[r], vy[r], vz[r]};
             ok[g] = claim[r] && inside_cells(t[g], pc.N);
         }
-        gather_two(t, ok, E, pc.N, ex, ey);
+        gather_field<2>(t, ok, E, pc.N, ex, ey);
 #pragma unroll
         for (int g = 0; g < 2; g++) {
             const int r = h + g;
@@ -1538,6 +1546,7 @@ __device__ __forceinline__ void inplace_round(const SpView &sp, uint32_t i, uint
 
 // The in-place pass with every option taken at run time (push_inplace_body's
 // comment says what an in-place pass is).
+template <int P>
 __device__ __forceinline__ void push_inplace_generic(
     SpView sp, const uint32_t *__restrict__ nptr, const float2 *__restrict__ E, PushConst pc,
     mcc::MccConst mc, uint32_t step, unsigned long long *__restrict__ q, int deposit, Spawn spn,
@@ -1546,7 +1555,7 @@ __device__ __forceinline__ void push_inplace_generic(
     const uint32_t n = *nptr;
     // the grid covers the capacity: blocks past the live count leave at once
     // (uniformly, before any barrier); bid: this block's index in the species
-    if (bid * (blockDim.x * IPP) >= n) return;
+    if (bid * (blockDim.x * P) >= n) return;
     __shared__ uint32_t sl[6];
     __shared__ uint32_t shole;
     __shared__ uint32_t se[8];
@@ -1555,19 +1564,19 @@ __device__ __forceinline__ void push_inplace_generic(
     if (threadIdx.x < 6) sl[threadIdx.x] = 0;
     if (threadIdx.x < 8) se[threadIdx.x] = 0;
     if (threadIdx.x == 0) shole = 0;
-    const uint32_t base = bid * (blockDim.x * IPP) + threadIdx.x;
+    const uint32_t base = bid * (blockDim.x * P) + threadIdx.x;
     // vz and the id are read only where something uses them: the magnetic
     // rotation, collisions, re-injection keyed by the id, and the wall
     // queue (surface physics needs the full velocity and the id's draws)
     const bool need_vz = pc.bfield != 0 || mc.on || spn.wall;
     const bool need_id = mc.on || spn.plop || spn.wall;
     const bool blk = mc.on && mc.mode == PIC_DEV_MODE_PHYS;
-    PState s[IPP];
-    uint32_t pid[IPP];
-    bool live[IPP];
-    float w[IPP];
+    PState s[P];
+    uint32_t pid[P];
+    bool live[P];
+    float w[P];
 #pragma unroll
-    for (int r = 0; r < IPP; r++) {  // every load first
+    for (int r = 0; r < P; r++) {  // every load first
         const uint32_t i = base + r * blockDim.x;
         s[r] = PState{};
         pid[r] = 0u;
@@ -1584,34 +1593,25 @@ __device__ __forceinline__ void push_inplace_generic(
     __shared__ float2 sbins[MCC_BINS];
     if (blk && mc.bins && threadIdx.x < MCC_BINS) sbins[threadIdx.x] = mc.bins[threadIdx.x];
     __syncthreads();  // counters initialised, bounds staged
-    int qs[IPP];
-    if (blk) block_collide_n<IPP>(live, s, pid, mc, step, qs, lds, mc.bins ? sbins : nullptr);
-    bool dep[IPP], kept[IPP];
-    // the rounds are spelled out so every array index is a compile-time constant
-    inplace_round(sp, base + 0 * blockDim.x, n, s[0], pid[0], live[0], dep[0], kept[0], E, pc,
-                  mc, step,
-                  spn, lost6, need_vz, blk, qs[0], sl, &shole, se, lds, w[0]);
-    inplace_round(sp, base + 1 * blockDim.x, n, s[1], pid[1], live[1], dep[1], kept[1], E, pc,
-                  mc, step,
-                  spn, lost6, need_vz, blk, qs[1], sl, &shole, se, lds, w[1]);
-    inplace_round(sp, base + 2 * blockDim.x, n, s[2], pid[2], live[2], dep[2], kept[2], E, pc,
-                  mc, step,
-                  spn, lost6, need_vz, blk, qs[2], sl, &shole, se, lds, w[2]);
-    inplace_round(sp, base + 3 * blockDim.x, n, s[3], pid[3], live[3], dep[3], kept[3], E, pc,
-                  mc, step,
-                  spn, lost6, need_vz, blk, qs[3], sl, &shole, se, lds, w[3]);
+    int qs[P];
+    if (blk) block_collide_n<P>(live, s, pid, mc, step, qs, lds, mc.bins ? sbins : nullptr);
+    bool dep[P], kept[P];
+#pragma unroll
+    for (int r = 0; r < P; r++)
+        inplace_round(sp, base + r * blockDim.x, n, s[r], pid[r], live[r], dep[r], kept[r], E, pc,
+                      mc, step, spn, lost6, need_vz, blk, qs[r], sl, &shole, se, lds, w[r]);
     // block_deposit_n passes a barrier before it writes the window, so every
     // round has read its collision result from the shared LDS by then
-    if (deposit) block_deposit_n<IPP, LDS_U64>(dep, s, w, q, pc.N, lds);
+    if (deposit) block_deposit_n<P, LDS_U64>(dep, s, w, q, pc.N, lds);
     __syncthreads();
     // ahead of a sort pass: the histogram of the cells the particles end the
     // step in, the keys that pass claims by (no k_key_count then)
     if (hist) {
-        uint32_t key[IPP];
+        uint32_t key[P];
 #pragma unroll
-        for (int r = 0; r < IPP; r++)
+        for (int r = 0; r < P; r++)
             key[r] = kept[r] ? bin_key(s[r].jx, s[r].jy, pc.tilesX) >> pc.keyshift : 0u;
-        block_key_hist<IPP>(kept, key, hist, reinterpret_cast<uint32_t *>(lds));
+        block_key_hist<P>(kept, key, hist, reinterpret_cast<uint32_t *>(lds));
     }
     if (threadIdx.x < 6 && sl[threadIdx.x])
         atomicAdd(&lost6[cnt_slot() * 6 + threadIdx.x], sl[threadIdx.x]);
@@ -1634,9 +1634,9 @@ constexpr int inplace_lds_u64() {
 // push as the sort pass, the state written back to its own slot, the
 // deposit through one LDS window per block.  A particle that leaves (or that
 // a collision removes) becomes a hole; the next sort pass compacts the store.
-// Each thread handles IPP particles (strided by the block size, so every
+// Each thread handles P particles (strided by the block size, so every
 // load and store stays coalesced): one deposit window and one flush of the
-// block's counters then serve 256 * IPP particles.  Reads 20-28 B and writes
+// block's counters then serve 256 * P particles.  Reads 20-28 B and writes
 // 20-24 B per particle, with no histogram or slot claims.
 //
 // Bound by HBM (257^2, 13.1 M particles: 129 us the ions, 149 us the
@@ -1649,7 +1649,7 @@ constexpr int inplace_lds_u64() {
 // for its own cell and then its own field loads, and the collision code was
 // inlined once more in every round (queue overflow): 269 VALU instructions
 // per ion and 374 per electron instead of 196 and 261, 158 and 210 us.
-template <int V>
+template <int V, int P>
 __device__ __forceinline__ void push_inplace_body(
     SpView sp, const uint32_t *__restrict__ nptr, const float2 *__restrict__ E, PushConst pc,
     mcc::MccConst mc, uint32_t step, unsigned long long *__restrict__ q, int deposit, Spawn spn,
@@ -1658,7 +1658,7 @@ __device__ __forceinline__ void push_inplace_body(
     pin_variant<V>(pc, mc, sp);
     pin_spawn<V>(spn);
     constexpr bool COLL = pv_coll_e(V) || pv_coll_i(V), WGT = pv_weighted(V);
-    const uint32_t n = *nptr, blk0 = bid * (256 * IPP);
+    const uint32_t n = *nptr, blk0 = bid * (256 * P);
     // the grid covers the capacity: blocks past the live count leave at once
     // (uniformly, before any barrier); bid: this block's index in the species
     if (blk0 >= n) return;
@@ -1667,19 +1667,19 @@ __device__ __forceinline__ void push_inplace_body(
     __shared__ uint32_t se[8];
     constexpr int LDS_U64 = inplace_lds_u64<V>();
     __shared__ unsigned long long lds[LDS_U64];
-    static_assert(!COLL || CQ_WORDS * IPP * 256 * 4 <= LDS_U64 * 8, "collision queue size");
+    static_assert(!COLL || CQ_WORDS * P * 256 * 4 <= LDS_U64 * 8, "collision queue size");
     const uint32_t tid = threadIdx.x;
     if (tid < 6) sl[tid] = 0;
     if (tid < 8) se[tid] = 0;
     if (tid == 0) shole = 0;
-    uint32_t c0[IPP], pid[IPP];
-    float ox[IPP], oy[IPP], vx[IPP], vy[IPP], vz[IPP], w[IPP];
+    uint32_t c0[P], pid[P];
+    float ox[P], oy[P], vx[P], vy[P], vz[P], w[P];
     {
         const uint32_t *pc_ = sp.cell + blk0, *pi = sp.id + blk0;
         const float *px = sp.ox + blk0, *py = sp.oy + blk0, *pu = sp.vx + blk0,
                     *pv = sp.vy + blk0, *pz = sp.vz + blk0;
 #pragma unroll
-        for (int r = 0; r < IPP; r++) {  // every load first
+        for (int r = 0; r < P; r++) {  // every load first
             c0[r] = pc_[tid + r * 256];
             if (COLL) pid[r] = pi[tid + r * 256];
             vx[r] = pu[tid + r * 256];
@@ -1693,35 +1693,36 @@ __device__ __forceinline__ void push_inplace_body(
     // the electrons' null-collision bounds in LDS (loaded beside the state)
     __shared__ float2 sbins[MCC_BINS];
     if (pv_coll_e(V) && mc.bins && tid < MCC_BINS) sbins[tid] = mc.bins[tid];
-    bool live[IPP];
+    bool live[P];
 #pragma unroll
-    for (int r = 0; r < IPP; r++) {
+    for (int r = 0; r < P; r++) {
         live[r] = blk0 + tid + r * 256 < n && cell_jx(c0[r]) != CELL_HOLE;
     }
     __syncthreads();  // counters initialised, bounds staged
     if (COLL)
-        collide_queue<IPP, pv_coll_e(V), false>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step,
+        collide_queue<P, pv_coll_e(V), false>(live, vx, vy, vz, pid, sp, blk0, E, pc, mc, step,
                                                 spn, lost6, se,
                                                 pv_coll_e(V) && mc.bins ? sbins : nullptr,
                                                 reinterpret_cast<float *>(lds));
-    PState s[IPP];
-    bool dep[IPP];
+    PState s[P];
+    bool dep[P];
     uint32_t *pc_ = sp.cell + blk0;
     float *px = sp.ox + blk0, *py = sp.oy + blk0, *pu = sp.vx + blk0, *pv = sp.vy + blk0;
+    constexpr int G = P > 1 ? 2 : 1;
 #pragma unroll
-    for (int h = 0; h < IPP; h += 2) {  // the field loads of two particles at a time
-        PState t[2];
-        bool ok[2];
-        float ex[2], ey[2];
+    for (int h = 0; h < P; h += G) {  // the field loads of two particles at a time
+        PState t[G];
+        bool ok[G];
+        float ex[G], ey[G];
 #pragma unroll
-        for (int g = 0; g < 2; g++) {
+        for (int g = 0; g < G; g++) {
             const int r = h + g;
             t[g] = PState{cell_jx(c0[r]), cell_jy(c0[r]), ox[r], oy[r], vx[r], vy[r], 0.0f};
             ok[g] = live[r] && inside_cells(t[g], pc.N);
         }
-        gather_two(t, ok, E, pc.N, ex, ey);
+        gather_field<G>(t, ok, E, pc.N, ex, ey);
 #pragma unroll
-        for (int g = 0; g < 2; g++) {
+        for (int g = 0; g < G; g++) {
             const int r = h + g;
             s[r] = t[g];
             move_sel(s[r], ok[g], ex[g], ey[g], pc);
@@ -1755,16 +1756,16 @@ __device__ __forceinline__ void push_inplace_body(
     }
     // block_deposit_n passes a barrier before it writes the window, so every
     // lane has read its collision result from the shared LDS by then
-    if (deposit) block_deposit_n<IPP, LDS_U64>(dep, s, w, q, pc.N, lds);
+    if (deposit) block_deposit_n<P, LDS_U64>(dep, s, w, q, pc.N, lds);
     __syncthreads();
     // ahead of a sort pass: the histogram of the cells the particles end the
     // step in, the keys that pass claims by (no k_key_count then)
     if (hist) {
-        uint32_t key[IPP];
+        uint32_t key[P];
 #pragma unroll
-        for (int r = 0; r < IPP; r++)
+        for (int r = 0; r < P; r++)
             key[r] = dep[r] ? bin_key(s[r].jx, s[r].jy, pc.tilesX) >> pc.keyshift : 0u;
-        block_key_hist<IPP>(dep, key, hist, reinterpret_cast<uint32_t *>(lds));
+        block_key_hist<P>(dep, key, hist, reinterpret_cast<uint32_t *>(lds));
     }
     if (tid < 6 && sl[tid]) atomicAdd(&lost6[cnt_slot() * 6 + tid], sl[tid]);
     if (COLL && tid < 8 && se[tid])
@@ -1777,13 +1778,16 @@ __device__ __forceinline__ void push_inplace_body(
         mcc::MccConst mc, uint32_t step, unsigned long long *__restrict__ q, int deposit,     \
         Spawn spn, unsigned long long *__restrict__ events, uint32_t *__restrict__ lost6,     \
         uint32_t *__restrict__ holes, uint32_t *__restrict__ hist
-template <int V>
+template <int V, int P>
 __global__ void __launch_bounds__(256) k_push_inplace(PUSH_INPLACE_PARAMS);
-template <>
-__global__ void __launch_bounds__(256) k_push_inplace<PV_GENERIC>(PUSH_INPLACE_PARAMS) {
-    push_inplace_generic(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes, hist,
-                         blockIdx.x);
-}
+#define INPLACE_GENERIC(P)                                                                      \
+    template <>                                                                                \
+    __global__ void __launch_bounds__(256) k_push_inplace<PV_GENERIC, P>(PUSH_INPLACE_PARAMS) { \
+        push_inplace_generic<P>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes, \
+                                hist, blockIdx.x);                                             \
+    }
+INPLACE_GENERIC(IPP)
+INPLACE_GENERIC(IPP_SMALL)
 // Waves per SIMD, measured over 4 to 8 at 257^2 and 1025^2 (20 and 10 steps
 // of the argon discharge): 7 for the collisionless variants (66-72 VGPRs) and
 // 5 for the collisional ones (87), 7.37 and 36.3 ms; 6 and 4: 7.58 and 37.0; 8
@@ -1792,13 +1796,16 @@ __global__ void __launch_bounds__(256) k_push_inplace<PV_GENERIC>(PUSH_INPLACE_P
 #define INPL_WAVES_COLL 5
 #define INPL_WAVES_COLL_I 7
 #define INPL_WAVES_W 6  // four weights more in registers
-#define INPLACE_FAST(V, WAVES)                                                                 \
+#define INPLACE_FAST_P(V, P, WAVES)                                                            \
     template <>                                                                                \
     __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))  \
-        k_push_inplace<V>(PUSH_INPLACE_PARAMS) {                                               \
-        push_inplace_body<V>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6, holes, \
-                             hist, blockIdx.x);                                                \
+        k_push_inplace<V, P>(PUSH_INPLACE_PARAMS) {                                            \
+        push_inplace_body<V, P>(sp, nptr, E, pc, mc, step, q, deposit, spn, events, lost6,     \
+                                holes, hist, blockIdx.x);                                      \
     }
+#define INPLACE_FAST(V, WAVES)    \
+    INPLACE_FAST_P(V, IPP, WAVES) \
+    INPLACE_FAST_P(V, IPP_SMALL, WAVES)
 INPLACE_FAST(PV_PLAIN, INPL_WAVES_PLAIN)
 INPLACE_FAST(PV_SPAWN, INPL_WAVES_PLAIN)
 INPLACE_FAST(PV_COLL_E, INPL_WAVES_COLL)
@@ -1811,14 +1818,15 @@ INPLACE_FAST((PV_COLL_I | PV_W), INPL_WAVES_W)
 // Both species' collisionless in-place passes in one launch (the first nba
 // blocks advance a, the rest b): the kernel of each species pass as it is,
 // one launch's fixed cost instead of two on the small grids
+template <int P>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(INPL_WAVES_PLAIN, INPL_WAVES_PLAIN)))
     k_push_inplace_pair(InplaceArgs a, InplaceArgs b, uint32_t nba,
                         const float2 *__restrict__ E, uint32_t step, int deposit) {
     if (blockIdx.x < nba)
-        push_inplace_body<PV_PLAIN>(a.sp, a.n, E, a.pc, a.mc, step, a.q, deposit, a.spn,
+        push_inplace_body<PV_PLAIN, P>(a.sp, a.n, E, a.pc, a.mc, step, a.q, deposit, a.spn,
                                     a.events, a.lost6, a.holes, a.hist, blockIdx.x);
     else
-        push_inplace_body<PV_PLAIN>(b.sp, b.n, E, b.pc, b.mc, step, b.q, deposit, b.spn,
+        push_inplace_body<PV_PLAIN, P>(b.sp, b.n, E, b.pc, b.mc, step, b.q, deposit, b.spn,
                                     b.events, b.lost6, b.holes, b.hist, blockIdx.x - nba);
 }
 
@@ -2460,7 +2468,7 @@ __device__ __forceinline__ void steady_sort_wave(const SteadyBufs &b, uint32_t l
 // otherwise one bucket after the other, and those above 64 entries by the
 // whole workgroup.  2 x 262 144 particles: 5.0 us, a workgroup per bucket
 // took 6.6.
-#define STEADY_BPW 32
+#define STEADY_BPW 8
 __global__ void __launch_bounds__(256) k_steady_sort(SteadyArgs a) {
     const SteadyBufs &b = a.b[blockIdx.y];
     __shared__ uint32_t sk[STEADY_LDS], sv[STEADY_LDS];
@@ -2692,15 +2700,22 @@ void launch_push_scatter(hipStream_t st, const SpView &src, const SpView &dst, c
 #undef SCATTER
 }
 
+static int inplace_ipp(int64_t cap) { return cap <= INPL_SMALL_MAX ? IPP_SMALL : IPP; }
+
 void launch_push_inplace(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
                          const float2 *E, const PushConst &pc, const mcc::MccConst &mc,
                          uint32_t step, unsigned long long *q, int deposit, const Spawn &spn,
                          unsigned long long *events, uint32_t *lost6, uint32_t *holes,
                          uint32_t *hist) {
-    const dim3 grid(blocks_for(cap, 256 * IPP)), blk(256);
-#define INPLACE(V)                                                                             \
-    hipLaunchKernelGGL(k_push_inplace<V>, grid, blk, 0, st, sp, n, E, pc, mc, step, q, deposit, \
-                       spn, events, lost6, holes, hist)
+    const int p = inplace_ipp(cap);
+    const dim3 grid(blocks_for(cap, 256 * p)), blk(256);
+#define INPLACE(V)                                                                              \
+    if (p == IPP)                                                                               \
+        hipLaunchKernelGGL((k_push_inplace<V, IPP>), grid, blk, 0, st, sp, n, E, pc, mc, step,  \
+                           q, deposit, spn, events, lost6, holes, hist);                        \
+    else                                                                                        \
+        hipLaunchKernelGGL((k_push_inplace<V, IPP_SMALL>), grid, blk, 0, st, sp, n, E, pc, mc,  \
+                           step, q, deposit, spn, events, lost6, holes, hist)
     switch (pass_variant(sp, pc, mc, &spn)) {
     case PV_PLAIN: INPLACE(PV_PLAIN); break;
     case PV_SPAWN: INPLACE(PV_SPAWN); break;
@@ -2722,10 +2737,15 @@ bool inplace_pair_ok(const InplaceArgs &a, const InplaceArgs &b) {
 
 void launch_push_inplace_pair(hipStream_t st, const InplaceArgs &a, const InplaceArgs &b,
                               const float2 *E, uint32_t step, int deposit) {
-    const uint32_t nba = (uint32_t)blocks_for(a.cap, 256 * IPP);
-    const uint32_t nb = nba + (uint32_t)blocks_for(b.cap, 256 * IPP);
-    hipLaunchKernelGGL(k_push_inplace_pair, dim3(nb), dim3(256), 0, st, a, b, nba, E, step,
-                       deposit);
+    const int p = inplace_ipp(std::max(a.cap, b.cap));
+    const uint32_t nba = (uint32_t)blocks_for(a.cap, 256 * p);
+    const uint32_t nb = nba + (uint32_t)blocks_for(b.cap, 256 * p);
+    if (p == IPP)
+        hipLaunchKernelGGL(k_push_inplace_pair<IPP>, dim3(nb), dim3(256), 0, st, a, b, nba, E, step,
+                           deposit);
+    else
+        hipLaunchKernelGGL(k_push_inplace_pair<IPP_SMALL>, dim3(nb), dim3(256), 0, st, a, b, nba, E,
+                           step, deposit);
 }
 
 void launch_mcc(hipStream_t st, const SpView &sp, const uint32_t *n, int64_t cap,
