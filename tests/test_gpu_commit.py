@@ -42,3 +42,24 @@ def test_largest_commit_is_in_key_order(largest):
     for s in (0, 1):
         assert np.array_equal(np.diff(largest[s]["id"]), np.ones(LARGEST - 1))
         assert len(np.unique(largest[s]["vx"])) > LARGEST // 2
+
+
+@pytest.mark.parametrize("n", [1, 1024, 1025, 4_300_000, 17_000_000])
+def test_wall_pass_keeps_the_store_order(n):
+    """The absorbing walls' compaction, whose scan takes one workgroup up to four
+    tiles of block counts (16.8 M particles) and three launches beyond: the
+    particles inside stay, in order."""
+    print(f"wall pass n={n}", flush=True)
+    p = workloads.discharge(16, 4, te=40.0)
+    p.init_particle_no = n
+    with pic2d.Pic(p) as sim:
+        sim.get_particle_electric_field(0)
+        sim.move_particles(0)
+        a = sim.get_state(0)
+        sim.boundary(1)
+        b = sim.get_state(0)
+        jx, jy = pic2d.cell_unpack(a["cell"])
+        keep = (jx >= 0) & (jx <= p.nodes - 2) & (jy >= 0) & (jy <= p.nodes - 2)
+        assert n < 1000 or 0 < keep.sum() < n
+        for k in ("id", "cell", "ox", "vx"):
+            assert np.array_equal(a[k][keep], b[k]), k
