@@ -63,3 +63,31 @@ def test_wall_pass_keeps_the_store_order(n):
         assert n < 1000 or 0 < keep.sum() < n
         for k in ("id", "cell", "ox", "vx"):
             assert np.array_equal(a[k][keep], b[k]), k
+
+
+@pytest.mark.parametrize("walls", [True, False])
+def test_gather_sorts_a_store_that_has_moved_and_passed_the_walls(walls):
+    """phase by phase, a gather after sort_interval moves sorts the particles by
+    tile (and drops none); without the wall pass the store keeps its order and
+    its particles outside"""
+    print(f"gather sort, walls {walls}", flush=True)
+    p = workloads.discharge(64, 4, te=40.0)
+    p.sort_key = 6  # one tile
+    p.sort_interval = 2
+    with pic2d.Pic(p) as sim:
+        for _ in range(2):
+            sim.get_particle_electric_field(0)
+            sim.move_particles(0)
+            if walls:
+                sim.boundary(1)
+        a = sim.get_state(0)
+        sim.get_particle_electric_field(0)
+        b = sim.get_state(0)
+        if walls:
+            jx, jy = pic2d.cell_unpack(b["cell"])
+            tile = (jy + 1) // 8 * 64 + (jx + 1) // 8  # of the halo grid
+            assert (np.diff(tile) < 0).sum() < len(tile) // 16
+            ia, ib = np.argsort(a["id"]), np.argsort(b["id"])
+            a, b = ({k: v[i] for k, v in d.items()} for d, i in ((a, ia), (b, ib)))
+        for k in ("id", "cell", "ox", "oy", "vx", "vy", "vz"):
+            assert np.array_equal(a[k], b[k]), k

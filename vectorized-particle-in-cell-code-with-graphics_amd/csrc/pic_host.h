@@ -32,6 +32,7 @@ struct Species {
     pic::StageView stage = {};  // particles created during a step
     int sort_interval = 1;  // particle passes per counting sort
     int since_sort = 0;   // in-place steps since the last sort pass
+    bool walled = false;  // pic_boundary has run since the last pic_species_move
     bool holes = false;   // the current buffer may hold empty slots
     // the last in-place pass (and the commits after it) counted the keys of
     // the next sort pass into this species' histogram
