@@ -135,9 +135,11 @@ typedef struct pic_params {
                                     k = 0..10 (0: per cell; 6: per 8x8-cell tile;
                                     7..10: 2..16 tiles along x); -1 = chosen by
                                     the library                                    */
-    int32_t mg_sweeps;           /* PIC_MG_TOL: red-black sweeps before and after
-                                    the coarse correction on each level, 1..3
-                                    (V(1,1)..V(3,3)); -1 = chosen by the library   */
+    int32_t mg_sweeps;           /* PIC_MG_TOL: -1 (the default): the direct sine-
+                                    transform solve up to 4097^2, V(2,2) cycles
+                                    above; 1..3: V(1,1)..V(3,3) cycles above 65^2
+                                    (sweeps before and after the coarse
+                                    correction), the direct solve up to 65^2       */
     int32_t null_bound;          /* physical-mode electron collisions: the null-
                                     collision bound per energy bin of the electron
                                     (PIC_NULL_BOUND_BINNED, the default) or one
@@ -148,7 +150,8 @@ typedef struct pic_params {
                                     as hipGraphs and replayed; 0 (default):
                                     launched kernel by kernel.  Results are
                                     identical; on MI355X the replay measured
-                                    slower (C2 field solve 0.235 vs 0.229 ms).     */
+                                    slower (257^2: 0.235 vs 0.229 ms a solve).  No
+                                    effect on the direct solve.                    */
 } pic_params;
 
 #define PIC_NULL_BOUND_BINNED 0
@@ -323,11 +326,11 @@ int pic_poisson_tol(const double *f, double *u, int32_t n, double length, double
                     int32_t max_iter, int32_t *cycles, double *relres);
 
 /* --------------------------------------------------------------- getters */
-/* multigrid work of the last solve: V-cycles (tolerance mode) or ncycle,
- * cumulative V-cycles, and the relative residual reached (tolerance mode).
- * Grids up to 65^2 are solved without a host wait during the step: this
- * call then waits for the last solve's verdict if the device has not
- * finished it. */
+/* work of the last solve: V-cycles, or 1 for the direct solve (tolerance
+ * mode), or ncycle; the cumulative count; and the relative residual reached
+ * (tolerance mode).  The direct solve runs without a host wait during the
+ * step: this call then sums the last solve's residual, waiting for the device
+ * if it has not finished it. */
 int pic_get_mg_stats(pic_handle *h, int32_t *last_cycles, int64_t *total_cycles, double *relres);
 int pic_particle_size(pic_handle *h, int32_t s, int64_t *n);        /* particle::particle_size */
 int pic_get_particles(pic_handle *h, int32_t s, pic_particle *out, int64_t cap); /* 48-B AoS copy */
