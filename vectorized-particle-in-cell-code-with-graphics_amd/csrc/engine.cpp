@@ -803,6 +803,7 @@ void push_species(pic_handle *h, int si, int do_push, int deposit) {
     s.cur = 1 - c;
     s.holes = do_push != 0;
     s.since_sort = 0;
+    s.order_seen = false;
 }
 
 // collisions + push + deposit of one species in place (no sort): removed
@@ -907,14 +908,14 @@ int absorb_species(pic_handle *h, int si, bool plop) {
 // A loop driven phase by phase moves its particles without a sort pass, and
 // gather and deposit slow down as the store loses its order (129^2, 1.05 M
 // particles per species: four steps take 1.22 ms then, 0.59 with the sorts).  A
-// gather after as many moves as the
-// fused step makes passes between sorts sorts first.  An uploaded store keeps
-// the caller's order, and one that has not passed the walls since its move its
-// particles outside (the sort would drop them).
+// gather after as many moves as the fused step makes passes between sorts
+// sorts first.  A store whose order the caller may know keeps it (loaded,
+// uploaded, or read since its last sort pass), and one that has not passed the
+// walls since its move keeps its particles outside (the sort would drop them).
 void resort(pic_handle *h, int si) {
     const Species &s = h->sp[si];
-    if (h->P.mode == PIC_MODE_PHYSICAL && s.walled && s.since_sort >= s.sort_interval &&
-        s.since_sort < (1 << 20))
+    if (h->P.mode == PIC_MODE_PHYSICAL && s.walled && !s.order_seen &&
+        s.since_sort >= s.sort_interval && s.since_sort < (1 << 20))
         push_species(h, si, 0, 0);
 }
 
@@ -1890,6 +1891,7 @@ int pic_get_state(pic_handle *h, int32_t s, uint32_t *cell, float *ox, float *oy
     int64_t n;
     CHECK(pic_particle_size(h, s, &n));
     if (n > cap) return seterr(h, PIC_ERR_CAPACITY, "output buffer too small");
+    h->sp[s].order_seen = true;
     const SpView &b = h->sp[s].buf[h->sp[s].cur];
     size_t bytes = 4 * (size_t)n;
     if (cell) HIPCHK(h, hipMemcpyAsync(cell, b.cell, bytes, hipMemcpyDeviceToHost, h->st));
@@ -1965,7 +1967,8 @@ int pic_get_weights(pic_handle *h, int32_t s, float *w, int64_t cap) {
     int64_t n;
     CHECK(pic_particle_size(h, s, &n));
     if (n > cap || (!w && n > 0)) return seterr(h, PIC_ERR_CAPACITY, "output buffer too small");
-    const Species &sp = h->sp[s];
+    Species &sp = h->sp[s];
+    sp.order_seen = true;
     if (!sp.weighted) {
         for (int64_t i = 0; i < n; i++) w[i] = (float)sp.weight;
         return PIC_OK;
@@ -1982,6 +1985,7 @@ int pic_set_weights(pic_handle *h, int32_t s, const float *w, int64_t n) {
     if (!w && n > 0) return seterr(h, PIC_ERR_ARG, "null array");
     Species &sp = h->sp[s];
     CHECK(enable_weights(h, sp));
+    sp.order_seen = true;
     HIPCHK(h, hipMemcpyAsync(sp.buf[sp.cur].w, w, 4 * (size_t)n, hipMemcpyHostToDevice, h->st));
     HIPCHK(h, hipStreamSynchronize(h->st));
     return PIC_OK;
@@ -2650,6 +2654,7 @@ int pic_checkpoint_read(pic_handle *h, const char *path) {
         Species &sp = h->sp[s];
         sp.since_sort = H.sp[s].since_sort;
         sp.walled = false;
+        sp.order_seen = true;
         sp.holes = H.sp[s].holes != 0;
         sp.weight = H.sp[s].weight;
         sp.scale = H.sp[s].scale;

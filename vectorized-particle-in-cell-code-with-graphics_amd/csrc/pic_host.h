@@ -33,6 +33,7 @@ struct Species {
     int sort_interval = 1;  // particle passes per counting sort
     int since_sort = 0;   // in-place steps since the last sort pass
     bool walled = false;  // pic_boundary has run since the last pic_species_move
+    bool order_seen = true;  // the caller may know the store's order (no sort pass since)
     bool holes = false;   // the current buffer may hold empty slots
     // the last in-place pass (and the commits after it) counted the keys of
     // the next sort pass into this species' histogram
