@@ -21,8 +21,12 @@ def by_id(sim, s):
     return {k: v[o] for k, v in d.items()}
 
 
+WEAK = 1e-30  # [T]: the generic passes, the same bits
+CELL_REMOVED = -16001  # pic_dev.h CELL_DEAD
+
+
 def run(n, gas, pressure, wall, weights, bfield=0.0, sort=16, steps=4, te=4.0,
-        emit=False):
+        emit=False, removed=False):
     p = workloads.discharge(16, 4, te=te)
     p.init_particle_no = n
     if pressure:
@@ -34,6 +38,11 @@ def run(n, gas, pressure, wall, weights, bfield=0.0, sort=16, steps=4, te=4.0,
     p.sort_interval = sort
     p.magnetic_field, p.angle = bfield, 0.0
     with pic2d.Pic(p) as sim:
+        if removed:
+            for s in (0, 1):
+                d = sim.get_state(s)
+                d["cell"][d["id"] % 7 == 0] = (CELL_REMOVED & 0xFFFF) | (3 << 16)
+                sim.set_state(s, d)
         if weights is not None:
             for s in (0, 1):
                 sim.set_weights(s, weights[s][sim.get_state(s)["id"]])
@@ -86,3 +95,23 @@ def test_weighted_passes_match_the_generic_pass(n, kind, sort):
     kw = dict(sort=sort, te=40.0 if emit else 4.0, emit=emit)
     compare(run(n, gas, pressure, wall, w, **kw), run(n, gas, pressure, wall, w, bfield=1e-30, **kw),
             kind, n)
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("kind", ["steady", "argon", "emit"])
+def test_uploaded_removed_particles_reach_no_wall(kind, weighted):
+    """a particle uploaded with the cell of one a collision removed is counted
+    as such and dropped by the next pass; it has not reached a wall, so no
+    pair is re-injected for it and the surface pass does not see it"""
+    n = 2000
+    gas, pressure, wall, emit = {
+        "steady": (pic2d.GAS_ARGON, 0.0, pic2d.WALL_STEADY, False),
+        "argon": (pic2d.GAS_ARGON, 66.0, pic2d.WALL_STEADY, False),
+        "emit": (pic2d.GAS_ARGON, 0.0, pic2d.WALL_ABSORB, True),
+    }[kind]
+    print(f"removed {kind} weighted={weighted}", flush=True)
+    w = [np.full(n, 0.5, dtype=np.float32)] * 2 if weighted else None
+    kw = dict(sort=16, steps=1, emit=emit, removed=True)
+    a = run(n, gas, pressure, wall, w, **kw)
+    assert all(a[2][s][4] >= n // 7 for s in (0, 1))
+    compare(a, run(n, gas, pressure, wall, w, bfield=WEAK, **kw), kind, n)

@@ -1425,10 +1425,13 @@ __device__ __forceinline__ void push_scatter_fast(PUSH_SCATTER_PARAMS) {
             move_sel(s[r], ok[g], ex[g], ey[g], pc);
             kept[r] = claim[r] && inside_cells(s[r], pc.N);
             if (claim[r] && !kept[r]) {
-                atomicAdd(&sl[classify(s[r], pc.N, pc.mode) - 1], 1u);
+                const int st = classify(s[r], pc.N, pc.mode);
+                atomicAdd(&sl[st - 1], 1u);
                 atomicAdd(&shole, 1u);
-                if (sp.lost_ids) queue_lost(sp, pid[r], w[r]);
-                if (sp.wall)  // waits for the surface pass
+                // (an uploaded CELL_DEAD particle has reached no wall; the
+                // first pass after an upload sorts, so no in-place pass meets one)
+                if (sp.lost_ids && st <= ST_TOP) queue_lost(sp, pid[r], w[r]);
+                if (sp.wall && st <= ST_TOP)  // waits for the surface pass
                     stage_put(sp.wq, &sp.cw->wall_count, &sp.cw->overflow, s[r],
                               (unsigned long long)pid[r], w[r]);
             }
