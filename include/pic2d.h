@@ -219,9 +219,12 @@ int pic_checkpoint_read(pic_handle *h, const char *path);
 
 /* Launch-shape choices of a live run (no reference counterpart; used by the
  * autotuner, autotune.py): particle passes per counting sort of electrons
- * and ions (0: leave) and red-black sweeps per leg of the tolerance solve
- * (0: leave, else 1..3).  Results do not depend on them.
- * pic_get_tuning: {sort interval e, sort interval i, sort key, sweeps}. */
+ * and ions (0: leave) and red-black sweeps per leg of the tolerance solve's
+ * V-cycles (0: leave, else 1..3).  Results do not depend on them.  The solver
+ * is chosen when the run is created (pic_params.mg_sweeps): a run with the
+ * direct solve accepts sweeps and has no use for them.
+ * pic_get_tuning: {sort interval e, sort interval i, sort key, sweeps}; sweeps
+ * 0: the direct solve, none in effect. */
 int pic_set_tuning(pic_handle *h, int32_t sort_interval_e, int32_t sort_interval_i,
                    int32_t mg_sweeps);
 int pic_get_tuning(pic_handle *h, int32_t *out4);

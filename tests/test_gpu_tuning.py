@@ -1,8 +1,8 @@
 """The launch-shape choices do not change results: the same run with every
 species sorted on every pass and with the tuned intervals (set on the live
 run through pic_set_tuning) ends with the same particles (by id), charge,
-phi and E, bit for bit; the tolerance solve meets its target with 1, 2 or 3
-sweeps per leg."""
+phi and E, bit for bit; the V-cycles of the tolerance solve meet their target
+with 1, 2 or 3 sweeps per leg, and the direct solve has no sweeps to set."""
 import numpy as np
 import pytest
 
@@ -52,13 +52,31 @@ def test_sort_intervals_do_not_change_results(collisions):
 def test_sweeps_meet_the_target(nu):
     p = workloads.discharge(128, 10, te=4.0)
     p.mg_tol = 1e-10
+    p.mg_sweeps = nu % 3 + 1  # V-cycles, with another sweep count
     with pic2d.Pic(p) as sim:
         sim.run(1)
+        assert sim.tuning()["mg_sweeps"] == nu % 3 + 1
         sim.set_tuning(0, 0, nu)
         assert sim.tuning()["mg_sweeps"] == nu
         sim.advance(3)
-        _, _, rr = sim.mg_stats()
-        assert rr <= 1e-10
+        cycles, _, rr = sim.mg_stats()
+        assert rr <= 1e-10 and cycles > 1
     with pytest.raises(pic2d.PicError):
         with pic2d.Pic(p) as sim:
             sim.set_tuning(0, 0, 4)
+
+
+def test_direct_solve_reports_no_sweeps():
+    """a run that holds the direct solve takes a sweep count and goes on
+    without: none is in effect, and the potential is the same"""
+    phi = []
+    for nu in (0, 3):
+        p = workloads.discharge(128, 10, te=4.0)
+        with pic2d.Pic(p) as sim:
+            sim.run(1)
+            sim.set_tuning(0, 0, nu)
+            assert sim.tuning()["mg_sweeps"] == 0
+            sim.advance(3)
+            assert sim.mg_stats()[0] == 1
+            phi.append(sim.get_phi())
+    assert np.array_equal(phi[0], phi[1])

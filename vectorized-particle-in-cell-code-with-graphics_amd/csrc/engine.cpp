@@ -1753,7 +1753,7 @@ int pic_get_tuning(pic_handle *h, int32_t *out4) {
     out4[0] = h->sp[0].sort_interval;
     out4[1] = h->sp[1].sort_interval;
     out4[2] = h->keyshift;
-    out4[3] = h->M.nu;
+    out4[3] = h->M.dir.n > 0 ? 0 : h->M.nu;  // the direct solve has no sweeps
     return PIC_OK;
 }
 

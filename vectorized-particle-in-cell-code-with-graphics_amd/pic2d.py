@@ -497,13 +497,15 @@ class Pic:
         self._c(self.lib.pic_checkpoint_write(self.h, str(path).encode()))
 
     def set_tuning(self, sort_interval_e=0, sort_interval_i=0, mg_sweeps=0):
-        """passes per counting sort of each species, tolerance-solve sweeps
-        per leg (0: leave as is); results do not depend on them"""
+        """passes per counting sort of each species, sweeps per leg of the
+        tolerance solve's V-cycles (0: leave as is; without effect on a run with
+        the direct solve); results do not depend on them"""
         self._c(self.lib.pic_set_tuning(self.h, int(sort_interval_e), int(sort_interval_i),
                                         int(mg_sweeps)))
 
     def tuning(self):
-        """{sort_interval_e, sort_interval_i, sort_key, mg_sweeps} in effect"""
+        """{sort_interval_e, sort_interval_i, sort_key, mg_sweeps} in effect
+        (mg_sweeps 0: the direct solve has none)"""
         a = (C.c_int32 * 4)()
         self._c(self.lib.pic_get_tuning(self.h, a))
         return dict(zip(("sort_interval_e", "sort_interval_i", "sort_key", "mg_sweeps"), a))
