@@ -91,9 +91,10 @@ def test_start_from_a_guess_with_wall_values(n):
 
 @pytest.mark.parametrize("cells", [32, 128])
 def test_steps_with_and_without_given_sweeps(cells):
-    """the library's choice (direct) and V-cycles asked for by mg_sweeps give
-    the potential of the same charge to the tolerance; a tolerance too tight
-    to be met by every first solve (verdict read per step) changes nothing"""
+    """the library's choice (direct) and V-cycles asked for by mg_sweeps (on
+    33^2 the direct solve as well) give the potential of the same charge to
+    the tolerance; a tolerance too tight to be met by every first solve (verdict
+    read per step) changes nothing"""
     phi = []
     for sweeps, tol in ((-1, 1e-9), (2, 1e-12), (-1, 1e-14)):
         p = workloads.discharge(cells, 20, te=4.0)
@@ -124,3 +125,40 @@ def test_graph_replayed_sweeps_match_launched_sweeps():
     for k in (0, 1, 2):
         assert np.array_equal(a[k], b[k]), k
     assert a[3][1] == b[3][1] > 12  # the same number of V-cycles, several a step
+
+
+@pytest.mark.parametrize("cells,sweeps", [(128, 3), (256, 1), (256, 3), (512, 2), (512, 3),
+                                          (1024, 1), (1024, 2), (1024, 3)])
+def test_given_sweeps_against_numpy_transforms(cells, sweeps):
+    """V-cycles on the grids where a sweep count selects them, the top leg fused
+    with the residual pass up to 513^2 and apart above: the potential of the
+    last step's own charge.  ||u - A^-1 f|| <= ||r|| / lambda_min, lambda_min =
+    2 pi^2 / L^2 to a part in cells^2"""
+    print(f"V({sweeps},{sweeps}) cells={cells}", flush=True)
+    p = workloads.discharge(cells, 4, te=4.0)
+    p.mg_tol, p.mg_sweeps, p.mg_max_iter = 1e-10, sweeps, 60
+    with pic2d.Pic(p) as sim:
+        sim.run(3)
+        cycles, total, rr = sim.mg_stats()
+        rho, phi = sim.get_rho(), sim.get_phi()
+    assert rr <= 1e-10 and cycles >= 1 and total > 3
+    f = -rho / p.epsilon
+    f[0] = f[-1] = f[:, 0] = f[:, -1] = 0.0
+    ref = poisson(f)
+    assert np.linalg.norm(phi - ref) <= 1.01 * rr * np.linalg.norm(f) * L ** 2 / (2 * np.pi ** 2) \
+        + 4 * EPS * np.log2(2 * cells) * np.linalg.norm(ref)
+
+
+def test_grid_beyond_the_transforms():
+    """above 4097^2 the tolerance solve takes V-cycles: one sine mode, whose
+    solution is known, to the bound of the residual (as above)"""
+    n, tol = 8192, 1e-7
+    print(f"V-cycles n={n}", flush=True)
+    x = np.arange(n + 1)
+    f = np.outer(np.sin(3 * np.pi * x / n), np.sin(5 * np.pi * x / n))
+    f[0] = f[-1] = f[:, 0] = f[:, -1] = 0.0
+    lam = -4.0 * (n / L) ** 2 * (np.sin(3 * np.pi / (2 * n)) ** 2 + np.sin(5 * np.pi / (2 * n)) ** 2)
+    u, cycles, rr = pic2d.poisson_tol(f, length=L, tol=tol)
+    assert rr <= tol and cycles > 1
+    u -= f / lam
+    assert np.linalg.norm(u) <= 1.01 * tol * np.linalg.norm(f) * L ** 2 / (2 * np.pi ** 2)
