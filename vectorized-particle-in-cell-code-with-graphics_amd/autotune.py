@@ -16,9 +16,10 @@ solve only and are carried over (MG_SWEEPS).
 
 It writes csrc/tuned.h (the table compiled into libpic2d.so; a species'
 best interval k becomes the constant c = k d of the rule k = round(c / d),
-d = sigma dt / dx its thermal displacement per step in cells) and tuned.json
-(every measurement).  Rebuild the library afterwards (make, or
-__graft_entry__.build()).  Results do not depend on any of these choices.
+d = sigma dt / dx its thermal displacement per step in cells; the choices of
+PAIRED replace those of its one run) and tuned.json (every measurement).
+Rebuild the library afterwards (make, or __graft_entry__.build()).  Results do
+not depend on any of these choices.
 
     python autotune.py [--classes 65,129,257,513,1025] [--steps 20]
 """
@@ -26,6 +27,7 @@ import argparse
 import json
 import os
 import sys
+import textwrap
 import time
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -38,6 +40,15 @@ KEYS = (6, 5, 7)  # the first is the default; another must beat it by ACCEPT
 INTERVALS_E = (1, 2, 3, 4, 6, 8, 12)
 INTERVALS_I = (4, 8, 16)
 MG_SWEEPS = {513: 3}  # measured with the V-cycles; 2 elsewhere
+# Choices decided by paired runs at other densities and gases of the class than
+# the one run below (20 steps at 257^2, 10 at 513^2), which it would lose
+PAIRED = {
+    129: (dict(e=16), "16 passes per electron sort (12 passes: 1.5 % faster alone, 1.4 % slower "
+                      "in an ensemble)"),
+    257: (dict(e=8), "8 passes per electron sort (200 particles per cell: 7.07 ms, 12 passes "
+                     "7.15; hydrogen 4.63 and 4.71)"),
+    513: (dict(sort_key=7), "key 7 (33 particles per cell: 3.53 ms, key 6 3.63)"),
+}
 ACCEPT = 0.01  # a candidate must beat the incumbent by 1 %
 D_FLOOR = 0.05  # the library's rule floors the displacement d at 0.05 cells
 
@@ -102,15 +113,20 @@ def tune_class(nodes, ppc, steps, warmup):
                 best = dict(sort_key=key, ms=base, **cur)
             dx = p.length / (p.nodes - 1)
             d = [p.sigma_load_e * p.dt / dx, p.sigma_load_i * p.dti / dx]
-    best["sort_c"] = [round(best["e"] * max(d[0], D_FLOOR), 3),
-                      round(best["i"] * max(d[1], D_FLOOR), 3)]
     best["displacement"] = d
+    best["sort_c"] = sort_c(best)
     log(f"N={nodes}: best {best}")
     return best, rows
 
 
-HEADER = """// tuned.h -- the library's launch-shape choices per grid size class, as the
-// autotuner (autotune.py) measured them; regenerate with it, do not edit.
+def sort_c(b):
+    return [round(b[k] * max(d, D_FLOOR), 3) for k, d in zip("ei", b["displacement"])]
+
+
+HEADER = """// tuned.h -- the library's launch-shape choices per grid size class, written by
+// the autotuner (autotune.py); regenerate with it, do not edit.  Measured there,
+// but for the entries that paired runs decided:
+%s
 // A row applies to grids of up to max_nodes nodes per side (the last row to
 // every larger grid):
 //   sort_c[s]  passes per counting sort of species s (0 electrons, 1 ions)
@@ -145,6 +161,21 @@ inline const TunedRow &tuned_row(int nodes) {
 """
 
 
+def header(note, results):
+    """tuned.h from the classes' measured choices (tuned.json's "best")"""
+    why, rows = [], []
+    for b in results:
+        n = b["max_nodes"]
+        choice, reason = PAIRED.get(n, ({}, None))
+        b = dict(b, **choice)
+        c = sort_c(b)
+        rows.append(f"    {{{n}, {{{c[0]}, {c[1]}}}, {b['sort_key']}, {b['nu']}}}")
+        if reason:
+            why += textwrap.wrap(f"{n}^2: {reason}", 86, initial_indent="//   ",
+                                 subsequent_indent="//     ")
+    return HEADER % ("\n".join(why), note, ",\n".join(rows))
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--classes", default="65,129,257,513,1025")
@@ -159,13 +190,10 @@ def main():
         best, r = tune_class(n, args.ppc, args.steps, args.warmup)
         results.append(dict(max_nodes=n, **best))
         rows += r
-    lines = ",\n".join(
-        f"    {{{b['max_nodes']}, {{{b['sort_c'][0]}, {b['sort_c'][1]}}}, {b['sort_key']}, {b['nu']}}}"
-        for b in results)
     note = (f"measured by autotune.py on an MI355X (gfx950): argon discharges, {args.ppc} "
             f"particles per cell per species, best of 2 x {args.steps} steps per choice")
     with open(os.path.join(args.out_dir, "csrc", "tuned.h"), "w") as f:
-        f.write(HEADER % (note, lines))
+        f.write(header(note, results))
     with open(os.path.join(args.out_dir, "tuned.json"), "w") as f:
         json.dump(dict(note=note, best=results, measurements=rows), f, indent=1)
     print(json.dumps(dict(best=results)))

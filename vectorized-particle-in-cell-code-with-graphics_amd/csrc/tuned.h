@@ -1,8 +1,11 @@
-// tuned.h -- the library's launch-shape choices per grid size class, as the
-// autotuner (autotune.py) measured them, but for three entries that paired runs
-// over more densities decided: 257^2 keeps 8 passes per electron sort (200 ppc:
-// 7.07 ms per 20 steps, 12 passes 7.15; hydrogen 4.63 and 4.71), 129^2 keeps
-// 16 (12 passes: 1.5 % faster alone, 1.4 % slower in an ensemble), 513^2 key 7 (33 ppc: 3.53 ms, key 6 3.63).
+// tuned.h -- the library's launch-shape choices per grid size class, written by
+// the autotuner (autotune.py); regenerate with it, do not edit.  Measured there,
+// but for the entries that paired runs decided:
+//   129^2: 16 passes per electron sort (12 passes: 1.5 % faster alone, 1.4 % slower
+//     in an ensemble)
+//   257^2: 8 passes per electron sort (200 particles per cell: 7.07 ms, 12 passes
+//     7.15; hydrogen 4.63 and 4.71)
+//   513^2: key 7 (33 particles per cell: 3.53 ms, key 6 3.63)
 // A row applies to grids of up to max_nodes nodes per side (the last row to
 // every larger grid):
 //   sort_c[s]  passes per counting sort of species s (0 electrons, 1 ions)
