@@ -65,18 +65,20 @@ def test_wall_pass_keeps_the_store_order(n):
             assert np.array_equal(a[k][keep], b[k]), k
 
 
-def test_gather_sorts_a_store_whose_order_nobody_knows():
-    """phase by phase, a gather after sort_interval moves sorts the particles by
-    tile, unless the store's order has been read since its last sort pass or
-    it has not passed the walls since the move; the particles are the same"""
+@pytest.mark.parametrize("fused", [4, 0])
+def test_gather_sorts_a_store_whose_order_nobody_knows(fused):
+    """phase by phase, from a new handle or after fused steps, a gather after
+    sort_interval moves sorts the particles by tile, unless the store's order
+    has been read since its last sort pass or it has not passed the walls
+    since the move; the particles are the same"""
     out = []
     for read, walls in ((False, True), (True, True), (True, False), (False, False)):
-        print(f"gather sort, read {read}, walls {walls}", flush=True)
+        print(f"gather sort, fused {fused}, read {read}, walls {walls}", flush=True)
         p = workloads.discharge(64, 4, te=40.0)
         p.sort_key = 6  # one tile
         p.sort_interval = 2
         with pic2d.Pic(p) as sim:
-            sim.advance(4)
+            sim.advance(fused)
             if read:
                 sim.get_state(0)
             for k in range(2):

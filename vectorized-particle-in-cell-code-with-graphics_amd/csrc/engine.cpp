@@ -907,11 +907,20 @@ int absorb_species(pic_handle *h, int si, bool plop) {
 
 // A loop driven phase by phase moves its particles without a sort pass, and
 // gather and deposit slow down as the store loses its order (129^2, 1.05 M
-// particles per species: four steps take 1.22 ms then, 0.59 with the sorts).  A
-// gather after as many moves as the fused step makes passes between sorts
-// sorts first.  A store whose order the caller may know keeps it (loaded,
-// uploaded, or read since its last sort pass), and one that has not passed the
-// walls since its move keeps its particles outside (the sort would drop them).
+// particles per species, a new run: four steps take 0.50 ms at first and 1.02
+// after a hundred steps; with the sorts 0.45 to 0.56 throughout).  A gather
+// after as many moves as the fused step makes passes between sorts sorts
+// first.  It does not where the caller may know the store's order or the sort
+// would drop particles that the walls have yet to see:
+//   - the particles came from the caller (a dump, pic_set_state, a checkpoint),
+//     or their order has been read (pic_get_state, pic_get_particles,
+//     pic_get_weights, a dump) since the last sort pass, a fused step's or one
+//     without a push.  A phase loop that reads its particles once stays
+//     unsorted from there;
+//   - pic_inject_particles has appended to the store since that sort pass (the
+//     new particles' places at its end are the caller's to find);
+//   - pic_boundary has not run since the move, or the walls emit;
+//   - reference mode, whose walls leave particles outside for later steps.
 void resort(pic_handle *h, int si) {
     const Species &s = h->sp[si];
     if (h->P.mode == PIC_MODE_PHYSICAL && s.walled && !s.order_seen &&
