@@ -323,17 +323,22 @@ int pic_mglin_noalloc(double *u, int32_t n, int32_t ncycle, double length, void 
 /* Residual-controlled Poisson solve (no reference counterpart; the
  * PIC_MG_TOL solver of the timestep): A u = f with the 5-point Laplacian of
  * mglin.cpp:133-144, zero walls; u (n*n) is the initial guess on entry and
- * the solution on exit.  FP32 V(1,1) cycles on the correction equation, FP64
- * residual and accumulation, until ||f-Au||_2 <= tol ||f||_2 (interior). */
+ * the solution on exit, ||f-Au||_2 <= tol ||f||_2 (interior).  Up to 4097^2
+ * the guess's residual is solved for directly (sine transforms, FP64) and added,
+ * again while that halves it; above, FP32 V-cycles on the correction equation
+ * with FP64 residual and accumulation.  *cycles: solves or V-cycles taken, at
+ * most max_iter. */
 int pic_poisson_tol(const double *f, double *u, int32_t n, double length, double tol,
                     int32_t max_iter, int32_t *cycles, double *relres);
 
 /* --------------------------------------------------------------- getters */
-/* work of the last solve: V-cycles, or 1 for the direct solve (tolerance
- * mode), or ncycle; the cumulative count; and the relative residual reached
- * (tolerance mode).  The direct solve runs without a host wait during the
- * step: this call then sums the last solve's residual, waiting for the device
- * if it has not finished it. */
+/* work of the last solve: V-cycles or direct solves (tolerance mode), or
+ * ncycle; the cumulative count; and the relative residual reached (tolerance
+ * mode).  Where mg_tol is at least 8 eps 4 (nodes-1)^2 / pi^2 (eps = 2.2e-16;
+ * 7.5e-10 at 1025^2) the direct solve is one, and the step does not wait for
+ * it: this call then sums its residual, waiting for the device if it has not
+ * finished.  With a tighter mg_tol the step waits for every solve's residual
+ * and refines the solution (one more solve at a time) where it has to. */
 int pic_get_mg_stats(pic_handle *h, int32_t *last_cycles, int64_t *total_cycles, double *relres);
 int pic_particle_size(pic_handle *h, int32_t s, int64_t *n);        /* particle::particle_size */
 int pic_get_particles(pic_handle *h, int32_t s, pic_particle *out, int64_t cap); /* 48-B AoS copy */

@@ -11,6 +11,11 @@
 // residual of rounding size, where the FP32 V-cycles with FP64 refinement
 // took 2 (65^2) to 5 (1025^2) cycles of 2 to 9 launches each.
 //
+// Methods: the Fourier solution of the 5-point problem is Hockney's (J. ACM 12,
+// 1965), the sine transform through the FFT of the odd extension Cooley, Lewis
+// and Welch's (J. Sound Vib. 12, 1970), the self-sorting FFT Stockham's
+// (Cochran et al., Proc. IEEE 55, 1967).
+//
 // The FFT (fft_fwd) keeps eight points per thread in registers and exchanges
 // them through LDS between radix-8 passes: thread t holds the points t + NT s,
 // s = 0..7, NT = L/8, before the first pass, and the same points of the

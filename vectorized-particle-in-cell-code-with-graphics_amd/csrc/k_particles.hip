@@ -196,11 +196,18 @@ __device__ __forceinline__ bool collide_take(bool blk, int qs, PState &s, int &e
 // block's particles of one key take consecutive slots.  Every particle's rank
 // within its key comes from the LDS counter of its entry.
 #define IPP (PASS_BLOCK / 256)
-// The in-place passes of a store of at most INPL_SMALL_MAX particles (with IPP
-// per thread less than a block for each of 256 CUs) take IPP_SMALL per thread:
-// there a pass is the latency of one block's chain, not throughput.  2 x
-// 262 144 particles in reference mode 2.55 -> 2.30 ms for ten steps, 33^2 148
-// -> 142 us; at 410 000 particles (65^2) 737 -> 796 us, two per thread 734.
+// The in-place passes of a store with room for at most INPL_SMALL_MAX particles
+// (its capacity, which the grid covers: half as much again as the initial count
+// where particles are created) take IPP_SMALL per thread: with IPP there are
+// fewer blocks than 256 CUs, and a pass is the latency of one block's chain,
+// not throughput.  A step with one and with four per thread, by capacity:
+//                              131 k       200 k       262 k       410-420 k
+//   257^2, reference mode   193 / 221   197 / 223   204 / 225   219 / 244 us
+//   257^2, collisionless     36 / 41     36 / 43     40 / 41     43 / 49
+//   65^2, collisionless      29 / 30     31 / 31     34 / 32     37 / 34
+//   65^2, argon              46 / 51     49 / 54     52 / 56     54 / 56
+// Dense cells cross over near 200 k (one particle per thread flushes four
+// windows where one would do), sparse ones above 420 k; 33^2 gains 148 -> 144 us.
 #define IPP_SMALL 1
 #define INPL_SMALL_MAX (256 * PASS_BLOCK)
 #define HASH_BITS 11

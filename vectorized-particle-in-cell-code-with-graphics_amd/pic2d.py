@@ -351,7 +351,8 @@ def cross_section(gas, channel, energy, mode=MODE_PHYSICAL):
 
 
 def poisson_tol(f, u0=None, length=1.0, tol=1e-10, max_iter=60):
-    """GPU mixed-precision multigrid to a relative residual; returns (u, cycles, relres)."""
+    """GPU Poisson solve to a relative residual (direct up to 4097^2, mixed-
+    precision multigrid above); returns (u, solves or V-cycles, relres)."""
     f = np.ascontiguousarray(f, dtype=np.float64)
     u = np.zeros_like(f) if u0 is None else np.ascontiguousarray(u0, dtype=np.float64).copy()
     cyc = C.c_int32()
@@ -622,7 +623,8 @@ class Pic:
         return v.value
 
     def mg_stats(self):
-        """(V-cycles of the last solve, cumulative V-cycles, last relative residual)"""
+        """(V-cycles or direct solves of the last solve, their cumulative count,
+        last relative residual)"""
         a, b, c = C.c_int32(), C.c_int64(), C.c_double()
         self._c(self.lib.pic_get_mg_stats(self.h, C.byref(a), C.byref(b), C.byref(c)))
         return a.value, b.value, c.value
