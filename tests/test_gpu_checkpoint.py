@@ -3,7 +3,8 @@ pic_checkpoint_read, k more steps -- against 2k uninterrupted steps of the
 same run: every particle (by id), counters, fixed-point
 charge, phi, E, the solver's statistics, collision and loss counts, the
 diagnostics' window sums and timeData rows, all bit for bit.  Covered: the
-tolerance solve (its warm start reads the previous two potentials), argon
+tolerance solve (direct, and V-cycles, whose warm start reads the previous two
+potentials), argon
 MCC with pair re-injection and energy-binned bounds, the reference's
 steady walls, per-particle weights (source and reduction on), and a graph
 window that spans the checkpoint."""
@@ -48,6 +49,10 @@ def case(name):
     if name == "tol":
         p = workloads.discharge(64, 20, mode=pic2d.MODE_PHYSICAL, mg_mode=pic2d.MG_TOL, te=4.0)
         p.mg_tol = 1e-9
+    elif name == "vcycles":
+        p = workloads.discharge(128, 10, mode=pic2d.MODE_PHYSICAL, mg_mode=pic2d.MG_TOL, te=4.0)
+        p.mg_tol = 1e-9
+        p.mg_sweeps = 1
     elif name == "argon":
         p = workloads.with_argon(workloads.discharge(64, 20, te=4.0), pressure_pa=60.0)
     elif name == "ref_steady":
@@ -71,7 +76,7 @@ def case(name):
     return p
 
 
-@pytest.mark.parametrize("name", ["tol", "argon", "ref_steady", "weighted_diag"])
+@pytest.mark.parametrize("name", ["tol", "vcycles", "argon", "ref_steady", "weighted_diag"])
 def test_resume_is_bit_exact(name, tmp_path):
     k = 8
     print(f"checkpoint {name}", flush=True)

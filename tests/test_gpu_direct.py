@@ -108,6 +108,41 @@ def test_steps_with_and_without_given_sweeps(cells):
         assert np.linalg.norm(x - phi[0]) < 1e-9 * np.linalg.norm(phi[0])
 
 
+@pytest.mark.parametrize("cells", [4, 32, 64, 128])
+@pytest.mark.parametrize("phases", [False, True])
+def test_nonzero_walls_and_field(cells, phases):
+    """phi with driven wall values and E from it, in one launch (fused step) and
+    apart (by phases): the walls hold their values, E is the oracle's of this
+    phi bit for bit, and A phi = -rho / epsilon up to the rounding of phi's
+    second differences, 8 eps max|phi| / h^2 a node"""
+    print(f"walls cells={cells} phases={phases}", flush=True)
+    p = workloads.discharge(cells, 20, te=4.0)
+    p.phi_left, p.phi_right, p.phi_bottom, p.phi_top = 1.5, -2.0, 0.5, 3.0
+    p.phi_period = 0.3
+    with pic2d.Pic(p) as sim:
+        sim.run(3)
+        step = 2  # of the last solve
+        if phases:
+            sim.grid_potential(p.phi_left, p.phi_right, p.phi_bottom, p.phi_top, step, p.phi_period)
+            sim.grid_electric_field()
+        phi, rho, (ex, ey), E32 = sim.get_phi(), sim.get_rho(), sim.get_E(), sim.get_E32()
+        assert sim.mg_stats()[0] == 1 and sim.mg_stats()[2] <= p.mg_tol
+    assert np.all(phi[0] == 0.5) and np.all(phi[-1] == 3.0)
+    assert np.all(phi[1:-1, 0] == 1.5)
+    assert np.allclose(phi[1:-1, -1], -2.0 * np.cos(0.3 * step), rtol=0, atol=1e-15)
+    h = p.length / cells
+    oex, oey = orc.ref_efield(phi, h)
+    assert np.array_equal(ex, oex) and np.array_equal(ey, oey)
+    k = len(E32) // 2
+    assert np.array_equal(E32[0::2], ex[:k].astype(np.float32))
+    assert np.array_equal(E32[1::2], ey[:k].astype(np.float32))
+    r = (phi[2:, 1:-1] + phi[:-2, 1:-1] + phi[1:-1, 2:] + phi[1:-1, :-2] - 4 * phi[1:-1, 1:-1]) / h ** 2 \
+        + rho[1:-1, 1:-1] / p.epsilon
+    # + the solve's own error, 4 eps log2(2n) |phi| (above), through A
+    bound = (8 + 8 * 4 * np.log2(2 * cells)) * EPS * np.abs(phi).max() / h ** 2
+    assert np.sqrt(np.mean(r ** 2)) <= bound, (np.sqrt(np.mean(r ** 2)), bound)
+
+
 def test_graph_replayed_sweeps_match_launched_sweeps():
     """explicit V(2,2) cycles (the direct solve records no graph): batches
     replayed from captured hipGraphs give the launched kernels' results, bit
