@@ -12,7 +12,7 @@ Prints ONE JSON line on stdout:
                  the reference's phase order) on a bounded sample of the same
                  workload, timed on this host
   latency_ms     p50 / p99 of per-step durations (HIP events around each step)
-  accuracy       phi / E error of the split-precision solver against the
+  accuracy       phi / E error of the tolerance solve against the
                  library's FP64 multigrid solve of the same charge density
                  (converged to 1e-12), reported every 100 steps of an untimed
                  continuation of the run

@@ -39,7 +39,7 @@ extern "C" {
 #define PIC_MODE_PHYSICAL 1 /* x<0 or x>=L leaves, null-collision MCC        */
 
 #define PIC_MG_FIXED 0 /* FP64 FMG, ncycle V(1,1) per level (fields.cpp:174) */
-#define PIC_MG_TOL 1   /* FP32 smoothing + FP64 residual refinement to tol  */
+#define PIC_MG_TOL 1   /* solved to a relative residual mg_tol (see mg_sweeps) */
 
 #define PIC_LOAD_RANDOM 0  /* Philox uniform positions, Maxwellian velocities */
 #define PIC_LOAD_LATTICE 1 /* particle.cpp:410-443 lattice, both species co-located */
@@ -72,7 +72,7 @@ typedef struct pic_params {
     int32_t sigma_ionization; /* SIGMA_IONIZATION (PIC_SIGMA_*)                     */
     int32_t mg_mode;          /* PIC_MG_*                                           */
     int32_t mg_ncycle;        /* V-cycles per FMG level (fields.cpp:174 uses 2)     */
-    int32_t mg_max_iter;      /* PIC_MG_TOL: refinement sweeps cap                  */
+    int32_t mg_max_iter;      /* PIC_MG_TOL: solves or V-cycles at most             */
     int32_t dt_dti;           /* DT_DTI                                             */
     int32_t run_time;         /* TOTAL_RUN_TIME                                     */
     int32_t number_to_inject; /* NUMBER_TO_INJECT: particles of each species created
@@ -264,7 +264,7 @@ int pic_inject_particles(pic_handle *h, int32_t s);
 int pic_contain_particle_growth(pic_handle *h, int32_t s);
 
 /* Accuracy of the last field solve against an FP64 multigrid (no reference
- * counterpart: the error report of the split-precision PIC_MG_TOL solver,
+ * counterpart: the error report of the PIC_MG_TOL solver,
  * which replaces Mglin's fixed-cycle FP64 FMG).  The last solve's folded
  * right-hand side (fields.cpp:169-220) is solved again by the FP64 multigrid
  * alone -- the full multigrid of pic_mglin (mglin.cpp:21-55), then FP64

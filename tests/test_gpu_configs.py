@@ -1,7 +1,7 @@
 """Parity at the benchmark workloads' own sizes.
 
 C1 (workloads.plain: 65^2 nodes, 409 600 particles per species, physical
-mode, mixed-precision multigrid to 1e-8): after 1 and 10 fused steps the GPU
+mode, the direct solve to 1e-8): after 1 and 10 fused steps the GPU
 tracks the FP64 reference-layout oracle (48-byte AoS, FP64 push and deposit,
 the potential solved to a converged 1e-12) within 1e-6 relative L2 on
 positions, velocities, phi and E; with the FP64 FMG solver it is bit-exact

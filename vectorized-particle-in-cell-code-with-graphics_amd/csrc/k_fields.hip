@@ -1142,7 +1142,7 @@ int mg_tol_solve(hipStream_t st, MgLevels &M, double length, double tol, int max
 }
 
 // ------------------------------------------- FP64 reference solve (report)
-// The accuracy report of the split-precision solver: the same folded
+// The accuracy report of the tolerance mode: the same folded
 // right-hand side solved by the FP64 multigrid alone (the full multigrid of
 // the fixed mode, then FP64 V(1,1) cycles, mglin.cpp:176-196) until
 // ||f - Au||_2 <= tol ||f||_2 on the interior.
